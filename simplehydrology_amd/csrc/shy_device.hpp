@@ -179,6 +179,16 @@ __host__ __device__ inline float div_rcp(float a, float b, float y) {
   return markstein_div(a, b, y);
 }
 
+// Ranges in which step_coupling_short takes the place of step_coupling: what
+// pack_kernel checks per cell (discharge and momentum) and the host per
+// terrain (momentumTransfer).
+__host__ __device__ inline bool short_flow_ok(float fx, float fy, float d) {
+  return __builtin_fabsf(fx) <= 0x1p60f && __builtin_fabsf(fy) <= 0x1p60f && d >= 0.0f &&
+         d <= 0x1p59f;
+}
+__host__ __device__ inline bool short_transfer_ok(float mt) {
+  return __builtin_fabsf(mt) <= 0x1p50f;
+}
 // water.h:95-111 after the gravity term: momentum coupling, fixed step of
 // length sqrt(2).  rf = inv_len(fx, fy), used only when |f| > 0.
 __device__ inline void step_coupling(const shy_params& P, float vol, float d, float fx, float fy,

@@ -74,6 +74,7 @@ struct shy_ctx {
   int4* ent = nullptr;       // partition entries in tile order: wave_cap start cells, then
                              // wave_cap {slot, tracks} (16 B per log slot in all)
   int32_t* vq = nullptr;     // [terrain][row] quantised volume track per step
+  float2* vt = nullptr;      // [terrain][row + 1] {volume, 1 / volume} per step
   size_t vq_cap = 0;
   int vq_rows = 0;
   bool vq_dirty = true;      // parameters changed since vq was built
@@ -210,23 +211,32 @@ void drop_graph(shy_ctx* c) {
 constexpr int kPartMaxTiles = 32768;
 
 // Offsets of every terrain's cells, drops and cascade tiles; uploads the table.
-// Whether every volume a drop carries into a step (vol_0 = 1, vol_k+1 =
-// evap_vol(vol_k), while age <= maxAge and vol >= minVol: water.h:74-82, 136)
-// lies where the walk's reciprocal-form division is exact.
-bool volumes_in_division_range(const shy_params& P) {
+// The steps after which a drop still on the map ends and how (vol_0 = 1,
+// vol_k+1 = evap_vol(vol_k), while age <= maxAge and vol >= minVol:
+// water.h:74-82, 136), and whether the walk's short arithmetic applies: every
+// volume on the way in [2^-60, 1], momentumTransfer in its range, and record
+// offsets and cell indices in 32 bits.
+void walk_limits(Terrain& t) {
+  const shy_params& P = t.P;
+  bool ok = short_transfer_ok(P.momentumTransfer) && t.nx < (1 << 24) && t.ny < (1 << 24) &&
+            pack_records(t.nx, t.ny) <= (1LL << 27);
   float vol = 1.0f;
-  for (int age = 0;; ++age) {
-    if ((float)age > P.maxAge || vol < P.minVol) return true;
-    if (!markstein_den_ok(vol)) return false;
+  int age = 0;
+  for (;; ++age) {
+    if ((float)age > P.maxAge || vol < P.minVol) break;
+    ok = ok && markstein_den_ok(vol) && vol <= 1.0f;
     vol = evap_vol(vol, P.evapRate);
   }
+  t.max_steps = age;
+  t.end_kind = (float)age > P.maxAge ? kEndAge : kEndVol;
+  t.vol_ok = ok ? 1 : 0;
 }
 
 int layout(shy_ctx* c) {
   long long cells = 0, drops = 0, tiles = 0, recs = 0;
   const int ty = kTileY[c->tune.tile], tx = kTileX[c->tune.tile];
   for (Terrain& t : c->ter) {
-    t.vol_ok = volumes_in_division_range(t.P) ? 1 : 0;
+    walk_limits(t);
     t.cell_off = cells;
     t.pack_off = recs;
     recs += pack_records(t.nx, t.ny);
@@ -376,9 +386,13 @@ int ensure_wave(shy_ctx* c) {
       drop_graph(c);
       HIPCHK(c, hipStreamSynchronize(c->stream));
       if (c->vq) hipFree(c->vq);
+      if (c->vt) hipFree(c->vt);
       c->vq = nullptr;
+      c->vt = nullptr;
       c->vq_cap = 0;
       HIPCHK(c, hipMalloc(&c->vq, vq_need * sizeof(int32_t)));
+      // rows + 1 <= 2 rows entries per terrain whatever split of vq_need
+      HIPCHK(c, hipMalloc(&c->vt, 2 * vq_need * sizeof(float2)));
       c->vq_cap = vq_need;
       c->vq_dirty = true;
     }
@@ -386,7 +400,7 @@ int ensure_wave(shy_ctx* c) {
       if (rows != c->vq_rows) drop_graph(c);
       c->vq_rows = rows;
       const int nter = (int)c->ter.size();
-      volq_kernel<<<(nter + 63) / 64, 64, 0, c->stream>>>(c->d_ter, nter, rows, c->vq);
+      volq_kernel<<<(nter + 63) / 64, 64, 0, c->stream>>>(c->d_ter, nter, rows, c->vq, c->vt);
       HIPCHK(c, hipGetLastError());
       c->vq_dirty = false;
     }
@@ -484,6 +498,8 @@ WaveArgs wave_args(shy_ctx* c, int p) {
   w.sr = c->sr;
   w.qstride = c->qstride;
   w.dlog = c->dlog;
+  w.vt = c->vt;
+  w.vt_rows = c->vq_rows + 1;
   w.steps = c->wsteps;
   w.hist = c->hist;
   w.perm = ordered(c) ? c->dperm : nullptr;
@@ -821,7 +837,7 @@ int shy_destroy(shy_ctx* c) {
   drop_graph(c);
   void* ptrs[] = {c->h[0], c->h[1], c->fld, c->root, c->visit[0], c->visit[1], c->first,
                   c->sr, c->dh, c->trk, c->deposit, c->slog, c->strk, c->qb, c->ent, c->gflag,
-                  c->vq, c->tcount, c->tsum, c->hist, c->hbsum, c->tstart, c->dlog, c->wsteps, c->dperm, c->tsteps, c->veg_px, c->veg_py, c->veg_alive, c->veg_cflag,
+                  c->vq, c->vt, c->tcount, c->tsum, c->hist, c->hbsum, c->tstart, c->dlog, c->wsteps, c->dperm, c->tsteps, c->veg_px, c->veg_py, c->veg_alive, c->veg_cflag,
                   c->veg_cx, c->veg_cy, c->veg_units, c->veg_st, c->veg_size, c->pack, c->d_ter, c->state, c->erf_a, c->part, c->perms, c->trace_buf,
                   c->trace_n, c->drop_buf};
   for (void* q : ptrs)

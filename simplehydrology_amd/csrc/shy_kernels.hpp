@@ -108,9 +108,13 @@ struct Terrain {
   unsigned long long seed;
   unsigned int id;  // terrain number in the spawn hash
   int has_root;
-  // every volume a drop of this terrain can carry into a step lies where the
-  // walk's reciprocal-form division is exact (markstein_den_ok; host)
+  // every volume a drop of this terrain can carry into a step lies in
+  // [2^-60, 1] and momentumTransfer in short_transfer_ok (host): the walk's
+  // short arithmetic applies unless a cell is flagged (gflag)
   int vol_ok;
+  // steps after which a drop still on the map ends, and how (water.h:74-82):
+  // its age and volume depend on the step number alone
+  int max_steps, end_kind;
   shy_params P;
 };
 
@@ -139,6 +143,8 @@ struct WaveArgs {
   int qstride;        // qb's stride per drop: log rows rounded up to kReplayDepth
   const float* __restrict__ sr;   // burst scale per cell (tile_count_kernel)
   int4* dlog;         // [drop] {steps, end kind, end cell, unused}
+  const float2* __restrict__ vt;  // [terrain][vt_rows] {volume, 1 / volume} of a drop's step (volq_kernel)
+  int vt_rows;
   int32_t* steps;     // [drop] steps of the walk (the log rows it filled)
   int32_t* hist;      // per-terrain [tile][walk block] step counts, when the walk counts them
   const int32_t* __restrict__ perm;  // [drop] the terrain's drop a thread walks (order_kernel), or null
@@ -223,6 +229,71 @@ __device__ inline void block_add_stats(long long (&v)[NC], long long* out) {
 }
 
 // ------------------------------------------------------------------ walk
+// sqrt(x) and 1/x, correctly rounded, in 5 and 3 instructions: the hardware
+// approximation and one FMA-based correction.  Equal to __builtin_sqrtf and
+// to the division for every float in [2^-100, 2^100] (all 1.7e9 of them
+// compared on the device); outside it, and for 0, not used.  The full
+// sequences (about 14 and 11 instructions each, four and three of them per
+// step) were 40% of the 220 VALU instructions of a walk step, which are 880 of
+// its 1540 cycles at 256^2 and of its 2060 at 1024^2.
+__device__ inline float sqrt_short(float x) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y, h = 0.5f * y;
+  return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+}
+__device__ inline float rcp_short(float x) {
+  const float q = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, q, 1.0f), q, q);
+}
+
+// a squared speed outside the short root's range (0 is fine: not normalised)
+__device__ inline bool short_s2_bad(float s2) {
+  return (s2 > 0x1p100f) | ((s2 < 0x1p-100f) & (s2 != 0.0f));
+}
+
+// v_cvt_i32_f32: truncation, saturating, NaN gives 0
+__device__ inline int cvt_i32(float v) {
+  int r;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+
+// The same values with the short root and reciprocal and without branches.
+// Returns false where an operand lies outside their range (the caller then
+// runs step_coupling); the cell's flow satisfies short_flow_ok,
+// momentumTransfer short_transfer_ok and vol lies in [2^-60, 1].  mt =
+// lodsize * momentumTransfer.
+//  * |f| > 0 iff rf > 0 (pack_kernel sets rf to 0 otherwise; with |fx|, |fy|
+//    <= 2^60 it cannot underflow); sqrt(s2) > 0 iff s2 > 0.
+//  * mt dt / (vol + d) is the correctly rounded quotient by Markstein's
+//    theorem (markstein_div) for 2^-60 <= |mt dt| <= 2^60, and 2^-60 <= vol +
+//    d <= 2^60 holds.  The sign of a zero quotient may differ from the
+//    division's: c f and the speed it is added to then keep their values up
+//    to the sign of a zero, which no later operation turns into anything but
+//    the sign of a zero (sums with a position, products that are quantised).
+//  * without coupling c = 0, and adding 0 f (f finite) changes nothing but a
+//    zero's sign.
+__device__ inline bool step_coupling_short(float mt, float vol, float d, float fx, float fy,
+                                           float rf, float& sx, float& sy) {
+  const float s2 = sx * sx + sy * sy;
+  const float rs = rcp_short(sqrt_short(s2));
+  const float dt = (fx * rf) * (sx * rs) + (fy * rf) * (sy * rs);
+  const float a = mt * dt, b = vol + d, y = rcp_short(b);
+  const float q = a * y;
+  float c = __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+  const bool on = (rf > 0.0f) & (s2 > 0.0f);
+  c = on ? c : 0.0f;
+  const bool bad = on & (__builtin_fabsf(a) < 0x1p-60f) & (a != 0.0f);
+  const float ux = sx + c * fx, uy = sy + c * fy;
+  const float u2 = ux * ux + uy * uy;
+  const float k2 = kLod * __builtin_sqrtf(2.0f);  // lodsize*sqrt(2.0f)
+  const float r = rcp_short(sqrt_short(u2));
+  const bool move = u2 > 0.0f;
+  sx = move ? k2 * (ux * r) : ux;
+  sy = move ? k2 * (uy * r) : uy;
+  return !(bad | short_s2_bad(s2) | short_s2_bad(u2));
+}
+
 // One cache line per step: {h, h(x-1), h(x+1), h(y-1)}, {h(y+1), mx, my, d},
 // {erf(0.4 d), root, 0, 0}; neighbours off the map repeat the cell's own
 // height, as load_unpacked's clamped reads do (the normal never uses them).
@@ -279,7 +350,7 @@ struct NoStepHook {
   __device__ void operator()(int) const {}
 };
 
-template <int MODE, class Hook = NoStepHook, bool PREFETCH = false, bool SAFE = false>
+template <int MODE, class Hook = NoStepHook, bool PREFETCH = false>
 __device__ int walk_drop(const WalkArgs& a, int lane_drop, float x0, float y0, int* end,
                          int* end_cell, shy_drop_step* tr, int max_tr, int* tr_n,
                          Hook step_hook = Hook(), uint32_t* pf_sink = nullptr) {
@@ -351,16 +422,9 @@ __device__ int walk_drop(const WalkArgs& a, int lane_drop, float x0, float y0, i
     float effD = P.depositionRate * (1.0f - c.root);  // water.h:86-87
     if (effD < 0) effD = 0;
     if constexpr (COUNT) {  // water.h:95-111
-      // the record holds the gravity terms k n (x, z).  SAFE: every gravity
-      // term of the terrain and every volume lies where the reciprocal-form
-      // division is exact; else each division checks its operands
-      if constexpr (SAFE) {
-        sx = sx + markstein_div(n0, vol, yv);
-        sy = sy + markstein_div(n2, vol, yv);
-      } else {
-        sx = sx + div_rcp(n0, vol, yv);
-        sy = sy + div_rcp(n2, vol, yv);
-      }
+      // the record holds the gravity terms k n (x, z)
+      sx = sx + div_rcp(n0, vol, yv);
+      sy = sy + div_rcp(n2, vol, yv);
       step_coupling(P, vol, c.d, c.mx, c.my, c.rf, sx, sy, px, py);
     } else {
       step_motion(P, n0, n2, vol, c.d, c.mx, c.my, sx, sy, px, py);
@@ -440,6 +504,139 @@ __device__ int walk_drop(const WalkArgs& a, int lane_drop, float x0, float y0, i
   return steps;
 }
 
+// A read-only table read at an index that is uniform over the wave (scalar
+// loads: the compiler cannot tell by itself that no store of the kernel
+// writes the table).
+typedef const __attribute__((address_space(4))) float ConstF32;
+__device__ inline float2 ld_uniform2(const float2* p, int k) {
+  ConstF32* q = (ConstF32*)(uintptr_t)(p + k);
+  return make_float2(q[0], q[1]);
+}
+
+// The count walk of a terrain whose volumes, transfer and cells all lie in the
+// range of the short arithmetic (Terrain::vol_ok, gflag): the same values as
+// walk_drop<kCount>, which any other terrain takes, with
+//  * the short root, reciprocal and coupling (step_coupling_short; a step
+//    whose operands leave their range repeats with the full sequences);
+//  * the step's volume and its reciprocal from a table at the step number,
+//    which is the same for every lane of the wave (scalar loads);
+//  * the end by age or volume as a step count;
+//  * the tracks without clamps: |speed| <= sqrt(2) (1 + 2^-22) after
+//    normalisation, or NaN (cvt_i32 gives 0, as quant_t), or tiny where it was
+//    not normalised, and vol <= 1; scaling the volume by 2^24 first is exact;
+//  * 32-bit byte offsets from a uniform base for the records and log rows.
+// vt[k] holds the step's {volume, 1 / volume}; pack holds at most 2^27 records
+// and ny < 2^24 (the host checks).  Measured (a cycle, before and after): 64^2
+// with 256 drops 234 -> 210 us, 256^2 with 1024 drops 653 -> 590, 1024^2 with
+// 65536 drops 1.24 -> 1.19 ms, the 64-terrain ensemble 24.9 -> 24.1 ms; the
+// prefetch's place behind the record load is half of the gain at 1024^2.
+template <class Hook, bool PREFETCH>
+__device__ int walk_short(const WalkArgs& a, const float2* __restrict__ vt, int max_steps,
+                          int end_kind, int lane_drop, float x0, float y0, int* end,
+                          int* end_cell, Hook step_hook, uint32_t* pf_sink) {
+  const int nx = a.nx, ny = a.ny;
+  const float fnx = (float)nx, fny = (float)ny;
+  const float mt = kLod * a.P.momentumTransfer, entr = a.P.entrainment;
+  const char* packb = reinterpret_cast<const char*>(a.pack);
+  const uint32_t lane_off = (uint32_t)lane_drop * 8u;
+  const size_t row_bytes = (size_t)a.drops * 8u;
+  auto rec_off = [&](int x, int y) {
+    const uint32_t b = __umul24((uint32_t)x >> 1, (uint32_t)(ny + 1) >> 1) + ((uint32_t)y >> 1);
+    return (b << 7) | (((uint32_t)x & 1u) << 6) | (((uint32_t)y & 1u) << 5);
+  };
+  auto cell_of = [&](int x, int y) { return (int)(__umul24((uint32_t)x, (uint32_t)ny) + (uint32_t)y); };
+  float px = x0, py = y0, sx = 0.0f, sy = 0.0f;
+  uint32_t ro = rec_off((int)x0, (int)y0);
+  int i0 = cell_of((int)x0, (int)y0);
+  // {h, gravity x, gravity z, erf(0.4 d)}, {mx, my, d, 1/|(mx, my)|}
+  float4 ca = *reinterpret_cast<const float4*>(packb + ro);
+  float4 cb = *reinterpret_cast<const float4*>(packb + ro + 16);
+  uint32_t pf_acc = 0;
+  float pf = 0.0f;
+  // stored one step late, as in walk_drop; the first store is a placeholder in
+  // the drop's own slot of row 0
+  int2 ps = make_int2(a.cell_off + i0, 0), pt = make_int2(0, 0);
+  char* srow = reinterpret_cast<char*>(a.slog);
+  char* trow = reinterpret_cast<char*>(a.strk);
+  float2 v = ld_uniform2(vt, 0);
+  int steps = 0;
+  // wait for the first record before the loop (see walk_drop)
+  __builtin_amdgcn_s_waitcnt(0);
+  for (int k = 0;; ++k) {
+    if (k >= max_steps) {  // water.h:74-82
+      *end = end_kind;
+      *end_cell = i0;
+      break;
+    }
+    const float2 vn = ld_uniform2(vt, k + 1);
+    steps = k + 1;
+    // water.h:95-111
+    {
+      const float q0 = ca.y * v.y, q1 = ca.z * v.y;  // markstein_div up to a zero's sign
+      const float gx = sx + __builtin_fmaf(__builtin_fmaf(-q0, v.x, ca.y), v.y, q0);
+      const float gy = sy + __builtin_fmaf(__builtin_fmaf(-q1, v.x, ca.z), v.y, q1);
+      sx = gx;
+      sy = gy;
+      if (__builtin_expect(!step_coupling_short(mt, v.x, cb.z, cb.x, cb.y, cb.w, sx, sy), 0)) {
+        float ux = 0.0f, uy = 0.0f;
+        sx = gx;
+        sy = gy;
+        step_coupling(a.P, v.x, cb.z, cb.x, cb.y, cb.w, sx, sy, ux, uy);
+      }
+      px = px + sx;
+      py = py + sy;
+    }
+    const int jx = cvt_i32(px), jy = cvt_i32(py);
+    const bool ex = !((px > -1.0f) & (px < fnx) & (py > -1.0f) & (py < fny));
+    const int j = cell_of(jx, jy);
+    // off the map the record is not used; loading the current cell's keeps
+    // the load unconditional, so its wait is counted exactly
+    ro = ex ? ro : rec_off(jx, jy);
+    const float4 na = *reinterpret_cast<const float4*>(packb + ro);
+    const float4 nb = *reinterpret_cast<const float4*>(packb + ro + 16);
+    // PREFETCH (see walk_drop): the record of the cell the drop reaches from
+    // there at its current speed, issued right behind the record it waits
+    // for, so the prefetch is a whole step ahead of the load it serves.  Its
+    // word is folded in a step later, after the wait for the next record.
+    const float pf_last = pf;
+    if constexpr (PREFETCH) {
+      const int qx = cvt_i32(__builtin_amdgcn_fmed3f(px + sx, 0.0f, fnx - 1.0f));
+      const int qy = cvt_i32(__builtin_amdgcn_fmed3f(py + sy, 0.0f, fny - 1.0f));
+      pf = *reinterpret_cast<const float*>(packb + rec_off(qx, qy));
+    }
+    st_stream(reinterpret_cast<int2*>(srow + lane_off), ps);
+    st_stream(reinterpret_cast<int2*>(trow + lane_off), pt);
+    if (k > 0) {
+      srow += row_bytes;
+      trow += row_bytes;
+    }
+    const float v24 = v.x * kTQ;  // the tracks, water.h:115-117
+    pt = make_int2(cvt_i32(__builtin_rintf(v24 * sx)), cvt_i32(__builtin_rintf(v24 * sy)));
+    step_hook(a.cell_off + i0);
+    float h2 = na.x;
+    if (__builtin_expect(ex, 0)) h2 = (float)((double)ca.x - 0.002);  // water.h:120-124
+    float c_eq = (1.0f + entr * ca.w) * (ca.x - h2);  // water.h:127
+    if (c_eq < 0) c_eq = 0;
+    ps = make_int2(a.cell_off + i0, __float_as_int(c_eq));
+    if constexpr (PREFETCH) pf_acc ^= __float_as_uint(pf_last);
+    if (ex) {  // water.h:139-142
+      *end = kEndExit;
+      *end_cell = i0;
+      break;
+    }
+    v = vn;
+    ca = na;
+    cb = nb;
+    i0 = j;
+  }
+  // the last step's log, in its own row
+  const size_t last = (size_t)(steps > 0 ? steps - 1 : 0) * row_bytes;
+  st_stream(reinterpret_cast<int2*>(reinterpret_cast<char*>(a.slog) + last + lane_off), ps);
+  st_stream(reinterpret_cast<int2*>(reinterpret_cast<char*>(a.strk) + last + lane_off), pt);
+  if (pf_sink) *pf_sink = pf_acc;
+  return steps;
+}
+
 // The count walk's 32-byte per-cell record for this cycle (load_packed),
 // every cell of every terrain: {h, normal x, normal z, erf(0.4 d)},
 // {momentum x, momentum y, discharge, 1/|momentum|}.  The normal
@@ -477,7 +674,8 @@ __global__ void pack_kernel(const Terrain* __restrict__ ter, int nter, size_t nr
   // and 1/|momentum| for the coupling term (read only where |momentum| > 0)
   const float k = kLod * T.P.gravity;
   const float a0 = k * n0, a2 = k * n2;
-  if (!(markstein_num_ok(a0) && markstein_num_ok(a2))) gflag[t] = 1;
+  if (!(markstein_num_ok(a0) && markstein_num_ok(a2) && short_flow_ok(f.x, f.y, f.z)))
+    gflag[t] = 1;
   const float rf = f.x * f.x + f.y * f.y > 0.0f ? inv_len(f.x, f.y) : 0.0f;
   pack[2 * g] = make_float4(hc, a0, a2, f.w);
   pack[2 * g + 1] = make_float4(f.x, f.y, f.z, rf);
@@ -543,13 +741,13 @@ __global__ void __launch_bounds__(1024) walk_kernel(WaveArgs w) {
         int end = 0, end_cell = 0;
         uint32_t sink = 0;
         const float x0 = (float)(cid / (uint32_t)T.ny), y0 = (float)(cid % (uint32_t)T.ny);
-        // uniform over the wave (one terrain per wave): the step loop without
-        // the division's operand checks wherever they cannot fail
+        // uniform over the wave (one terrain per wave)
         if (T.vol_ok && !w.gflag[t])
-          dl.x = walk_drop<kCount, decltype(count_step), PREFETCH, true>(
-              a, g, x0, y0, &end, &end_cell, nullptr, 0, nullptr, count_step, &sink);
+          dl.x = walk_short<decltype(count_step), PREFETCH>(
+              a, w.vt + (size_t)t * w.vt_rows, T.max_steps, T.end_kind, g, x0, y0, &end,
+              &end_cell, count_step, &sink);
         else
-          dl.x = walk_drop<kCount, decltype(count_step), PREFETCH, false>(
+          dl.x = walk_drop<kCount, decltype(count_step), PREFETCH>(
               a, g, x0, y0, &end, &end_cell, nullptr, 0, nullptr, count_step, &sink);
         dl.w = (int)sink;  // not read: it keeps the record prefetches
         dl.y = end;
@@ -1266,18 +1464,23 @@ __global__ void tile_count_finish_kernel(const int32_t* __restrict__ part, size_
   cell_count_finish(i, k, sr, first, visit, fld, root, ter, nter);
 }
 
-// quant_t of the volume a drop of terrain t carries into step k, for every
-// terrain and step: vol_0 = 1, vol_k+1 = evap_vol(vol_k) (water.h:136), the
-// same rounding as the walk.  [terrain][rows]
-__global__ void volq_kernel(const Terrain* __restrict__ ter, int nter, int rows, int32_t* vq) {
+// The volume a drop of terrain t carries into step k, for every terrain and
+// step: vol_0 = 1, vol_k+1 = evap_vol(vol_k) (water.h:136).  vq [terrain][rows]
+// holds its quant_t, vt [terrain][rows + 1] {volume, 1 / volume}, which the walk
+// reads instead of evaluating them per lane: every lane of a wave is on the
+// same step, so the read is a scalar one.
+__global__ void volq_kernel(const Terrain* __restrict__ ter, int nter, int rows, int32_t* vq,
+                            float2* vt) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nter) return;
   const float e = ter[t].P.evapRate;
   float vol = 1.0f;
   for (int k = 0; k < rows; ++k) {
     vq[(size_t)t * rows + k] = quant_t(vol);
+    vt[(size_t)t * (rows + 1) + k] = make_float2(vol, 1.0f / vol);
     vol = evap_vol(vol, e);
   }
+  vt[(size_t)t * (rows + 1) + rows] = make_float2(vol, 1.0f / vol);
 }
 
 // Per tile: the height commits (gathered from the replay's drop-major
