@@ -125,7 +125,9 @@ typedef struct shy_terrain_desc {
    walk_block  threads per block of the walk kernels (64..1024, multiple of 64)
    walk_grid   0: one lane per drop; > 0: a persistent grid of that many blocks
                walking the wave's drops grid-stride
-   tile        cascade/blend stencil tile: 0 = 32x8, 1 = 64x4, 2 = 16x16 cells */
+   tile        cascade/blend stencil tile: 0 = 32x8, 1 = 64x4, 2 = 16x16 cells
+   With the default walk_block (256) and walk_grid (0), cycles of at most 4096
+   drops run one wave per drop instead of one lane per drop. */
 typedef struct shy_tuning {
   int walk_block;
   int walk_grid;

@@ -32,6 +32,9 @@
 //                       split over kCountSplit / kReduceSplit blocks
 // A device table of Terrain entries maps drops, cells and cascade tiles to
 // their terrain, so every kernel covers the whole ensemble in one launch.
+// A cycle of few drops (kSoloMaxDrops) runs one wave per drop and needs no
+// partition: its log ([drop][step], in slog's memory), the per-cell step
+// counts scnt, and atomics on dh and trk, which pack_kernel clears.
 // Parity p = cycle & 1 selects h and visit; the cascade/blend kernel of cycle
 // p clears visit[p^1] for the next cycle, so a cycle needs no memset and two
 // cycles form a replayable hipGraph.
@@ -94,6 +97,9 @@ struct shy_ctx {
   int32_t* tcount = nullptr;    // per-part tile counts (kCountSplit parts per tile)
   long long* tsum = nullptr;    // per-part tile sums (kReduceSplit parts per tile)
   bool tile_split = false;      // tiles split over several blocks (the part buffers are small)
+  bool solo = false;        // the cycle runs one wave per drop (kSoloMaxDrops)
+  int solo_stride = 0;      // log entries per drop then (log rows rounded up to 64)
+  int32_t* scnt = nullptr;  // [cell] its step counts then, zero between cycles
   int4* dlog = nullptr;  // [drop] how each walk ended
   bool dlog_valid = false;  // dlog holds a cycle of the current wave geometry
   int32_t* dperm = nullptr;  // [drop] the terrain's drop each walk thread takes (order_kernel)
@@ -144,6 +150,26 @@ bool ordered(const shy_ctx* c) {
   return c->drop_order < 0 ? c->total_drops >= kOrderMinDrops : c->drop_order != 0;
 }
 constexpr int kReplayBlock = 256;
+// Drops (with padding) up to which a cycle runs one wave per drop
+// (walk_solo_kernel), and the map sides it takes (its window needs unit steps
+// to move a position by at most two cells).  A cycle, one wave per drop
+// against one lane per drop and the partition: 128^2 with 512 drops 104
+// against 260 us; 256^2 with 1024 228 / 634, with 4096 280 / 544; 512^2 with
+// 512 238 / 679, with 4096 572 / 666, with 6144 726 / 655; 1024^2 with 1024
+// 286 / 759, with 4096 634 / 782, with 6144 885 / 796.
+// A launch shape or drop order that the caller asked for is one of the walk
+// with a lane per drop, and keeps that walk.
+constexpr int kSoloMaxDrops = 4096;
+constexpr int kSoloMaxSide = 1 << 22;
+constexpr int kWalkBlock = 256;  // default threads per block of the walk
+
+bool solo_cycle(const shy_ctx* c) {
+  if (c->total_drops < 1 || c->total_drops > kSoloMaxDrops) return false;
+  if (c->tune.walk_block != kWalkBlock || c->tune.walk_grid != 0 || c->drop_order > 0) return false;
+  for (const Terrain& t : c->ter)
+    if (t.nx > kSoloMaxSide || t.ny > kSoloMaxSide) return false;
+  return true;
+}
 
 std::string g_noctx_err;
 
@@ -333,12 +359,24 @@ size_t part_geometry(const shy_ctx* c, int walk_block, std::vector<Terrain>* t, 
 // Size the logs, the partition and the per-drop buffers for the current
 // drops (never inside a capture).
 int ensure_wave(shy_ctx* c) {
-  const size_t need = wave_steps(c);
+  size_t need = wave_steps(c);
   const size_t need_d = (size_t)std::max(c->total_drops, 1);
   if (need > (size_t)INT32_MAX - 16384)  // slot indices plus a round stay in int
     return fail(c, SHY_ERR_ARG, "drops x (maxAge+1) exceeds 2^31 log slots per wave");
   const int drops = std::max(c->total_drops, 1);
   const int rows = (int)(need / (size_t)drops);
+  const bool solo = solo_cycle(c);
+  const int solo_stride = (rows + 63) / 64 * 64;
+  if (solo != c->solo || (solo && solo_stride != c->solo_stride)) drop_graph(c);
+  c->solo = solo;
+  c->solo_stride = solo_stride;
+  if (solo) {
+    need = std::max(need, (size_t)drops * solo_stride);
+    if (!c->scnt) {
+      HIPCHK(c, hipMalloc(&c->scnt, c->n * sizeof(int32_t)));
+      HIPCHK(c, hipMemsetAsync(c->scnt, 0, c->n * sizeof(int32_t), c->stream));
+    }
+  }
   // The walk itself counts steps per tile (an LDS histogram per block) when
   // its blocks can be the partition blocks: one drop per thread (no
   // persistent grid), blocks inside one terrain (one terrain, or a block
@@ -500,6 +538,14 @@ WaveArgs wave_args(shy_ctx* c, int p) {
   w.dlog = c->dlog;
   w.vt = c->vt;
   w.vt_rows = c->vq_rows + 1;
+  w.solo = c->slog;
+  w.solo_stride = c->solo_stride;
+  w.scnt = c->scnt;
+  w.dh = c->dh;
+  w.td = c->trk;
+  w.tmx = c->trk + c->n;
+  w.tmy = c->trk + 2 * c->n;
+  w.vq = c->vq;
   w.steps = c->wsteps;
   w.hist = c->hist;
   w.perm = ordered(c) ? c->dperm : nullptr;
@@ -522,6 +568,27 @@ int launch_cascade(shy_ctx* c, const CascArgs& a) {
   return SHY_OK;
 }
 
+// the cascade/blend stencil of the cycle of parity p
+int launch_stencil(shy_ctx* c, int p) {
+  CascArgs a;
+  const int q = p ^ 1;
+  a.ter = c->d_ter;
+  a.nter = (int)c->ter.size();
+  a.h_in = c->h[p];
+  a.h_out = c->h[q];
+  a.dh = c->dh;
+  a.visit = c->visit[p];
+  a.td = c->trk;
+  a.tmx = c->trk + c->n;
+  a.tmy = c->trk + 2 * c->n;
+  a.visit_clear = c->visit[q];
+  a.fld = c->fld;
+  a.erf_a = c->erf_a;
+  a.state = c->state;
+  a.gflag = c->gflag;
+  return launch_cascade(c, a);
+}
+
 // One cycle of every terrain.  ev, when given, receives events after the
 // walk-record pack, the count walk, the partition + tile counts and the
 // commit replay.  ensure_wave(c) must have sized the wave buffers.
@@ -537,13 +604,36 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
     const size_t nrec = (size_t)c->pack_recs;
     pack_kernel<<<(unsigned)((nrec + 255) / 256), 256, 0, c->stream>>>(c->d_ter, nter, nrec,
                                                                         c->h[p], c->fld, c->pack,
-                                                                        c->gflag);
-    if (ordered(c))
+                                                                        c->gflag,
+                                                                        c->solo ? c->dh : nullptr,
+                                                                        c->trk, n);
+    if (ordered(c) && !c->solo)
       order_kernel<<<c->order_chunks, 1024, 0, c->stream>>>(c->d_ter, nter, c->total_drops, bs, c->state,
                                                  c->dperm);
     HIPCHK(c, hipGetLastError());
   }
   if (ev) HIPCHK(c, hipEventRecord(ev[0], c->stream));
+  bool root = false;
+  for (const Terrain& T : c->ter) root = root || T.has_root;
+  if (c->solo) {
+    // one wave per drop (kSoloMaxDrops)
+    const unsigned nb = (unsigned)((c->total_drops + 3) / 4);
+    walk_solo_kernel<<<(unsigned)((c->total_drops + kSoloWaves - 1) / kSoloWaves),
+                       2 * kSoloWaves * 64, 0, c->stream>>>(w);
+    HIPCHK(c, hipGetLastError());
+    c->dlog_valid = true;
+    if (ev) HIPCHK(c, hipEventRecord(ev[1], c->stream));
+    solo_cells_kernel<<<(unsigned)((n + 255) / 256), 256, 0, c->stream>>>(
+        n, c->scnt, c->sr, c->first, c->visit[p], c->fld, c->root, c->d_ter, nter);
+    if (ev) HIPCHK(c, hipEventRecord(ev[2], c->stream));
+    if (root)
+      replay_solo_kernel<true><<<nb, 256, 0, c->stream>>>(w);
+    else
+      replay_solo_kernel<false><<<nb, 256, 0, c->stream>>>(w);
+    HIPCHK(c, hipGetLastError());
+    if (ev) HIPCHK(c, hipEventRecord(ev[3], c->stream));
+    return launch_stencil(c, p);
+  }
   if (walk) {
     // the record prefetch pays where every drop runs at once (the walk is
     // bound by its chain's latency): the same waves the drop order leaves off
@@ -617,8 +707,6 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
   HIPCHK(c, hipGetLastError());
   if (ev) HIPCHK(c, hipEventRecord(ev[2], c->stream));
   if (walk) {
-    bool root = false;
-    for (const Terrain& T : c->ter) root = root || T.has_root;
     const unsigned nb = (unsigned)((c->total_drops + kReplayBlock - 1) / kReplayBlock);
     if (root)
       replay_kernel<true><<<nb, kReplayBlock, 0, c->stream>>>(w);
@@ -639,23 +727,7 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
         c->deposit, n, c->dh, c->trk, c->trk + n, c->trk + 2 * n, nullptr);
   }
   HIPCHK(c, hipGetLastError());
-  CascArgs a;
-  const int q = p ^ 1;
-  a.ter = c->d_ter;
-  a.nter = nter;
-  a.h_in = c->h[p];
-  a.h_out = c->h[q];
-  a.dh = c->dh;
-  a.visit = c->visit[p];
-  a.td = c->trk;
-  a.tmx = c->trk + n;
-  a.tmy = c->trk + 2 * n;
-  a.visit_clear = c->visit[q];
-  a.fld = c->fld;
-  a.erf_a = c->erf_a;
-  a.state = c->state;
-  a.gflag = c->gflag;
-  return launch_cascade(c, a);
+  return launch_stencil(c, p);
 }
 
 int refresh_erf(shy_ctx* c) {
@@ -837,7 +909,7 @@ int shy_destroy(shy_ctx* c) {
   drop_graph(c);
   void* ptrs[] = {c->h[0], c->h[1], c->fld, c->root, c->visit[0], c->visit[1], c->first,
                   c->sr, c->dh, c->trk, c->deposit, c->slog, c->strk, c->qb, c->ent, c->gflag,
-                  c->vq, c->vt, c->tcount, c->tsum, c->hist, c->hbsum, c->tstart, c->dlog, c->wsteps, c->dperm, c->tsteps, c->veg_px, c->veg_py, c->veg_alive, c->veg_cflag,
+                  c->vq, c->vt, c->scnt, c->tcount, c->tsum, c->hist, c->hbsum, c->tstart, c->dlog, c->wsteps, c->dperm, c->tsteps, c->veg_px, c->veg_py, c->veg_alive, c->veg_cflag,
                   c->veg_cx, c->veg_cy, c->veg_units, c->veg_st, c->veg_size, c->pack, c->d_ter, c->state, c->erf_a, c->part, c->perms, c->trace_buf,
                   c->trace_n, c->drop_buf};
   for (void* q : ptrs)

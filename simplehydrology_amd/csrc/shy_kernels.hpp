@@ -53,6 +53,10 @@
 //                        applies the quantised transfers, blends
 //                        discharge/momentum (world.h:80-86), refreshes
 //                        erf(0.4 d) and clears the other parity's marks.
+//
+// Cycles of few drops take walk_solo_kernel, solo_cells_kernel and
+// replay_solo_kernel between the pack and the stencil instead: one wave per
+// drop, counts and commits by integer atomics, the same results.
 #pragma once
 
 #include "shy_device.hpp"
@@ -142,6 +146,14 @@ struct WaveArgs {
   int32_t* qb;        // [drop][step] height commit of the step, 2^-20 (replay)
   int qstride;        // qb's stride per drop: log rows rounded up to kReplayDepth
   const float* __restrict__ sr;   // burst scale per cell (tile_count_kernel)
+  // waves of one drop (walk_solo_kernel): [drop][solo_stride] {start cell, c_eq
+  // bits}, the per-cell step counts and the accumulators of the commits
+  int2* solo;
+  int solo_stride;
+  int32_t* scnt;
+  int32_t* dh;
+  long long *td, *tmx, *tmy;
+  const int32_t* __restrict__ vq;  // [terrain][vt_rows - 1] quantised volume track
   int4* dlog;         // [drop] {steps, end kind, end cell, unused}
   const float2* __restrict__ vt;  // [terrain][vt_rows] {volume, 1 / volume} of a drop's step (volq_kernel)
   int vt_rows;
@@ -231,11 +243,13 @@ __device__ inline void block_add_stats(long long (&v)[NC], long long* out) {
 // ------------------------------------------------------------------ walk
 // sqrt(x) and 1/x, correctly rounded, in 5 and 3 instructions: the hardware
 // approximation and one FMA-based correction.  Equal to __builtin_sqrtf and
-// to the division for every float in [2^-100, 2^100] (all 1.7e9 of them
+// to the division for every float in [2^-100, 2^126) (all 1.9e9 of them
 // compared on the device); outside it, and for 0, not used.  The full
 // sequences (about 14 and 11 instructions each, four and three of them per
 // step) were 40% of the 220 VALU instructions of a walk step, which are 880 of
-// its 1540 cycles at 256^2 and of its 2060 at 1024^2.
+// its 1540 cycles at 256^2 and of its 2060 at 1024^2.  (1/sqrt(x) from the
+// root's own approximation instead of a second one is wrong for one mantissa;
+// with that excluded by a test it was no faster.)
 __device__ inline float sqrt_short(float x) {
   const float y = __builtin_amdgcn_rsqf(x);
   const float g = x * y, h = 0.5f * y;
@@ -246,11 +260,6 @@ __device__ inline float rcp_short(float x) {
   return __builtin_fmaf(__builtin_fmaf(-x, q, 1.0f), q, q);
 }
 
-// a squared speed outside the short root's range (0 is fine: not normalised)
-__device__ inline bool short_s2_bad(float s2) {
-  return (s2 > 0x1p100f) | ((s2 < 0x1p-100f) & (s2 != 0.0f));
-}
-
 // v_cvt_i32_f32: truncation, saturating, NaN gives 0
 __device__ inline int cvt_i32(float v) {
   int r;
@@ -259,12 +268,12 @@ __device__ inline int cvt_i32(float v) {
 }
 
 // The same values with the short root and reciprocal and without branches.
-// Returns false where an operand lies outside their range (the caller then
-// runs step_coupling); the cell's flow satisfies short_flow_ok,
-// momentumTransfer short_transfer_ok and vol lies in [2^-60, 1].  mt =
-// lodsize * momentumTransfer.
-//  * |f| > 0 iff rf > 0 (pack_kernel sets rf to 0 otherwise; with |fx|, |fy|
-//    <= 2^60 it cannot underflow); sqrt(s2) > 0 iff s2 > 0.
+// Returns false where an operand lies outside their range or a speed is NaN
+// (the caller then runs step_coupling); the cell's flow satisfies
+// short_flow_ok, momentumTransfer short_transfer_ok and vol lies in [2^-60, 1].
+// mt = lodsize * momentumTransfer.
+//  * sqrt(s2) > 0 iff s2 > 0; |f| > 0 iff rf > 0 (pack_kernel sets rf to 0
+//    otherwise), and with rf = 0 the numerator and c are 0.
 //  * mt dt / (vol + d) is the correctly rounded quotient by Markstein's
 //    theorem (markstein_div) for 2^-60 <= |mt dt| <= 2^60, and 2^-60 <= vol +
 //    d <= 2^60 holds.  The sign of a zero quotient may differ from the
@@ -273,6 +282,9 @@ __device__ inline int cvt_i32(float v) {
 //    the sign of a zero (sums with a position, products that are quantised).
 //  * without coupling c = 0, and adding 0 f (f finite) changes nothing but a
 //    zero's sign.
+//  * The range test reads exponents (v_frexp_exp, 0 for a zero, which is in
+//    range): s2, u2 >= 2^-100 and |mt dt| >= 2^-60; s2 > 2^126 makes u2 NaN or
+//    at least as large.
 __device__ inline bool step_coupling_short(float mt, float vol, float d, float fx, float fy,
                                            float rf, float& sx, float& sy) {
   const float s2 = sx * sx + sy * sy;
@@ -281,9 +293,7 @@ __device__ inline bool step_coupling_short(float mt, float vol, float d, float f
   const float a = mt * dt, b = vol + d, y = rcp_short(b);
   const float q = a * y;
   float c = __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
-  const bool on = (rf > 0.0f) & (s2 > 0.0f);
-  c = on ? c : 0.0f;
-  const bool bad = on & (__builtin_fabsf(a) < 0x1p-60f) & (a != 0.0f);
+  c = s2 > 0.0f ? c : 0.0f;
   const float ux = sx + c * fx, uy = sy + c * fy;
   const float u2 = ux * ux + uy * uy;
   const float k2 = kLod * __builtin_sqrtf(2.0f);  // lodsize*sqrt(2.0f)
@@ -291,7 +301,10 @@ __device__ inline bool step_coupling_short(float mt, float vol, float d, float f
   const bool move = u2 > 0.0f;
   sx = move ? k2 * (ux * r) : ux;
   sy = move ? k2 * (uy * r) : uy;
-  return !(bad | short_s2_bad(s2) | short_s2_bad(u2));
+  const int e1 = __builtin_amdgcn_frexp_expf(s2), e2 = __builtin_amdgcn_frexp_expf(u2);
+  const int ea = __builtin_amdgcn_frexp_expf(a) - 41;
+  const int e12 = e1 < e2 ? e1 : e2, em = e12 < ea ? e12 : ea;
+  return (int)(em > -100) & (int)(u2 < 0x1p100f);
 }
 
 // One cache line per step: {h, h(x-1), h(x+1), h(y-1)}, {h(y+1), mx, my, d},
@@ -587,7 +600,7 @@ __device__ int walk_short(const WalkArgs& a, const float2* __restrict__ vt, int 
       py = py + sy;
     }
     const int jx = cvt_i32(px), jy = cvt_i32(py);
-    const bool ex = !((px > -1.0f) & (px < fnx) & (py > -1.0f) & (py < fny));
+    const bool ex = !((int)(px > -1.0f) & (int)(px < fnx) & (int)(py > -1.0f) & (int)(py < fny));
     const int j = cell_of(jx, jy);
     // off the map the record is not used; loading the current cell's keeps
     // the load unconditional, so its wait is counted exactly
@@ -647,9 +660,12 @@ __device__ int walk_short(const WalkArgs& a, const float2* __restrict__ vt, int 
 // One thread per record, numbered over all terrains in record order
 // (Terrain::pack_off), so that four consecutive threads write one 128-byte
 // line; padding records (odd nx or ny) are skipped and never read.
+// clear_dh, clear_trk: the commit accumulators of a cycle of few drops
+// (clear_n cells; trk three arrays), cleared here; else null.
 __global__ void pack_kernel(const Terrain* __restrict__ ter, int nter, size_t nrec,
                             const float* __restrict__ h, const float4* __restrict__ fld,
-                            float4* pack, int* gflag) {
+                            float4* pack, int* gflag, int32_t* clear_dh, long long* clear_trk,
+                            size_t clear_n) {
   const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= nrec) return;
   const int t = find_terrain(nter, (long long)g, [&](int q) { return ter[q].pack_off; });
@@ -677,6 +693,13 @@ __global__ void pack_kernel(const Terrain* __restrict__ ter, int nter, size_t nr
   if (!(markstein_num_ok(a0) && markstein_num_ok(a2) && short_flow_ok(f.x, f.y, f.z)))
     gflag[t] = 1;
   const float rf = f.x * f.x + f.y * f.y > 0.0f ? inv_len(f.x, f.y) : 0.0f;
+  if (clear_dh) {
+    const size_t ci = (size_t)T.cell_off + i;
+    clear_dh[ci] = 0;
+    clear_trk[ci] = 0;
+    clear_trk[clear_n + ci] = 0;
+    clear_trk[2 * clear_n + ci] = 0;
+  }
   pack[2 * g] = make_float4(hc, a0, a2, f.w);
   pack[2 * g + 1] = make_float4(f.x, f.y, f.z, rf);
 }
@@ -768,6 +791,269 @@ __global__ void __launch_bounds__(1024) walk_kernel(WaveArgs w) {
     __syncthreads();
     for (int r = threadIdx.x; r < wn; r += blockDim.x) w.hist[hbase + (long long)r * hstride] = th[r];
   }
+}
+
+// ------------------------------------------------- cycles of few drops
+// A cycle of up to a few thousand drops leaves the chip nearly empty when
+// every lane walks a drop (1024 drops: 16 waves on 1024 SIMDs), and its time is
+// the length of one drop's chain.  Here a wave walks one drop and its 64 lanes
+// shorten the chain:
+//  * The lanes hold the records of the 8x8 cells around the drop, loaded two
+//    steps before they are used: a step of length at most sqrt(2) (1 + 2^-22)
+//    moves at most 2 cells along an axis and two steps at most 3, so the
+//    window issued at one step (origin 3 cells back on both axes) holds the
+//    cell the drop reaches two steps later.  No step waits for memory; the
+//    record comes by v_readlane.
+//  * What nothing waits for (c_eq, the tracks, the log, the count of the cell)
+//    is a second wave's work: the walker leaves its position and speed of
+//    every step in LDS, its helper takes them 64 steps at a time.  Memory
+//    operations of one wave complete in issue order, so in the walker itself
+//    the helper's atomics would hold up the windows behind them.
+//  * One wave issues an instruction about every 4 cycles, so the walker's step
+//    is as short as it can be made: no per-step bounds (a window cell off the
+//    map loads some record, which no step on the map reads), and a drop that
+//    left the map is noticed every second step.
+// The counts and, in the replay, the commits go straight to the map in integer
+// atomics (order-free, so the results are those of the partitioned path): at
+// 27 G atomics/s a cycle of 0.5 M steps needs about 0.1 ms of them, spread
+// under the two chains, where the partition's seven launches took 0.2 ms.
+// Measured (a cycle): see kSoloMaxDrops.
+constexpr int kSoloWaves = 4;   // drops per block
+constexpr int kSoloRing = 128;  // steps of a drop in LDS: two batches of 64
+
+struct SoloShared {
+  float4 ring[kSoloWaves][kSoloRing];  // {position, speed} at the start / after the step
+  // 4 x the steps in the ring so far (whole batches until the walk is over)
+  // plus 0: more to come, 1: over on the map, 2: over off the map
+  int ready[kSoloWaves];
+  int taken[kSoloWaves];  // batches the helper has read
+};
+
+__device__ inline int lds_load_acquire(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline void lds_store_release(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// byte offset of cell (x, y)'s record, in 32-byte units: pack_rec with one
+// multiply and no masks (2 (x >> 1) + (x & 1) = x)
+__device__ inline int solo_rec(int x, int y, int stride4) {
+  return __mul24(x >> 1, stride4) + ((x << 1) + (((y >> 1) << 1) + y));
+}
+
+// The walker.  SHORT: the arithmetic of walk_short; else the full sequences.
+// Both need positions below 2^22 (window, exact unit steps); the host checks.
+template <bool SHORT>
+__device__ __forceinline__ void solo_walker(const WaveArgs& w, const Terrain& T,
+                                            const float2* __restrict__ vt, SoloShared& sh,
+                                            int slot, int x0, int y0) {
+  const int lane = threadIdx.x & 63;
+  const int nx = T.nx, ny = T.ny;
+  const int stride4 = (((ny + 1) >> 1) - 1) * 4;
+  const int nrec = ((nx + 1) >> 1) * ((ny + 1) >> 1) * 4;
+  const float mt = kLod * T.P.momentumTransfer;
+  const char* pack = reinterpret_cast<const char*>(w.pack + 2 * T.pack_off);
+  const int lx = (lane >> 3) - 3, ly = (lane & 7) - 3;
+  // the window around (x, y): lane l holds cell (x - 3 + l / 8, y - 3 + l % 8)
+  struct Win {
+    float4 a, b;
+    int base;  // lane of cell (0, 0)
+  };
+  auto load_win = [&](Win& v, int ix, int iy) {
+    v.base = 27 - ix * 8 - iy;
+    int r = solo_rec(ix + lx, iy + ly, stride4);
+    r = r < 0 ? 0 : (r > nrec - 1 ? nrec - 1 : r);
+    const size_t o = (uint32_t)r << 5;
+    v.a = *reinterpret_cast<const float4*>(pack + o);
+    v.b = *reinterpret_cast<const float4*>(pack + o + 16);
+  };
+  auto pick = [&](float f, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), l));
+  };
+  Win A, B;
+  load_win(A, x0, y0);
+  int ix = x0, iy = y0;
+  float px = (float)x0, py = (float)y0, sx = 0.0f, sy = 0.0f;
+  float n0, n2, mx, my, d, rf;
+  auto take = [&](const Win& v, int x, int y) {
+    const int l = x * 8 + y + v.base;
+    n0 = pick(v.a.y, l);
+    n2 = pick(v.a.z, l);
+    mx = pick(v.b.x, l);
+    my = pick(v.b.y, l);
+    d = pick(v.b.z, l);
+    rf = pick(v.b.w, l);
+  };
+  take(A, ix, iy);
+  const int last = T.max_steps;
+  float2 lvol = make_float2(1.0f, 1.0f);  // lane k: the volume of step k of the batch
+  // Step kk of the batch: the next record comes from X, the window around the
+  // present position goes into Y.  Negative when the drop left the map (what
+  // is computed after that is never read).
+  auto step = [&](int kk, const Win& X, Win& Y, float4* slotp) {
+    load_win(Y, ix, iy);
+    const float vol = pick(lvol.x, kk), yv = pick(lvol.y, kk);
+    int nan = 0;
+    if constexpr (SHORT) {
+      const float q0 = n0 * yv, q1 = n2 * yv;
+      const float gx = sx + __builtin_fmaf(__builtin_fmaf(-q0, vol, n0), yv, q0);
+      const float gy = sy + __builtin_fmaf(__builtin_fmaf(-q1, vol, n2), yv, q1);
+      sx = gx;
+      sy = gy;
+      // (a NaN speed also comes here)
+      if (__builtin_expect(!step_coupling_short(mt, vol, d, mx, my, rf, sx, sy), 0)) {
+        float ux = 0.0f, uy = 0.0f;
+        sx = gx;
+        sy = gy;
+        step_coupling(T.P, vol, d, mx, my, rf, sx, sy, ux, uy);
+        nan = -__builtin_amdgcn_readfirstlane((int)__builtin_isunordered(sx, sy));
+      }
+    } else {
+      float ux = 0.0f, uy = 0.0f;
+      sx = sx + div_rcp(n0, vol, yv);
+      sy = sy + div_rcp(n2, vol, yv);
+      step_coupling(T.P, vol, d, mx, my, rf, sx, sy, ux, uy);
+      nan = -__builtin_amdgcn_readfirstlane((int)__builtin_isunordered(sx, sy));
+    }
+    if (lane == 0) *slotp = make_float4(px, py, sx, sy);
+    px = px + sx;
+    py = py + sy;
+    ix = __builtin_amdgcn_readfirstlane(cvt_i32(px));
+    iy = __builtin_amdgcn_readfirstlane(cvt_i32(py));
+    take(X, ix, iy);
+    // negative iff ix or iy lies outside [0, nx) or [0, ny)
+    return ix | (nx - 1 - ix) | iy | (ny - 1 - iy) | nan;
+  };
+  float2 nvol = vt[lane < last ? lane : last];  // vt has max_steps + 1 entries at least
+  for (int k0 = 0;; k0 += 64) {
+    // the batch's volumes, loaded a batch ahead; the empty statement takes
+    // them here: pending at the loop's entry they would make its first wait
+    // cover the windows in flight, on every turn
+    lvol = nvol;
+    asm volatile("" : "+v"(lvol.x), "+v"(lvol.y));
+    nvol = vt[k0 + 64 + lane < last ? k0 + 64 + lane : last];
+    // the ring half this batch goes into was read
+    if (k0 >= kSoloRing)
+      while (lds_load_acquire(&sh.taken[slot]) < k0 / 64 - 1) __builtin_amdgcn_s_sleep(1);
+    float4* ring = &sh.ring[slot][k0 & 64];
+    const int m = last - k0 < 64 ? last - k0 : 64;
+    int o1 = 0, o2 = 0, kk = 0;
+    // no memory operation but the windows in this loop
+    for (; kk < m; kk += 2) {
+      o1 = step(kk, A, B, ring + kk);
+      o2 = step(kk + 1, B, A, ring + kk + 1);
+      if ((o1 | o2) < 0) break;
+    }
+    int cnt = m, end = k0 + m >= last ? 1 : 0;
+    if (kk < m) {  // left in this pair (the second step counts if there is one)
+      if (o1 < 0) {
+        cnt = kk + 1;
+        end = 2;
+      } else if (kk + 1 < m) {
+        cnt = kk + 2;
+        end = 2;
+      }
+    }
+    if (lane == 0) lds_store_release(&sh.ready[slot], (k0 + cnt) * 4 + end);
+    if (end) return;
+  }
+}
+
+// The helper: logs and counts the walker's steps.
+__device__ __forceinline__ void solo_helper(const WaveArgs& w, const Terrain& T,
+                                            const float2* __restrict__ vt, SoloShared& sh,
+                                            int slot, int g, uint32_t cid) {
+  const int lane = threadIdx.x & 63;
+  const int ny = T.ny, stride4 = (((ny + 1) >> 1) - 1) * 4;
+  const char* pack = reinterpret_cast<const char*>(w.pack + 2 * T.pack_off);
+  int2* log = w.solo + (size_t)g * w.solo_stride;
+  for (int k0 = 0;; k0 += 64) {
+    int v;
+    while (((v = lds_load_acquire(&sh.ready[slot])) & 3) == 0 && (v >> 2) < k0 + 64)
+      __builtin_amdgcn_s_sleep(2);
+    v = __builtin_amdgcn_readfirstlane(v);
+    const int steps = v >> 2, cnt = steps - k0 < 64 ? steps - k0 : 64;
+    const bool over = (v & 3) != 0 && steps <= k0 + 64;
+    const float4 s = sh.ring[slot][(k0 & 64) + lane];
+    if (lane == 0) lds_store_release(&sh.taken[slot], k0 / 64 + 1);
+    int end_cell = (int)cid;  // of a drop that takes no step
+    if (lane < cnt) {
+      const int x = cvt_i32(s.x), y = cvt_i32(s.y);
+      const bool ex = over && (v & 3) == 2 && lane + 1 == cnt;
+      // where the step led (the walker's own sum)
+      const int jx = ex ? x : cvt_i32(s.x + s.z), jy = ex ? y : cvt_i32(s.y + s.w);
+      const float4 ra =
+          *reinterpret_cast<const float4*>(pack + ((size_t)(uint32_t)solo_rec(x, y, stride4) << 5));
+      const float hn = *reinterpret_cast<const float*>(
+          pack + ((size_t)(uint32_t)solo_rec(jx, jy, stride4) << 5));
+      const float vol = vt[k0 + lane].x;
+      const float h2 = ex ? (float)((double)ra.x - 0.002) : hn;   // water.h:120-124
+      float c_eq = (1.0f + T.P.entrainment * ra.w) * (ra.x - h2);  // water.h:127
+      if (c_eq < 0) c_eq = 0;
+      const int cell = (int)T.cell_off + x * ny + y;
+      log[k0 + lane] = make_int2(cell, __float_as_int(c_eq));
+      atomic_add_i32(&w.scnt[cell], 1);
+      // the momentum tracks, water.h:116-117
+      atomic_add_i64(&w.tmx[cell], quant_t(vol * s.z));
+      atomic_add_i64(&w.tmy[cell], quant_t(vol * s.w));
+      end_cell = jx * ny + jy;
+    }
+    if (over) {
+      end_cell = __builtin_amdgcn_readlane(end_cell, cnt > 0 ? cnt - 1 : 0);
+      if (lane == 0) {
+        w.dlog[g] = make_int4(steps, (v & 3) == 2 ? (int)kEndExit : T.end_kind, end_cell, 0);
+        w.steps[g] = steps;
+        if (steps > 0) {  // as walk_kernel
+          atomic_add_i32(&w.first[T.cell_off + cid], 1);
+          if ((v & 3) != 2) w.visit[T.cell_off + end_cell] = 1;
+        }
+      }
+      return;
+    }
+  }
+}
+
+// kSoloWaves drops per block: waves 0 .. kSoloWaves - 1 walk, the others help
+// (wave i and its helper i + 4 share a SIMD).  Every wait ends: a walker's
+// steps are bounded and wait only for its helper, which takes every batch as
+// it comes.
+__global__ void __launch_bounds__(2 * kSoloWaves * 64) walk_solo_kernel(WaveArgs w) {
+  __shared__ SoloShared sh;
+  if (threadIdx.x < kSoloWaves) {
+    sh.ready[threadIdx.x] = 0;
+    sh.taken[threadIdx.x] = 0;
+  }
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int slot = wave & (kSoloWaves - 1);
+  const int g = (int)blockIdx.x * kSoloWaves + slot;
+  if (g >= w.total_drops) return;
+  const int lane = threadIdx.x & 63;
+  const int t = __builtin_amdgcn_readfirstlane(
+      find_terrain(w.nter, g, [&](int k) { return (long long)w.ter[k].drop_off; }));
+  const Terrain T = w.ter[t];
+  const int loc = g - T.drop_off;
+  const uint32_t ncell = (uint32_t)T.nx * (uint32_t)T.ny;
+  const uint32_t cid = __builtin_amdgcn_readfirstlane(
+      spawn_cell(cycle_key(T.seed, T.id, w.state->cycle), (uint32_t)loc, ncell));
+  if (loc >= T.drops || !((double)w.h[T.cell_off + cid] >= 0.1)) {  // world.h:71-72
+    if (wave == slot && lane == 0) {
+      w.dlog[g] = make_int4(0, loc >= T.drops ? kEndPad : kEndSkipped, 0, 0);
+      w.steps[g] = 0;
+    }
+    return;
+  }
+  const float2* vt = w.vt + (size_t)t * w.vt_rows;
+  if (wave != slot) {
+    solo_helper(w, T, vt, sh, slot, g, cid);
+    return;
+  }
+  const int x0 = (int)(cid / (uint32_t)T.ny), y0 = (int)(cid % (uint32_t)T.ny);
+  if (T.vol_ok && !w.gflag[t])
+    solo_walker<true>(w, T, vt, sh, slot, x0, y0);
+  else
+    solo_walker<false>(w, T, vt, sh, slot, x0, y0);
 }
 
 // The commits of every drop from its step log.  The arithmetic is the
@@ -1462,6 +1748,162 @@ __global__ void tile_count_finish_kernel(const int32_t* __restrict__ part, size_
 #pragma unroll
   for (int s = 0; s < S; ++s) k += part[(t * S + s) * kTileCells + j];
   cell_count_finish(i, k, sr, first, visit, fld, root, ter, nter);
+}
+
+// Between walk and replay of a cycle of few drops, one thread per cell: the
+// burst scale and the cascade site from the cell's step count, the counts
+// cleared.
+__global__ void solo_cells_kernel(size_t n, int32_t* scnt, float* sr, int32_t* first,
+                                  uint8_t* visit, const float4* __restrict__ fld,
+                                  const float* __restrict__ root,
+                                  const Terrain* __restrict__ ter, int nter) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int k = scnt[i];
+  if (k == 0) return;  // no step starts here: no replay reads its scale, and first is 0
+  scnt[i] = 0;
+  cell_count_finish(i, k, sr, first, visit, fld, root, ter, nter);
+}
+
+// quant_h for a replay's chain: the same integer (NaN gives 0, the clamp on
+// the rounded integer instead of the float)
+__device__ inline int quant_h_sat(float v) {
+  int q = cvt_i32(__builtin_rintf(v * kHQ));
+  q = q < -1073741824 ? -1073741824 : q;
+  return q > 1073741824 ? 1073741824 : q;
+}
+
+// value of the lane below (lane 0: old)
+__device__ inline float lane_below(float old, float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v),
+                                                    0x138 /* wave_shr:1 */, 0xf, 0xf, false));
+}
+__device__ inline double lane_below(double old, double v) {
+  const long long o = __double_as_longlong(old), x = __double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)o, (int)x, 0x138, 0xf, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(o >> 32), (int)(x >> 32), 0x138,
+                                                            0xf, 0xf, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The commit replay of a cycle of few drops: one wave per drop, lane k holding
+// step k of every 64.  Everything but the sediment recurrence (log, burst
+// scale, root density, commits) is loaded and committed 64 steps at a time.
+// The recurrence runs as a systolic shift: each iteration every lane takes the
+// sediment its lower neighbour ended with and does its own step; lane 0's
+// input is the carry, so lane u holds its final values from iteration u on, and
+// after as many iterations as steps all do.  One step costs the recurrence's
+// own ~20 instructions, where a lane per drop stalled 560 of its 890 cycles
+// per step on the L1 fill of its 64 gathers.  Operation for operation
+// replay_kernel's arithmetic.
+template <bool ROOT>
+__global__ void __launch_bounds__(256) replay_solo_kernel(WaveArgs w) {
+  __shared__ int bsteps;
+  LaneStats S;
+  long long walked = 0, skipped = 0;
+  const int lane = threadIdx.x & 63;
+  const int g = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  // drop ranges are padded to at least 64 drops: a block's four share a terrain
+  const int t = __builtin_amdgcn_readfirstlane(
+      find_terrain(w.nter, (int)blockIdx.x * 4,
+                   [&](int k) { return (long long)w.ter[k].drop_off; }));
+  if (threadIdx.x == 0) bsteps = 0;
+  __syncthreads();
+  if (g < w.total_drops) {
+    const Terrain T = w.ter[t];
+    const int4 dl = w.dlog[g];
+    const int n = __builtin_amdgcn_readfirstlane(dl.y <= kEndExit ? dl.x : 0);
+    if (dl.y == kEndSkipped && lane == 0) skipped = 1;
+    if (dl.y <= kEndExit) {
+      const float dep = T.P.depositionRate, e = T.P.evapRate;
+      const double ce = 1.0 - (double)e, ye = 1.0 / ce;
+      const int2* log = w.solo + (size_t)g * w.solo_stride;
+      const int32_t* vq = w.vq + (size_t)t * (w.vt_rows - 1);
+      float carry = 0.0f;
+      double gain = 0.0;
+      // a batch's entries, and the scale (and root density) of their cells,
+      // loaded one and two batches ahead; rows past the last step repeat it
+      auto row = [&](int k) { return log[k < n ? k : n - 1]; };
+      int2 ec = make_int2(0, 0), en = ec;
+      float scn = 0.0f, rtn = 0.0f;
+      int vqn = 0;
+      if (n > 0) {
+        ec = row(lane);
+        en = row(64 + lane);
+        scn = w.sr[ec.x];
+        rtn = ROOT ? w.root[ec.x] : 0.0f;
+        vqn = vq[lane < n ? lane : n - 1];
+      }
+      for (int k0 = 0; k0 < n; k0 += 64) {
+        const int2 c = ec;
+        const float sc = scn, rt = rtn;
+        const int vqk = vqn;
+        const int m = n - k0 < 64 ? n - k0 : 64;
+        float effD = dep * (1.0f - rt);  // water.h:86-87
+        if (effD < 0) effD = 0;
+        const float cq = __int_as_float(c.y);
+        int q = 0;
+        float s1 = 0.0f;
+        double gs = 0.0;
+        // (whole eights: a lane's values no longer change once they are final)
+        for (int it = 0; it < m; it += 8) {
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const float sin = lane_below(carry, s1);
+            const double gin = lane_below(gain, gs);
+            const float cdiff = cq - sin;
+            q = quant_h_sat((effD * cdiff) * sc);
+            const float sed = sin + (float)q * kHQInv;
+            s1 = evap_sed_rcp(sed, ce, ye);
+            gs = gin + ((double)s1 - (double)sed);
+          }
+        }
+        carry = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s1), m - 1));
+        gain = __shfl(gs, m - 1, 64);
+        if (k0 + 64 >= n) {  // the last batch
+          if (lane < m) {
+            S.walk_dh -= q;
+            atomic_add_i32(&w.dh[c.x], -q);
+            atomic_add_i64(&w.td[c.x], vqk);
+          }
+          break;
+        }
+        // the next batch's loads go out before this batch's commits: memory
+        // operations complete in issue order, and the commits are
+        // unconditional, so that the next batch's waits are counted exactly
+        // and cover none of them
+        ec = en;
+        scn = w.sr[ec.x];
+        rtn = ROOT ? w.root[ec.x] : 0.0f;
+        en = row(k0 + 128 + lane);
+        vqn = vq[k0 + 64 + lane < n ? k0 + 64 + lane : n - 1];
+        S.walk_dh -= q;
+        atomic_add_i32(&w.dh[c.x], -q);
+        atomic_add_i64(&w.td[c.x], vqk);
+      }
+      if (lane == 0) {
+        walked = 1;
+        S.steps = n;
+        if (dl.y == kEndExit) {
+          S.exits = 1;
+          S.export40 = quant_40((double)carry);
+        } else {
+          const int32_t q = quant_h(carry);
+          atomic_add_i32(&w.dh[T.cell_off + dl.z], q);
+          S.walk_dh += q;
+          if (dl.y == kEndAge) S.ends_age = 1; else S.ends_vol = 1;
+        }
+        S.gain40 = quant_40(gain);
+        if (n) atomicAdd(&bsteps, n);
+      }
+    }
+  }
+  long long v[ST_CASC_MOVES] = {S.steps, walked, skipped, S.exits, S.ends_age,
+                                S.ends_vol, S.export40, S.gain40, S.walk_dh};
+  block_add_stats<ST_CASC_MOVES>(v, w.state->stats);
+  if (w.tsteps && threadIdx.x == 0 && bsteps)
+    __hip_atomic_fetch_add(&w.tsteps[t], (long long)bsteps, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The volume a drop of terrain t carries into step k, for every terrain and
