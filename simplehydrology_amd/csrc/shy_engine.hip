@@ -73,7 +73,7 @@ struct shy_ctx {
   int2* strk = nullptr;      // [step][drop] the steps' momentum tracks
   int32_t* qb = nullptr;     // [drop][step] height commits of the replay
   size_t qb_cap = 0;         // ints qb holds
-  int qstride = 0;           // qb's stride per drop (log rows rounded up to kReplayDepth)
+  int qstride = 0;           // qb's stride per drop (log rows rounded up to kReplayDepth, then 32)
   int4* ent = nullptr;       // partition entries in tile order: wave_cap start cells, then
                              // wave_cap {slot, tracks} (16 B per log slot in all)
   int32_t* vq = nullptr;     // [terrain][row] quantised volume track per step
@@ -410,7 +410,8 @@ int ensure_wave(shy_ctx* c) {
   c->part_maxw = 0;
   for (const Terrain& t : c->ter) c->part_maxw = std::max(c->part_maxw, t.part_dwidth);
   const size_t hist_need = entries + 1;
-  const int qstride = (rows + kReplayDepth - 1) / kReplayDepth * kReplayDepth;
+  const int qstride =
+      ((rows + kReplayDepth - 1) / kReplayDepth * kReplayDepth + 31) / 32 * 32;
   const size_t qb_need = (size_t)c->total_drops * qstride;
   if (qstride != c->qstride) drop_graph(c);
   c->qstride = qstride;
@@ -535,6 +536,7 @@ WaveArgs wave_args(shy_ctx* c, int p) {
   w.qb = c->qb;
   w.sr = c->sr;
   w.qstride = c->qstride;
+  w.log_rows = c->part_rows;
   w.dlog = c->dlog;
   w.vt = c->vt;
   w.vt_rows = c->vq_rows + 1;
