@@ -35,6 +35,57 @@ __host__ __device__ inline long long pack_records(int nx, int ny) {
   return (long long)((nx + 1) >> 1) * ((ny + 1) >> 1) * 4;
 }
 
+// Tile order of a terrain's cells: the index under which the step log names a
+// cell.  Blocks of 2^a x 2^b cells (64 x 64 where the sides allow), the blocks
+// x-major, so that the partition's 4096 consecutive indices are a square
+// neighbourhood in which a drop stays for tens of steps; within a block 4 x 8
+// sub-blocks, whose 32 four-byte values share one 128-byte line.  Blocks past
+// the map's end leave unused indices, at most 1/16 of the cells; a terrain too
+// small or thin for that keeps the x-major index (a = b = 0).
+// The line at 1/16: an unused index costs the tile kernels what a cell costs.
+// Measured against the x-major order, kernel times of a cycle in us: 65536
+// drops on 1024^2: scatter 229 -> 211, replay 233 -> 196, sums 233 -> 203;
+// 64 maps of 512^2 with 16384 drops each: scatter 5364 -> 4655, sums 3580 -> 3690.
+struct TileMap {
+  int a, b;      // log2 of the block's sides
+  int nyb;       // blocks along y (x-major order: ny)
+  int mxh, myh;  // the coordinate bits above the sub-block's and below the block's
+  int mxl, myl;  // the sub-block's
+};
+__host__ __device__ inline long long tile_cells(const TileMap& m, int nx, int ny) {
+  const long long px = (((long long)nx + (1 << m.a) - 1) >> m.a) << m.a;
+  const long long py = (((long long)ny + (1 << m.b) - 1) >> m.b) << m.b;
+  return px * py;
+}
+inline TileMap tile_map(int nx, int ny, bool blocks) {
+  TileMap m{6, 6, 0, 0, 0, 0, 0};
+  auto side = [](int n, int l) { return (double)((((long long)n + (1 << l) - 1) >> l) << l) / n; };
+  while (blocks && 16.0 * side(nx, m.a) * side(ny, m.b) > 17.0) {
+    if (m.a > 2 && (side(nx, m.a) >= side(ny, m.b) || m.b == 3)) --m.a;
+    else if (m.b > 3) --m.b;
+    else blocks = false;
+  }
+  if (!blocks) m.a = m.b = 0;
+  m.nyb = (int)(((long long)ny + (1 << m.b) - 1) >> m.b);
+  if (blocks) {
+    m.mxl = 3;
+    m.myl = 7;
+    m.mxh = ((1 << m.a) - 1) & ~3;
+    m.myh = ((1 << m.b) - 1) & ~7;
+  }
+  return m;
+}
+__host__ __device__ inline int tile_index(const TileMap& m, int x, int y) {
+  const int blk = (x >> m.a) * m.nyb + (y >> m.b);
+  return (blk << (m.a + m.b)) |
+         ((x & m.mxh) << m.b | (y & m.myh) << 2 | (x & m.mxl) << 3 | (y & m.myl));
+}
+__host__ __device__ inline void tile_xy(const TileMap& m, int i, int& x, int& y) {
+  const int blk = i >> (m.a + m.b), bx = blk / m.nyb, by = blk - bx * m.nyb;
+  x = (bx << m.a) | ((i >> m.b) & m.mxh) | ((i >> 3) & m.mxl);
+  y = (by << m.b) | ((i >> 2) & m.myh) | (i & m.myl);
+}
+
 // ---------------------------------------------------------------- hashing
 // SplitMix64 output function (Steele, Lea, Flood, OOPSLA 2014).
 __host__ __device__ inline uint64_t mix64(uint64_t z) {

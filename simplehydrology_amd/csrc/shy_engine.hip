@@ -28,8 +28,9 @@
 //   pack        float4x2 per cell: the count walk's 32-byte record of the
 //                       cycle's start (height, normal, flow), by pack_kernel
 //   sr          float   burst scale per cell (tile_count_kernel)
-//   tcount, tsum int32, int64x4  per-part tile counts and sums when a tile is
-//                       split over kCountSplit / kReduceSplit blocks
+//   tlist, tmulti       the tile kernels' work: parts of the tiles' entries
+//   tcount, tsum int32, int64x4  counts and sums of the parts of tiles that
+//                       have several
 // A device table of Terrain entries maps drops, cells and cascade tiles to
 // their terrain, so every kernel covers the whole ensemble in one launch.
 // A cycle of few drops (kSoloMaxDrops) runs one wave per drop and needs no
@@ -57,6 +58,7 @@ struct shy_ctx {
   Terrain* d_ter = nullptr;
   int* gflag = nullptr;      // [terrain] a gravity term out of the walk's division range (pack)
   size_t n = 0;              // cells, all terrains
+  size_t np = 0;             // indices in tile order, all terrains (Terrain::tm)
   int total_drops = 0;
   int total_tiles = 0;
   uint32_t cycle = 0;        // host mirror of state->cycle
@@ -66,6 +68,7 @@ struct shy_ctx {
   uint8_t* visit[2] = {nullptr, nullptr};
   int32_t* first = nullptr;
   float* sr = nullptr;
+  float* rootp = nullptr;    // root density in tile order (allocated with the first root)
   int32_t* dh = nullptr;
   long long* trk = nullptr;  // 3*n: d, mx, my
   int32_t* deposit = nullptr;
@@ -94,9 +97,14 @@ struct shy_ctx {
   int part_maxw = 0;         // widest partition block (drops)
   bool walk_counts = false;  // the walk builds the partition's tile counts
   int ntiles = 0;            // cell tiles of kTileCells cells
-  int32_t* tcount = nullptr;    // per-part tile counts (kCountSplit parts per tile)
-  long long* tsum = nullptr;    // per-part tile sums (kReduceSplit parts per tile)
-  bool tile_split = false;      // tiles split over several blocks (the part buffers are small)
+  int parts = 0;                // parts of the tiles' entries (tile_parts_kernel) that the
+                                // buffers below hold
+  int list_cap = 0;             // parts tlist holds
+  TileParts* tparts = nullptr;
+  TilePart* tlist = nullptr;
+  TileMulti* tmulti = nullptr;
+  int32_t* tcount = nullptr;    // counts of the parts of tiles of several (2 x parts slots)
+  long long* tsum = nullptr;    // their sums
   bool solo = false;        // the cycle runs one wave per drop (kSoloMaxDrops)
   int solo_stride = 0;      // log entries per drop then (log rows rounded up to 64)
   int32_t* scnt = nullptr;  // [cell] its step counts then, zero between cycles
@@ -259,12 +267,20 @@ void walk_limits(Terrain& t) {
 }
 
 int layout(shy_ctx* c) {
-  long long cells = 0, drops = 0, tiles = 0, recs = 0;
+  long long cells = 0, drops = 0, tiles = 0, recs = 0, base = 0;
+  // tile order, unless its unused indices would exceed what the partition takes
+  bool blocks = true;
+  for (const Terrain& t : c->ter) base += tile_cells(tile_map(t.nx, t.ny, true), t.nx, t.ny);
+  if ((base + kTileCells - 1) / kTileCells > kPartMaxTiles) blocks = false;
+  base = 0;
   const int ty = kTileY[c->tune.tile], tx = kTileX[c->tune.tile];
   for (Terrain& t : c->ter) {
     walk_limits(t);
     t.cell_off = cells;
     t.pack_off = recs;
+    t.tm = tile_map(t.nx, t.ny, blocks);
+    t.tile_base = base;
+    base += tile_cells(t.tm, t.nx, t.ny);
     recs += pack_records(t.nx, t.ny);
     t.drop_off = (int)drops;
     t.tiles_y = (t.ny + ty - 1) / ty;
@@ -281,7 +297,8 @@ int layout(shy_ctx* c) {
     return fail(c, SHY_ERR_ARG, "context too large: at most 2^27 cells over all terrains");
   c->total_drops = (int)drops;
   c->total_tiles = (int)tiles;
-  c->ntiles = (int)((cells + kTileCells - 1) / kTileCells);
+  c->np = (size_t)base;
+  c->ntiles = (int)((base + kTileCells - 1) / kTileCells);
   c->vq_dirty = true;
   c->dlog_valid = false;
   drop_graph(c);
@@ -302,13 +319,11 @@ size_t wave_steps(const shy_ctx* c) {
 // Partition blocks: at most kPartMaxBlocks, each a whole number of waves of
 // drops over all log rows (the [tile][block] matrix stays small).
 constexpr int kPartMaxBlocks = 512;
-// blocks per tile in the tile kernels: the largest tiles hold several times
-// the mean's entries; the counts split 4 ways, the sums (whose parts are
-// 32 B per cell) 2 ways (1024^2 cycle: 1.185 ms at 4 and 4, 1.171 at 2 and 2,
-// 1.165 at 4 and 2)
-constexpr int kCountSplit = 4;
-constexpr int kReduceSplit = 2;
-constexpr int kTileSplitMaxTiles = 2048;
+// Parts that the tiles' entries are cut into (tile_parts_kernel): two per CU,
+// and at least kPartMin entries each (a part costs a pass over its tile's
+// cells).
+constexpr int kTileParts = 512;
+constexpr int kPartMin = 16384;
 // partition blocks up to which each takes a CU's whole LDS (the scatter's
 // rounds of 8192 entries): no more blocks than CUs
 constexpr int kBigRoundBlocks = 256;
@@ -335,8 +350,9 @@ size_t part_geometry(const shy_ctx* c, int walk_block, std::vector<Terrain>* t, 
       dwidth = std::max(kWaveDrops, (per + kWaveDrops - 1) / kWaveDrops * kWaveDrops);
     }
     const int nb = (padded + dwidth - 1) / dwidth;
-    const int lo = (int)(T.cell_off >> kTileBits);
-    const int tn = (int)((T.cell_off + (long long)T.nx * T.ny - 1) >> kTileBits) - lo + 1;
+    const int lo = (int)(T.tile_base >> kTileBits);
+    const int tn =
+        (int)((T.tile_base + tile_cells(T.tm, T.nx, T.ny) - 1) >> kTileBits) - lo + 1;
     if (t) {
       Terrain& o = (*t)[k];
       o.part_off = (long long)off;
@@ -370,6 +386,12 @@ int ensure_wave(shy_ctx* c) {
   if (solo != c->solo || (solo && solo_stride != c->solo_stride)) drop_graph(c);
   c->solo = solo;
   c->solo_stride = solo_stride;
+  if (!c->rootp)
+    for (const Terrain& t : c->ter)
+      if (t.has_root && !c->rootp) {
+        drop_graph(c);
+        HIPCHK(c, hipMalloc(&c->rootp, c->np * sizeof(float)));
+      }
   if (solo) {
     need = std::max(need, (size_t)drops * solo_stride);
     if (!c->scnt) {
@@ -445,23 +467,31 @@ int ensure_wave(shy_ctx* c) {
     }
   }
   {
-    // split each tile's entries over several blocks while the per-part
-    // buffers stay modest (up to 2048 tiles: 640 MiB of partial sums)
-    const bool split = c->ntiles <= kTileSplitMaxTiles;
-    if (split != c->tile_split || (split && !c->tcount)) {
+    // parts of the tiles' entries: as many as a full log would need
+    const int full =
+        (int)std::min<size_t>(kTileParts, std::max<size_t>(1, wave_steps(c) / kPartMin));
+    const int parts = std::max(full, c->parts);
+    if (parts > c->parts || c->ntiles + parts > c->list_cap) {
       drop_graph(c);
       HIPCHK(c, hipStreamSynchronize(c->stream));
-      if (c->tcount) hipFree(c->tcount);
-      if (c->tsum) hipFree(c->tsum);
+      void* old[] = {c->tparts, c->tlist, c->tmulti, c->tcount, c->tsum};
+      for (void* q : old)
+        if (q) hipFree(q);
+      c->tparts = nullptr;
+      c->tlist = nullptr;
+      c->tmulti = nullptr;
       c->tcount = nullptr;
       c->tsum = nullptr;
-      c->tile_split = false;
-      if (split) {
-        const size_t cells = (size_t)c->ntiles * kTileCells;
-        HIPCHK(c, hipMalloc(&c->tcount, cells * kCountSplit * sizeof(int32_t)));
-        HIPCHK(c, hipMalloc(&c->tsum, 4 * cells * kReduceSplit * sizeof(long long)));
-        c->tile_split = true;
-      }
+      c->parts = 0;
+      c->list_cap = 0;
+      const size_t slot_cells = 2 * (size_t)parts * kTileCells;
+      HIPCHK(c, hipMalloc(&c->tparts, sizeof(TileParts)));
+      HIPCHK(c, hipMalloc(&c->tlist, ((size_t)c->ntiles + parts) * sizeof(TilePart)));
+      HIPCHK(c, hipMalloc(&c->tmulti, (size_t)parts * sizeof(TileMulti)));
+      HIPCHK(c, hipMalloc(&c->tcount, slot_cells * sizeof(int32_t)));
+      HIPCHK(c, hipMalloc(&c->tsum, 4 * slot_cells * sizeof(long long)));
+      c->parts = parts;
+      c->list_cap = c->ntiles + parts;
     }
   }
   if (c->ntiles > c->tstart_cap) {
@@ -535,6 +565,7 @@ WaveArgs wave_args(shy_ctx* c, int p) {
   w.strk = c->strk;
   w.qb = c->qb;
   w.sr = c->sr;
+  w.rootp = c->rootp;
   w.qstride = c->qstride;
   w.log_rows = c->part_rows;
   w.dlog = c->dlog;
@@ -695,17 +726,23 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
   }
   tile_start_kernel<<<(c->ntiles + 256) / 256, 256, 0, c->stream>>>(
       c->d_ter, nter, c->ntiles, nh > 0 ? c->hist : nullptr, (long long)nh, c->tstart);
-  if (c->tile_split) {
-    tile_count_kernel<kCountSplit><<<c->ntiles * kCountSplit, 1024, 0, c->stream>>>(
-        c->tstart, pa.ecell, n, c->sr, c->first, c->visit[p], c->fld, c->root, c->d_ter, nter,
-        c->tcount);
-    tile_count_finish_kernel<kCountSplit><<<(unsigned)((n + 255) / 256), 256, 0, c->stream>>>(
-        c->tcount, n, c->sr, c->first, c->visit[p], c->fld, c->root, c->d_ter, nter);
-  } else {
-    tile_count_kernel<1><<<c->ntiles, 1024, 0, c->stream>>>(c->tstart, pa.ecell, n, c->sr,
-                                                            c->first, c->visit[p], c->fld,
-                                                            c->root, c->d_ter, nter, nullptr);
-  }
+  const size_t np = c->np;
+  TileCountOut co;
+  co.sr = c->sr;
+  co.rootp = root ? c->rootp : nullptr;
+  co.first = c->first;
+  co.visit = c->visit[p];
+  co.fld = c->fld;
+  co.root = c->root;
+  co.ter = c->d_ter;
+  co.nter = nter;
+  const int parts = c->parts;
+  tile_parts_kernel<<<1, 1024, 0, c->stream>>>(c->tstart, c->ntiles, parts, kPartMin, c->tparts,
+                                               c->tlist, c->tmulti);
+  tile_count_kernel<<<c->ntiles + parts, 1024, 0, c->stream>>>(c->tparts, c->tlist, pa.ecell, np,
+                                                               co, c->tcount);
+  tile_count_finish_kernel<<<dim3(parts, kTileCells / 1024), 1024, 0, c->stream>>>(
+      c->tparts, c->tmulti, c->tcount, np, co);
   HIPCHK(c, hipGetLastError());
   if (ev) HIPCHK(c, hipEventRecord(ev[2], c->stream));
   if (walk) {
@@ -717,17 +754,19 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
     HIPCHK(c, hipGetLastError());
   }
   if (ev) HIPCHK(c, hipEventRecord(ev[3], c->stream));
-  if (c->tile_split) {
-    tile_reduce_kernel<kReduceSplit><<<c->ntiles * kReduceSplit, 1024, 0, c->stream>>>(
-        c->tstart, pa.ecell, pa.erest, c->qb, c->qstride, c->vq, c->vq_rows, pa.drops, c->d_ter, nter,
-        c->deposit, n, c->dh, c->trk, c->trk + n, c->trk + 2 * n, c->tsum);
-    tile_reduce_finish_kernel<kReduceSplit><<<(unsigned)((n + 255) / 256), 256, 0, c->stream>>>(
-        c->tsum, c->deposit, n, c->dh, c->trk, c->trk + n, c->trk + 2 * n);
-  } else {
-    tile_reduce_kernel<1><<<c->ntiles, 1024, 0, c->stream>>>(
-        c->tstart, pa.ecell, pa.erest, c->qb, c->qstride, c->vq, c->vq_rows, pa.drops, c->d_ter, nter,
-        c->deposit, n, c->dh, c->trk, c->trk + n, c->trk + 2 * n, nullptr);
-  }
+  TileSumOut so;
+  so.deposit = c->deposit;
+  so.dh = c->dh;
+  so.td = c->trk;
+  so.tmx = c->trk + n;
+  so.tmy = c->trk + 2 * n;
+  so.ter = c->d_ter;
+  so.nter = nter;
+  tile_reduce_kernel<<<c->ntiles + parts, 1024, 0, c->stream>>>(
+      c->tparts, c->tlist, pa.ecell, pa.erest, c->qb, c->qstride, c->vq, c->vq_rows, pa.drops, np,
+      so, c->tsum);
+  tile_reduce_finish_kernel<<<dim3(parts, kTileCells / 1024), 1024, 0, c->stream>>>(
+      c->tparts, c->tmulti, c->tsum, np, so);
   HIPCHK(c, hipGetLastError());
   return launch_stencil(c, p);
 }
@@ -911,7 +950,8 @@ int shy_destroy(shy_ctx* c) {
   drop_graph(c);
   void* ptrs[] = {c->h[0], c->h[1], c->fld, c->root, c->visit[0], c->visit[1], c->first,
                   c->sr, c->dh, c->trk, c->deposit, c->slog, c->strk, c->qb, c->ent, c->gflag,
-                  c->vq, c->vt, c->scnt, c->tcount, c->tsum, c->hist, c->hbsum, c->tstart, c->dlog, c->wsteps, c->dperm, c->tsteps, c->veg_px, c->veg_py, c->veg_alive, c->veg_cflag,
+                  c->vq, c->vt, c->scnt, c->rootp, c->tparts, c->tlist, c->tmulti, c->tcount,
+                  c->tsum, c->hist, c->hbsum, c->tstart, c->dlog, c->wsteps, c->dperm, c->tsteps, c->veg_px, c->veg_py, c->veg_alive, c->veg_cflag,
                   c->veg_cx, c->veg_cy, c->veg_units, c->veg_st, c->veg_size, c->pack, c->d_ter, c->state, c->erf_a, c->part, c->perms, c->trace_buf,
                   c->trace_n, c->drop_buf};
   for (void* q : ptrs)
@@ -974,7 +1014,7 @@ int shy_ensemble_create(const shy_terrain_desc* desc, int nter, shy_ctx** out) {
   if ((e = hipMalloc(&c->fld, n * sizeof(float4))) != hipSuccess) return bail(e, "hipMalloc fld");
   if ((e = hipMalloc(&c->root, n * sizeof(float))) != hipSuccess) return bail(e, "hipMalloc root");
   if ((e = hipMalloc(&c->first, n * sizeof(int32_t))) != hipSuccess) return bail(e, "hipMalloc first");
-  if ((e = hipMalloc(&c->sr, n * sizeof(float))) != hipSuccess) return bail(e, "hipMalloc sr");
+  if ((e = hipMalloc(&c->sr, c->np * sizeof(float))) != hipSuccess) return bail(e, "hipMalloc sr");
   c->pack_recs = recs;
   if ((e = hipMalloc(&c->pack, 2 * (size_t)recs * sizeof(float4))) != hipSuccess)
     return bail(e, "hipMalloc pack");
@@ -996,7 +1036,7 @@ int shy_ensemble_create(const shy_terrain_desc* desc, int nter, shy_ctx** out) {
   hipMemsetAsync(c->fld, 0, n * sizeof(float4), c->stream);
   hipMemsetAsync(c->root, 0, n * sizeof(float), c->stream);
   hipMemsetAsync(c->first, 0, n * sizeof(int32_t), c->stream);
-  hipMemsetAsync(c->sr, 0, n * sizeof(float), c->stream);
+  hipMemsetAsync(c->sr, 0, c->np * sizeof(float), c->stream);
   hipMemsetAsync(c->dh, 0, n * sizeof(int32_t), c->stream);
   hipMemsetAsync(c->trk, 0, 3 * n * sizeof(long long), c->stream);
   hipMemsetAsync(c->deposit, 0, n * sizeof(int32_t), c->stream);

@@ -99,6 +99,8 @@ struct DeviceState {
 struct Terrain {
   long long cell_off;
   long long pack_off;  // the terrain's first packed walk record (pack_rec)
+  long long tile_base;  // its first index in tile order, and that order (tile_index)
+  TileMap tm;
   int nx, ny;
   int drop_off, drops;
   int tile_off, tiles_y;
@@ -123,8 +125,8 @@ struct Terrain {
 };
 
 // Whole-ensemble arguments of the walk kernels (concatenated arrays).
-// The partition's cell tiles: 2^kTileBits consecutive cell indices over all
-// terrains.
+// The partition's cell tiles: 2^kTileBits consecutive indices in tile order
+// (Terrain::tm) over all terrains.
 constexpr int kTileBits = 12;             // cells per tile = 4096
 constexpr int kTileCells = 1 << kTileBits;
 constexpr int kFuseMaxTiles = 4096;       // most tiles of a terrain whose walk blocks count in LDS
@@ -141,12 +143,13 @@ struct WaveArgs {
   const float4* __restrict__ fld;
   const float* __restrict__ root;
   int32_t* first;     // drops whose first step starts at the cell
-  int2* slog;         // [step][drop] {start cell over all terrains, c_eq bits}
+  int2* slog;         // [step][drop] {start cell in tile order over all terrains, c_eq bits}
   int2* strk;         // [step][drop] {qt(vol sx), qt(vol sy)}: the step's momentum tracks
   int32_t* qb;        // [drop][step] height commit of the step, 2^-20 (replay)
   int log_rows;       // rows of slog
   int qstride;        // qb's stride per drop: log rows rounded up to kReplayDepth, then to 32
-  const float* __restrict__ sr;   // burst scale per cell (tile_count_kernel)
+  const float* __restrict__ sr;   // burst scale per cell (tile_count_kernel), in tile order
+  const float* __restrict__ rootp;  // root density in tile order, where a terrain has one
   // waves of one drop (walk_solo_kernel): [drop][solo_stride] {start cell, c_eq
   // bits}, the per-cell step counts and the accumulators of the commits
   int2* solo;
@@ -182,6 +185,29 @@ __device__ inline int find_terrain(int nter, long long v, Key key) {
   return lo;
 }
 
+// A read-only table read at an index that is uniform over the wave (scalar
+// loads: the compiler cannot tell by itself that no store of the kernel
+// writes the table).
+typedef const __attribute__((address_space(4))) float ConstF32;
+__device__ inline float2 ld_uniform2(const float2* p, int k) {
+  ConstF32* q = (ConstF32*)(uintptr_t)(p + k);
+  return make_float2(q[0], q[1]);
+}
+// A wave's terrain entry, t uniform: into scalar registers, also where the
+// kernel has stored to memory before.
+__device__ inline Terrain ld_terrain(const Terrain* ter, int t) {
+  typedef const __attribute__((address_space(4))) int ConstI32;
+  static_assert(sizeof(Terrain) % 4 == 0, "copied by words");
+  ConstI32* q = (ConstI32*)(uintptr_t)(ter + t);
+  union {
+    Terrain T;
+    int w[sizeof(Terrain) / 4];
+  } u;
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(Terrain) / 4); ++i) u.w[i] = q[i];
+  return u.T;
+}
+
 // One terrain's view, as one drop walks it (pointers offset to the terrain).
 struct WalkArgs {
   const float* __restrict__ h;
@@ -189,7 +215,8 @@ struct WalkArgs {
   const float* __restrict__ root;  // nullptr when the map has no root density
   int2* slog;                      // [step][drop] step log (count pass): {cell, c_eq}
   int2* strk;                      // [step][drop] its tracks
-  int cell_off;                    // the terrain's first cell over all terrains
+  int tile_base;                   // the terrain's first cell in tile order, and that order
+  TileMap tm;
   const float4* __restrict__ pack; // packed cells, or nullptr (read h, fld, root)
   uint8_t* visit;                  // cascade sites
   DeviceState* state;
@@ -385,7 +412,7 @@ __device__ int walk_drop(const WalkArgs& a, int lane_drop, float x0, float y0, i
   // real log overwrites one step later or, for a drop that takes no step,
   // which no reader looks at (its step count is 0)
   size_t pk = (size_t)lane_drop;
-  int2 ps = make_int2(a.cell_off + i0, 0), pt = make_int2(0, 0);
+  int2 ps = make_int2(a.tile_base + (COUNT ? tile_index(a.tm, ix, iy) : 0), 0), pt = make_int2(0, 0);
   // the count walk reads the cycle's packed records, the trace the map arrays
   auto load_cell = [&](int x, int y, int i) {
     if constexpr (COUNT) return load_packed(a.pack, pack_rec(x, y, a.ny));
@@ -474,9 +501,9 @@ __device__ int walk_drop(const WalkArgs& a, int lane_drop, float x0, float y0, i
       // everything of the step that the snapshot fixes; the tracks
       // (water.h:115-117) use the volume before this step's evaporation
       pk = klog;
-      ps = make_int2(a.cell_off + i0, __float_as_int(c_eq));
+      ps = make_int2(a.tile_base + tile_index(a.tm, ix, iy), __float_as_int(c_eq));
       pt = make_int2(quant_t(vol * sx), quant_t(vol * sy));
-      step_hook(a.cell_off + i0);
+      step_hook(ps.x);
     }
     if (TRACE) {
       const float ero = effD * (c_eq - sed);  // water.h:128-132
@@ -518,15 +545,6 @@ __device__ int walk_drop(const WalkArgs& a, int lane_drop, float x0, float y0, i
   return steps;
 }
 
-// A read-only table read at an index that is uniform over the wave (scalar
-// loads: the compiler cannot tell by itself that no store of the kernel
-// writes the table).
-typedef const __attribute__((address_space(4))) float ConstF32;
-__device__ inline float2 ld_uniform2(const float2* p, int k) {
-  ConstF32* q = (ConstF32*)(uintptr_t)(p + k);
-  return make_float2(q[0], q[1]);
-}
-
 // The count walk of a terrain whose volumes, transfer and cells all lie in the
 // range of the short arithmetic (Terrain::vol_ok, gflag): the same values as
 // walk_drop<kCount>, which any other terrain takes, with
@@ -552,16 +570,22 @@ __device__ int walk_short(const WalkArgs& a, const float2* __restrict__ vt, int 
   const float fnx = (float)nx, fny = (float)ny;
   const float mt = kLod * a.P.momentumTransfer, entr = a.P.entrainment;
   const char* packb = reinterpret_cast<const char*>(a.pack);
-  const uint32_t lane_off = (uint32_t)lane_drop * 8u;
+  const size_t lane_off = (size_t)lane_drop * 8u;
   const size_t row_bytes = (size_t)a.drops * 8u;
   auto rec_off = [&](int x, int y) {
     const uint32_t b = __umul24((uint32_t)x >> 1, (uint32_t)(ny + 1) >> 1) + ((uint32_t)y >> 1);
     return (b << 7) | (((uint32_t)x & 1u) << 6) | (((uint32_t)y & 1u) << 5);
   };
-  auto cell_of = [&](int x, int y) { return (int)(__umul24((uint32_t)x, (uint32_t)ny) + (uint32_t)y); };
+  // tile_index over all terrains
+  const int ma = a.tm.a, mb = a.tm.b, mab = ma + mb;
+  auto cell_of = [&](int x, int y) {
+    const uint32_t blk = __umul24((uint32_t)x >> ma, (uint32_t)a.tm.nyb) + ((uint32_t)y >> mb);
+    return a.tile_base + (int)((blk << mab) | ((x & a.tm.mxh) << mb | (y & a.tm.myh) << 2 |
+                                               (x & a.tm.mxl) << 3 | (y & a.tm.myl)));
+  };
   float px = x0, py = y0, sx = 0.0f, sy = 0.0f;
-  uint32_t ro = rec_off((int)x0, (int)y0);
-  int i0 = cell_of((int)x0, (int)y0);
+  int ix = (int)x0, iy = (int)y0;
+  uint32_t ro = rec_off(ix, iy);
   // {h, gravity x, gravity z, erf(0.4 d)}, {mx, my, d, 1/|(mx, my)|}
   float4 ca = *reinterpret_cast<const float4*>(packb + ro);
   float4 cb = *reinterpret_cast<const float4*>(packb + ro + 16);
@@ -569,19 +593,15 @@ __device__ int walk_short(const WalkArgs& a, const float2* __restrict__ vt, int 
   float pf = 0.0f;
   // stored one step late, as in walk_drop; the first store is a placeholder in
   // the drop's own slot of row 0
-  int2 ps = make_int2(a.cell_off + i0, 0), pt = make_int2(0, 0);
+  int2 ps = make_int2(cell_of(ix, iy), 0), pt = make_int2(0, 0);
   char* srow = reinterpret_cast<char*>(a.slog);
   char* trow = reinterpret_cast<char*>(a.strk);
   float2 v = ld_uniform2(vt, 0);
-  int steps = 0;
+  int steps = 0, left = end_kind;
   // wait for the first record before the loop (see walk_drop)
   __builtin_amdgcn_s_waitcnt(0);
   for (int k = 0;; ++k) {
-    if (k >= max_steps) {  // water.h:74-82
-      *end = end_kind;
-      *end_cell = i0;
-      break;
-    }
+    if (k >= max_steps) break;  // water.h:74-82
     const float2 vn = ld_uniform2(vt, k + 1);
     steps = k + 1;
     // water.h:95-111
@@ -602,7 +622,6 @@ __device__ int walk_short(const WalkArgs& a, const float2* __restrict__ vt, int 
     }
     const int jx = cvt_i32(px), jy = cvt_i32(py);
     const bool ex = !((int)(px > -1.0f) & (int)(px < fnx) & (int)(py > -1.0f) & (int)(py < fny));
-    const int j = cell_of(jx, jy);
     // off the map the record is not used; loading the current cell's keeps
     // the load unconditional, so its wait is counted exactly
     ro = ex ? ro : rec_off(jx, jy);
@@ -626,23 +645,26 @@ __device__ int walk_short(const WalkArgs& a, const float2* __restrict__ vt, int 
     }
     const float v24 = v.x * kTQ;  // the tracks, water.h:115-117
     pt = make_int2(cvt_i32(__builtin_rintf(v24 * sx)), cvt_i32(__builtin_rintf(v24 * sy)));
-    step_hook(a.cell_off + i0);
+    const int cell = cell_of(ix, iy);
+    step_hook(cell);
     float h2 = na.x;
     if (__builtin_expect(ex, 0)) h2 = (float)((double)ca.x - 0.002);  // water.h:120-124
     float c_eq = (1.0f + entr * ca.w) * (ca.x - h2);  // water.h:127
     if (c_eq < 0) c_eq = 0;
-    ps = make_int2(a.cell_off + i0, __float_as_int(c_eq));
+    ps = make_int2(cell, __float_as_int(c_eq));
     if constexpr (PREFETCH) pf_acc ^= __float_as_uint(pf_last);
     if (ex) {  // water.h:139-142
-      *end = kEndExit;
-      *end_cell = i0;
+      left = kEndExit;
       break;
     }
     v = vn;
     ca = na;
     cb = nb;
-    i0 = j;
+    ix = jx;
+    iy = jy;
   }
+  *end = left;
+  *end_cell = ix * ny + iy;
   // the last step's log, in its own row
   const size_t last = (size_t)(steps > 0 ? steps - 1 : 0) * row_bytes;
   st_stream(reinterpret_cast<int2*>(reinterpret_cast<char*>(a.slog) + last + lane_off), ps);
@@ -741,48 +763,51 @@ __global__ void __launch_bounds__(1024) walk_kernel(WaveArgs w) {
     const int g0 = __builtin_amdgcn_readfirstlane(g);
     const int t = __builtin_amdgcn_readfirstlane(
         find_terrain(w.nter, g0, [&](int k) { return (long long)w.ter[k].drop_off; }));
-    const Terrain T = w.ter[t];
+    const Terrain T = ld_terrain(w.ter, t);
     int4 dl = make_int4(0, kEndPad, 0, 0);
     const int loc = w.perm ? w.perm[g] : g - T.drop_off;  // the drop this thread walks
+    WalkArgs a{};
+    a.h = w.h + T.cell_off;
+    a.fld = w.fld + T.cell_off;
+    a.root = T.has_root ? w.root + T.cell_off : nullptr;
+    a.tile_base = (int)T.tile_base;
+    a.tm = T.tm;
+    a.slog = w.slog;
+    a.strk = w.strk;
+    a.pack = w.pack ? w.pack + 2 * T.pack_off : nullptr;
+    a.nx = T.nx;
+    a.ny = T.ny;
+    a.drops = w.total_drops;  // log stride
+    a.P = T.P;
+    uint32_t cid = 0;
+    bool walks = false;
     if (loc < T.drops) {  // not a padding lane
-      WalkArgs a{};
-      a.h = w.h + T.cell_off;
-      a.fld = w.fld + T.cell_off;
-      a.root = T.has_root ? w.root + T.cell_off : nullptr;
-      a.cell_off = (int)T.cell_off;
-      a.slog = w.slog;
-      a.strk = w.strk;
-      a.pack = w.pack ? w.pack + 2 * T.pack_off : nullptr;
-      a.nx = T.nx;
-      a.ny = T.ny;
-      a.drops = w.total_drops;  // log stride
-      a.P = T.P;
       const uint32_t ncell = (uint32_t)T.nx * (uint32_t)T.ny;
-      const uint32_t cid =
-          spawn_cell(cycle_key(T.seed, T.id, cycle), (uint32_t)loc, ncell);
+      cid = spawn_cell(cycle_key(T.seed, T.id, cycle), (uint32_t)loc, ncell);
+      walks = (double)a.h[cid] >= 0.1;  // world.h:71-72
       dl.y = kEndSkipped;
-      if ((double)a.h[cid] >= 0.1) {  // world.h:71-72
-        int end = 0, end_cell = 0;
-        uint32_t sink = 0;
-        const float x0 = (float)(cid / (uint32_t)T.ny), y0 = (float)(cid % (uint32_t)T.ny);
-        // uniform over the wave (one terrain per wave)
-        if (T.vol_ok && !w.gflag[t])
-          dl.x = walk_short<decltype(count_step), PREFETCH>(
-              a, w.vt + (size_t)t * w.vt_rows, T.max_steps, T.end_kind, g, x0, y0, &end,
-              &end_cell, count_step, &sink);
-        else
-          dl.x = walk_drop<kCount, decltype(count_step), PREFETCH>(
-              a, g, x0, y0, &end, &end_cell, nullptr, 0, nullptr, count_step, &sink);
-        dl.w = (int)sink;  // not read: it keeps the record prefetches
-        dl.y = end;
-        dl.z = end_cell;
-        if (dl.x > 0) {
-          // arrivals = steps past the first; a walk that ended after a step
-          // ended on its last arrival (water.h:151)
-          __hip_atomic_fetch_add(&w.first[T.cell_off + cid], 1, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-          if (end != kEndExit) w.visit[T.cell_off + end_cell] = 1;
-        }
+    }
+    if (walks) {
+      int end = 0, end_cell = 0;
+      uint32_t sink = 0;
+      const float x0 = (float)(cid / (uint32_t)T.ny), y0 = (float)(cid % (uint32_t)T.ny);
+      // uniform over the wave (one terrain per wave)
+      if (T.vol_ok && !w.gflag[t])
+        dl.x = walk_short<decltype(count_step), PREFETCH>(
+            a, w.vt + (size_t)t * w.vt_rows, T.max_steps, T.end_kind, g, x0, y0, &end, &end_cell,
+            count_step, &sink);
+      else
+        dl.x = walk_drop<kCount, decltype(count_step), PREFETCH>(
+            a, g, x0, y0, &end, &end_cell, nullptr, 0, nullptr, count_step, &sink);
+      dl.w = (int)sink;  // not read: it keeps the record prefetches
+      dl.y = end;
+      dl.z = end_cell;
+      if (dl.x > 0) {
+        // arrivals = steps past the first; a walk that ended after a step
+        // ended on its last arrival (water.h:151)
+        __hip_atomic_fetch_add(&w.first[T.cell_off + cid], 1, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        if (end != kEndExit) w.visit[T.cell_off + end_cell] = 1;
       }
     }
     w.dlog[g] = dl;
@@ -1033,7 +1058,7 @@ __global__ void __launch_bounds__(2 * kSoloWaves * 64) walk_solo_kernel(WaveArgs
   const int lane = threadIdx.x & 63;
   const int t = __builtin_amdgcn_readfirstlane(
       find_terrain(w.nter, g, [&](int k) { return (long long)w.ter[k].drop_off; }));
-  const Terrain T = w.ter[t];
+  const Terrain T = ld_terrain(w.ter, t);
   const int loc = g - T.drop_off;
   const uint32_t ncell = (uint32_t)T.nx * (uint32_t)T.ny;
   const uint32_t cid = __builtin_amdgcn_readfirstlane(
@@ -1080,7 +1105,7 @@ __device__ inline int quant_h_sat(float v) {
 // L2), and one row per step did so at every step.  One wave per SIMD is all a
 // 65536-drop wave fills, so these loads are the latency hiding.
 // Measured against a row loaded and a gather issued per step, 32 ahead:
-// 65536 drops on 1024^2 248 -> 233 us.
+// 65536 drops on 1024^2 248 -> 233 us (196 with the map in tile order).
 constexpr int kReplayBatch = 16;
 // steps of a turn of three batches: qb's stride per drop is a multiple (and of
 // 32, so that a drop's runs of 32 commits are whole 128-byte lines)
@@ -1099,14 +1124,14 @@ __global__ void __launch_bounds__(256) replay_kernel(WaveArgs w) {
     const int g0 = __builtin_amdgcn_readfirstlane(g);
     const int t = __builtin_amdgcn_readfirstlane(
         find_terrain(w.nter, g0, [&](int k) { return (long long)w.ter[k].drop_off; }));
-    const Terrain T = w.ter[t];
+    const Terrain T = ld_terrain(w.ter, t);
     const int4 dl = w.dlog[g];
     const int n = dl.y <= kEndExit ? dl.x : 0;
     if (dl.y == kEndSkipped) skipped += 1;
     if (dl.y <= kEndExit) {
       walked += 1;
       const float* __restrict__ sr = w.sr;
-      const float* __restrict__ rmap = w.root;
+      const float* __restrict__ rmap = w.rootp;
       const float dep = T.P.depositionRate, e = T.P.evapRate;
       const double ce = 1.0 - (double)e, ye = 1.0 / ce;  // evaporation divisor, its reciprocal
       float sed = 0.0f;
@@ -1436,7 +1461,7 @@ __global__ void tile_start_kernel(const Terrain* __restrict__ ter, int nter, int
     return;
   }
   const int q = find_terrain(nter, (long long)t << kTileBits,
-                             [&](int k) { return ter[k].cell_off; });
+                             [&](int k) { return ter[k].tile_base; });
   const Terrain& T = ter[q];
   start[t] = hist[T.part_off + (long long)(t - T.tile_lo) * T.part_blocks];
 }
@@ -1681,59 +1706,168 @@ __global__ void __launch_bounds__(1024, RS <= 4096 ? 8 : 4) part_scatter_staged_
 }
 
 
-// Per tile: the walk steps starting at each cell (LDS histogram of the
-// tile's entries) -> burst scale, the replay's 4-byte gather per step;
-// cascade sites where more steps
-// start than first steps (an arrival, water.h:151); clears the first-step
-// counts.  With S > 1 each tile's entries are split over S blocks (block
-// t*S + s takes the s-th part), which write their counts to part[block] and
-// tile_count_finish_kernel adds them: the largest tiles hold several times
-// the mean's entries, and one block per tile would wait for them.
+// The tile kernels' work: each tile's entries in parts of at most C = max(part_min,
+// all / parts) entries, one block per part.  The entries follow the rivers, so
+// a few square tiles hold many times the mean, and the kernels' time was the
+// largest tile's (1024^2: sums 313 us for 111 us of work over 256 CUs).  A
+// tile of one part is finished by its block; the parts of a larger one go to
+// slots that a finishing kernel adds (integers, so any order gives the same).
+// At most ntiles + parts parts, parts tiles of more than one, 2 parts slots.
+struct TileParts {
+  int n;      // parts
+  int multi;  // tiles of more than one
+};
+struct TilePart {
+  int tile, e0, e1, slot;  // slot -1: the tile's only part
+};
+struct TileMulti {
+  int tile, slot, parts, unused;
+};
 
-// entry range of part s of tile t
-template <int S>
-__device__ inline void tile_part(const int32_t* __restrict__ start, int t, int s, int& a, int& b) {
-  const int e0 = start[t], e1 = start[t + 1];
-  if (S == 1) {
-    a = e0;
-    b = e1;
-  } else {
-    const long long len = e1 - e0;
-    a = e0 + (int)(len * s / S);
-    b = e0 + (int)(len * (s + 1) / S);
+// Blocks are dealt to the 8 XCDs by their number, so a map's columns of tiles
+// would each stay on one XCD: the list goes by falling size (kPartClasses
+// steps of C), which spreads the tiles and leaves the small ones for the end.
+constexpr int kPartClasses = 32;
+
+__global__ void __launch_bounds__(1024) tile_parts_kernel(const int32_t* __restrict__ start,
+                                                          int ntiles, int parts, int part_min,
+                                                          TileParts* np, TilePart* list,
+                                                          TileMulti* multi) {
+  __shared__ unsigned long long wsum[16];
+  __shared__ unsigned long long base;
+  __shared__ int cls[kPartClasses];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const long long all = start[ntiles];
+  const long long even = (all + parts - 1) / parts;
+  const int C = even > part_min ? (int)even : part_min;
+  // class 0: the largest parts; a part holds at most C
+  auto part_class = [&](int len, int p) {
+    const int c = (int)((float)(len / p) / (float)C * kPartClasses);
+    return c >= kPartClasses ? 0 : kPartClasses - 1 - c;
+  };
+  if (tid == 0) base = 0;
+  if (tid < kPartClasses) cls[tid] = 0;
+  __syncthreads();
+  for (int t = tid; t < ntiles; t += 1024) {
+    const int len = start[t + 1] - start[t];
+    const int p = len > C ? (len + C - 1) / C : 1;
+    atomicAdd(&cls[part_class(len, p)], p);
   }
+  __syncthreads();
+  if (tid < 64) {
+    const int c = lane < kPartClasses ? cls[lane] : 0;
+    int x = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane < kPartClasses) cls[lane] = x - c;
+    if (lane == 63) np->n = x;
+  }
+  __syncthreads();
+  for (int t0 = 0; t0 < ntiles; t0 += 1024) {
+    const int t = t0 + tid;
+    int e0 = 0, len = 0, p = 0;
+    if (t < ntiles) {
+      e0 = start[t];
+      len = start[t + 1] - e0;
+      p = len > C ? (len + C - 1) / C : 1;
+    }
+    // two counters in one scan: slots and tiles of several parts
+    const unsigned long long v = p > 1 ? (unsigned long long)p | 1ULL << 32 : 0ULL;
+    unsigned long long x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const unsigned long long y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[wv] = x;
+    __syncthreads();
+    unsigned long long before = base, total = 0;
+    for (int i = 0; i < 16; ++i) {
+      if (i < wv) before += wsum[i];
+      total += wsum[i];
+    }
+    before += x - v;
+    if (p > 0) {
+      const int at = atomicAdd(&cls[part_class(len, p)], p);
+      const int slot = (int)(before & 0xffffffffu);
+      if (p > 1) multi[before >> 32] = TileMulti{t, slot, p, 0};
+      for (int s = 0; s < p; ++s)
+        list[at + s] = TilePart{t, e0 + (int)((long long)len * s / p),
+                                e0 + (int)((long long)len * (s + 1) / p), p > 1 ? slot + s : -1};
+    }
+    __syncthreads();
+    if (tid == 0) base += total;
+    __syncthreads();
+  }
+  if (tid == 0) np->multi = (int)(base >> 32);
 }
 
-// burst scale and cascade site of cell i, k steps starting there
-__device__ inline void cell_count_finish(size_t i, int k, float* sr, int32_t* first,
-                                         uint8_t* visit, const float4* __restrict__ fld,
-                                         const float* __restrict__ root,
-                                         const Terrain* __restrict__ ter, int nter) {
-  const int t = find_terrain(nter, (long long)i, [&](int q) { return ter[q].cell_off; });
-  const shy_params& P = ter[t].P;
-  const float rd = ter[t].has_root ? root[i] : 0.0f;
+// Per tile: the walk steps starting at each cell (LDS histogram of the tile's
+// entries) -> burst scale, the replay's 4-byte gather per step; cascade sites
+// where more steps start than first steps (an arrival, water.h:151); clears
+// the first-step counts.
+// burst scale (into *sr) and cascade site of cell i of terrain T, k steps
+// starting there; returns its root density
+__device__ inline float cell_count_finish(size_t i, int k, float* sr, int32_t* first,
+                                          uint8_t* visit, const float4* __restrict__ fld,
+                                          const float* __restrict__ root, const Terrain& T) {
+  const shy_params& P = T.P;
+  const float rd = T.has_root ? root[i] : 0.0f;
   float effD = P.depositionRate * (1.0f - rd);
   if (effD < 0) effD = 0;
-  sr[i] = burst_scale(k, effD, P.entrainment, fld[i].w);
+  *sr = burst_scale(k, effD, P.entrainment, fld[i].w);
   const int f = first[i];
   if (k > f) visit[i] = 1;
   if (f) first[i] = 0;
+  return rd;
 }
 
-template <int S>
-__global__ void __launch_bounds__(1024) tile_count_kernel(
-    const int32_t* __restrict__ start, const int32_t* __restrict__ ecell, size_t n,
-    float* sr, int32_t* first, uint8_t* visit, const float4* __restrict__ fld,
-    const float* __restrict__ root, const Terrain* __restrict__ ter, int nter, int32_t* part) {
+// The terrain and x-major cell index of index i in tile order; false for an
+// index that no cell has.
+__device__ inline bool tile_cell(const Terrain* __restrict__ ter, int nter, size_t i,
+                                 const Terrain*& T, size_t& lin) {
+  T = ter + find_terrain(nter, (long long)i, [&](int q) { return ter[q].tile_base; });
+  int x, y;
+  tile_xy(T->tm, (int)((long long)i - T->tile_base), x, y);
+  lin = (size_t)T->cell_off + (size_t)x * T->ny + y;
+  return x < T->nx && y < T->ny;
+}
+
+struct TileCountOut {
+  float* sr;
+  float* rootp;  // or null
+  int32_t* first;
+  uint8_t* visit;
+  const float4* __restrict__ fld;
+  const float* __restrict__ root;
+  const Terrain* __restrict__ ter;
+  int nter;
+};
+
+__device__ inline void tile_count_cell(const TileCountOut& o, size_t i, int k) {
+  const Terrain* T;
+  size_t lin;
+  if (!tile_cell(o.ter, o.nter, i, T, lin)) return;
+  const float rd = cell_count_finish(lin, k, o.sr + i, o.first, o.visit, o.fld, o.root, *T);
+  if (o.rootp) o.rootp[i] = rd;
+}
+
+__global__ void __launch_bounds__(1024) tile_count_kernel(const TileParts* __restrict__ np,
+                                                          const TilePart* __restrict__ list,
+                                                          const int32_t* __restrict__ ecell,
+                                                          size_t n, TileCountOut o,
+                                                          int32_t* slots) {
   __shared__ int cnt[kTileCells];
+  if ((int)blockIdx.x >= np->n) return;
+  const TilePart P = list[blockIdx.x];
   for (int j = threadIdx.x; j < kTileCells; j += blockDim.x) cnt[j] = 0;
   __syncthreads();
-  const int t = blockIdx.x / S, s = blockIdx.x % S;
-  const int base = t << kTileBits;
-  int e0, e1;
-  tile_part<S>(start, t, s, e0, e1);
+  const int base = P.tile << kTileBits, e1 = P.e1;
   // four entries per thread in flight
-  for (int e = e0 + (int)threadIdx.x; e < e1; e += 4 * blockDim.x) {
+  for (int e = P.e0 + (int)threadIdx.x; e < e1; e += 4 * blockDim.x) {
     int c[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -1746,30 +1880,29 @@ __global__ void __launch_bounds__(1024) tile_count_kernel(
   }
   __syncthreads();
   for (int j = threadIdx.x; j < kTileCells; j += blockDim.x) {
-    if (S > 1) {
-      part[(size_t)blockIdx.x * kTileCells + j] = cnt[j];
+    if (P.slot >= 0) {
+      slots[(size_t)P.slot * kTileCells + j] = cnt[j];
     } else {
       const size_t i = (size_t)base + j;
       if (i >= n) break;
-      cell_count_finish(i, cnt[j], sr, first, visit, fld, root, ter, nter);
+      tile_count_cell(o, i, cnt[j]);
     }
   }
 }
 
-// the S parts' counts of every cell (fixed order), then as tile_count_kernel
-template <int S>
-__global__ void tile_count_finish_kernel(const int32_t* __restrict__ part, size_t n, float* sr,
-                                         int32_t* first, uint8_t* visit,
-                                         const float4* __restrict__ fld,
-                                         const float* __restrict__ root,
-                                         const Terrain* __restrict__ ter, int nter) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+// the parts' counts of every cell of a tile of several, then as
+// tile_count_kernel; block (m, c): cells 1024 c .. of the m-th such tile
+__global__ void __launch_bounds__(1024) tile_count_finish_kernel(
+    const TileParts* __restrict__ np, const TileMulti* __restrict__ multi,
+    const int32_t* __restrict__ slots, size_t n, TileCountOut o) {
+  if ((int)blockIdx.x >= np->multi) return;
+  const TileMulti M = multi[blockIdx.x];
+  const int j = blockIdx.y * 1024 + threadIdx.x;
+  const size_t i = ((size_t)M.tile << kTileBits) + j;
   if (i >= n) return;
-  const size_t t = i >> kTileBits, j = i & (kTileCells - 1);
   int k = 0;
-#pragma unroll
-  for (int s = 0; s < S; ++s) k += part[(t * S + s) * kTileCells + j];
-  cell_count_finish(i, k, sr, first, visit, fld, root, ter, nter);
+  for (int s = 0; s < M.parts; ++s) k += slots[(size_t)(M.slot + s) * kTileCells + j];
+  tile_count_cell(o, i, k);
 }
 
 // Between walk and replay of a cycle of few drops, one thread per cell: the
@@ -1784,7 +1917,8 @@ __global__ void solo_cells_kernel(size_t n, int32_t* scnt, float* sr, int32_t* f
   const int k = scnt[i];
   if (k == 0) return;  // no step starts here: no replay reads its scale, and first is 0
   scnt[i] = 0;
-  cell_count_finish(i, k, sr, first, visit, fld, root, ter, nter);
+  const int t = find_terrain(nter, (long long)i, [&](int q) { return ter[q].cell_off; });
+  cell_count_finish(i, k, sr + i, first, visit, fld, root, ter[t]);
 }
 
 // value of the lane below (lane 0: old)
@@ -1824,7 +1958,7 @@ __global__ void __launch_bounds__(256) replay_solo_kernel(WaveArgs w) {
   if (threadIdx.x == 0) bsteps = 0;
   __syncthreads();
   if (g < w.total_drops) {
-    const Terrain T = w.ter[t];
+    const Terrain T = ld_terrain(w.ter, t);
     const int4 dl = w.dlog[g];
     const int n = __builtin_amdgcn_readfirstlane(dl.y <= kEndExit ? dl.x : 0);
     if (dl.y == kEndSkipped && lane == 0) skipped = 1;
@@ -1943,16 +2077,34 @@ __global__ void volq_kernel(const Terrain* __restrict__ ter, int nter, int rows,
 // output) and the tracks of every step starting at each cell, summed in
 // LDS in integers (so the result does not depend on the order drops ran),
 // plus the terminal deposits; clears the deposits.  The volume track of a
-// step is vq[terrain][step row].  With S > 1 the tile's entries are split as
-// in tile_count_kernel and tile_reduce_finish_kernel adds the parts.
-template <int S>
+// step is vq[terrain][step row].  Parts as in tile_count_kernel.
+struct TileSumOut {
+  int32_t* deposit;
+  int32_t* dh;
+  long long *td, *tmx, *tmy;
+  const Terrain* __restrict__ ter;
+  int nter;
+};
+
+__device__ inline void tile_sum_cell(const TileSumOut& o, size_t i, const long long (&a)[4]) {
+  const Terrain* T;
+  size_t c;
+  if (!tile_cell(o.ter, o.nter, i, T, c)) return;
+  o.dh[c] = (int32_t)(a[0] + o.deposit[c]);
+  o.td[c] = a[1];
+  o.tmx[c] = a[2];
+  o.tmy[c] = a[3];
+  o.deposit[c] = 0;
+}
+
 __global__ void __launch_bounds__(1024) tile_reduce_kernel(
-    const int32_t* __restrict__ start, const int32_t* __restrict__ ecell,
-    const EntRest* __restrict__ erest,
+    const TileParts* __restrict__ np, const TilePart* __restrict__ list,
+    const int32_t* __restrict__ ecell, const EntRest* __restrict__ erest,
     const int32_t* __restrict__ qb, int qstride, const int32_t* __restrict__ vq, int rows,
-    int drops, const Terrain* __restrict__ ter, int nter, int32_t* deposit, size_t n,
-    int32_t* dh, long long* td, long long* tmx, long long* tmy, long long* part) {
+    int drops, size_t n, TileSumOut o, long long* slots) {
   __shared__ unsigned long long acc[4][kTileCells];
+  if ((int)blockIdx.x >= np->n) return;
+  const TilePart P = list[blockIdx.x];
   for (int j = threadIdx.x; j < kTileCells; j += blockDim.x) {
     acc[0][j] = 0;
     acc[1][j] = 0;
@@ -1960,18 +2112,17 @@ __global__ void __launch_bounds__(1024) tile_reduce_kernel(
     acc[3][j] = 0;
   }
   __syncthreads();
-  const int tile = blockIdx.x / S, s = blockIdx.x % S;
-  const int base = tile << kTileBits;
+  const int base = P.tile << kTileBits, e1 = P.e1;
   // terrains of the tile's first and last cell: one terrain in nearly every tile
-  auto key = [&](int q) { return ter[q].cell_off; };
+  const Terrain* __restrict__ ter = o.ter;
+  const int nter = o.nter;
+  auto key = [&](int q) { return ter[q].tile_base; };
   const int t_lo = find_terrain(nter, (long long)base, key);
   const long long last = (long long)base + kTileCells - 1 < (long long)n ? base + kTileCells - 1
                                                                           : (long long)n - 1;
   const int t_hi = find_terrain(nter, last, key);
-  int e0, e1;
-  tile_part<S>(start, tile, s, e0, e1);
   // four entries per thread in flight: the entry loads, then their gathers
-  for (int e = e0 + (int)threadIdx.x; e < e1; e += 4 * blockDim.x) {
+  for (int e = P.e0 + (int)threadIdx.x; e < e1; e += 4 * blockDim.x) {
     int4 p[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -2008,43 +2159,38 @@ __global__ void __launch_bounds__(1024) tile_reduce_kernel(
   }
   __syncthreads();
   for (int j = threadIdx.x; j < kTileCells; j += blockDim.x) {
-    if (S > 1) {
-      long long* o = part + (size_t)blockIdx.x * 4 * kTileCells + j;
+    if (P.slot >= 0) {
+      long long* s = slots + (size_t)P.slot * 4 * kTileCells + j;
 #pragma unroll
-      for (int f = 0; f < 4; ++f) o[(size_t)f * kTileCells] = (long long)acc[f][j];
+      for (int f = 0; f < 4; ++f) s[(size_t)f * kTileCells] = (long long)acc[f][j];
     } else {
       const size_t i = (size_t)base + j;
       if (i >= n) break;
-      dh[i] = (int32_t)((long long)acc[0][j] + deposit[i]);
-      td[i] = (long long)acc[1][j];
-      tmx[i] = (long long)acc[2][j];
-      tmy[i] = (long long)acc[3][j];
-      deposit[i] = 0;
+      const long long a[4] = {(long long)acc[0][j], (long long)acc[1][j], (long long)acc[2][j],
+                              (long long)acc[3][j]};
+      tile_sum_cell(o, i, a);
     }
   }
 }
 
-// the S parts' sums of every cell (fixed order), then as tile_reduce_kernel
-template <int S>
-__global__ void tile_reduce_finish_kernel(const long long* __restrict__ part, int32_t* deposit,
-                                          size_t n, int32_t* dh, long long* td, long long* tmx,
-                                          long long* tmy) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+// the parts' sums of every cell of a tile of several, then as
+// tile_reduce_kernel; blocks as in tile_count_finish_kernel
+__global__ void __launch_bounds__(1024) tile_reduce_finish_kernel(
+    const TileParts* __restrict__ np, const TileMulti* __restrict__ multi,
+    const long long* __restrict__ slots, size_t n, TileSumOut o) {
+  if ((int)blockIdx.x >= np->multi) return;
+  const TileMulti M = multi[blockIdx.x];
+  const int j = blockIdx.y * 1024 + threadIdx.x;
+  const size_t i = ((size_t)M.tile << kTileBits) + j;
   if (i >= n) return;
-  const size_t t = i >> kTileBits, j = i & (kTileCells - 1);
   long long a[4] = {0, 0, 0, 0};
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const long long* o = part + (t * S + s) * 4 * kTileCells + j;
+  for (int s = 0; s < M.parts; ++s) {
+    const long long* p = slots + (size_t)(M.slot + s) * 4 * kTileCells + j;
 #pragma unroll
     for (int f = 0; f < 4; ++f)
-      a[f] = (long long)((unsigned long long)a[f] + (unsigned long long)o[(size_t)f * kTileCells]);
+      a[f] = (long long)((unsigned long long)a[f] + (unsigned long long)p[(size_t)f * kTileCells]);
   }
-  dh[i] = (int32_t)(a[0] + deposit[i]);
-  td[i] = a[1];
-  tmx[i] = a[2];
-  tmy[i] = a[3];
-  deposit[i] = 0;
+  tile_sum_cell(o, i, a);
 }
 
 __global__ void trace_kernel(WalkArgs a, float x0, float y0, shy_drop_step* out, int max_steps,

@@ -156,3 +156,18 @@ def test_few_drops_ensemble(shy, orc):
             assert np.array_equal(bits(e.field(i, name)), bits(ref)), (i, name)
         assert e.terrain_steps()[i] == steps, i
     e.close()
+
+
+@pytest.mark.parametrize("nx,ny,drops,kw", [
+    (64, 64, 5000, dict()),                   # every step in one tile: all parts are its
+    (70, 64, 4200, dict(maxAge=3.0)),         # two tiles, fewer entries than one part's least
+    (200, 136, 5000, dict(maxAge=120.0)),     # tiles of one part beside tiles of several
+    (4400, 1000, 4500, dict(maxAge=30.0)),    # more tiles than the block listing them has threads
+])
+def test_tile_parts(shy, orc, nx, ny, drops, kw):
+    """The tile kernels' work is cut by entries: tiles of one part, of
+    several, and the sums of a tile's parts."""
+    x, y = np.meshgrid(np.arange(nx), np.arange(ny), indexing="ij")
+    # valleys, so that some tiles hold most of the steps
+    h = (0.5 + 2e-4 * (np.abs(x % 97 - 48) + np.abs(y % 89 - 44))).astype(np.float32)
+    check_cycles(shy, orc, h, drops, 2, kw)
