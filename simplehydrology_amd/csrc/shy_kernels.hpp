@@ -1881,18 +1881,34 @@ __global__ void __launch_bounds__(1024) tile_count_kernel(const TileParts* __res
   const TilePart P = list[blockIdx.x];
   for (int j = threadIdx.x; j < kTileCells; j += blockDim.x) cnt[j] = 0;
   __syncthreads();
-  const int base = P.tile << kTileBits, e1 = P.e1;
-  // four entries per thread in flight
-  for (int e = P.e0 + (int)threadIdx.x; e < e1; e += 4 * blockDim.x) {
-    int c[4];
+  const int base = P.tile << kTileBits;
+  // unsigned: indices run up to five rounds past the last entry
+  const uint32_t e1 = (uint32_t)P.e1;
+  // the next four entries of the thread are in flight while four are counted
+  // (unconditional loads: past the end the last entry, not counted; without
+  // that 65 us for 27.7 M entries of 1024^2, with it 45)
+  if (P.e0 < P.e1) {
+    int c[2][4];
+    auto load = [&](int b, uint32_t e) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int x = e + u * (int)blockDim.x;
-      c[u] = x < e1 ? ecell[x] - base : -1;
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t x = e + u * 1024;
+        c[b][u] = ecell[x < e1 ? x : e1 - 1];
+      }
+    };
+    const uint32_t e = (uint32_t)P.e0 + threadIdx.x;
+    const int rounds = (P.e1 - P.e0 + 4095) / 4096;
+    load(0, e);
+    for (int r = 0; r < rounds; r += 2) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const uint32_t eb = e + (r + b) * 4096;
+        load(b ^ 1, eb + 4096);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (eb + u * 1024 < e1) atomicAdd(&cnt[c[b][u] - base], 1);
+      }
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (c[u] >= 0) atomicAdd(&cnt[c[u]], 1);
   }
   __syncthreads();
   for (int j = threadIdx.x; j < kTileCells; j += blockDim.x) {
