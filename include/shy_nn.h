@@ -91,6 +91,12 @@ int shy_nn_conv_wgrad_noalloc(const void* x, const void* g, float* dw, int N, in
 /* db[c] = sum over pixels of g[p][c]; part holds part_rows*C floats */
 int shy_nn_bias_grad(const void* g, float* db, float* part, int part_rows, int P, int C,
                      void* stream);
+/* dw and db of one convolution (shy_nn_conv_wgrad and shy_nn_bias_grad), in
+   one pass over g where Cin and Cout are multiples of 32, taps = 9 and
+   part_splits > 1 */
+int shy_nn_conv_wgrad_bias(const void* x, const void* g, float* dw, float* db, float* part,
+                           int part_splits, float* bias_part, int bias_rows, int N, int H, int W,
+                           int Cin, int Cout, int taps, void* stream);
 int shy_nn_relu_bwd(const void* y, const void* g, void* out, size_t n, void* stream);
 /* 2x2 average pool (backward: x = dy, y = dx at full size) */
 int shy_nn_pool2(const void* x, void* y, int N, int H, int W, int C, int backward, void* stream);

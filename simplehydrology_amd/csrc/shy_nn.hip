@@ -771,141 +771,172 @@ __global__ void __launch_bounds__(64) conv_wgrad_kernel(WgradArgs a) {
 }
 
 // Weight gradient for Cin and Cout multiples of 32, TAPS = 9, staged through
-// LDS: dW[co][tap*Cin + ci] = sum_p g[p][co] x[p + tap][ci].  The reduction
-// runs over pixels, so both MFMA operands need 8 consecutive pixels of one
-// channel per lane: each 16x8 pixel tile is staged transposed (channel-major)
-// -- G^T [16*MT][128 pixels] and X^T [32][10 rows][24] (the tile with its
-// 1-pixel halo) -- four pixels per 8-byte LDS write.  A block owns 16*MT
-// output channels x one 32-channel input chunk x all 9 taps (18 N tiles of
-// 16), wave w the N tiles w, w+4, ...; it sums its range of pixel tiles into
-// one FP32 partial.  The +1 / +2 pixel shifts of the taps read two aligned
-// 16-byte rows of X^T and realign in registers.
-constexpr int kWgTW = 16, kWgTH = 8, kWgPix = kWgTW * kWgTH;
-constexpr int kXR = 24;  // X^T row: 18 halo columns padded to 24
-
-__device__ inline bf16x8 shift_pixels(bf16x8 lo, bf16x8 hi, int dx) {
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  if (dx == 0) return lo;
-  const u32x4 a = __builtin_bit_cast(u32x4, lo), b = __builtin_bit_cast(u32x4, hi);
-  u32x4 r;
-  if (dx == 2) {
-    r = u32x4{a[1], a[2], a[3], b[0]};
-  } else {  // one bf16 to the left: v_alignbyte of neighbouring dwords
-    r[0] = __builtin_amdgcn_alignbyte(a[1], a[0], 2);
-    r[1] = __builtin_amdgcn_alignbyte(a[2], a[1], 2);
-    r[2] = __builtin_amdgcn_alignbyte(a[3], a[2], 2);
-    r[3] = __builtin_amdgcn_alignbyte(b[0], a[3], 2);
-  }
-  return __builtin_bit_cast(bf16x8, r);
-}
+// LDS: dW[co][tap*Cin + ci] = sum_p g[p][co] x[p + tap][ci], and with a.bias
+// the bias gradient sum_p g[p][co] from the same tiles (a product with ones).
+// The reduction runs over pixels, so both MFMA operands need 8 pixels of one
+// channel per lane, while the tiles lie pixel by pixel: G [4 rows][32 pixels][co]
+// and X [6 rows][34 pixels][32 ci] (the 1-pixel halo).  They are staged as they
+// lie, and ds_read_b64_tr_b16 transposes while reading: each 16 lanes give four
+// pixels x 16 channels, lane j receives channel j of the four.  A tap's shift is
+// then only an address, also for odd columns.
+// A block owns 32*MTW output channels x 32 input channels x all 9 taps; wave w
+// the input channels 16*(w%2).. and the output channels of half w/2.  It goes
+// down the rows of X: a row's three column shifts are read once and serve the
+// three rows of G around it, which stay in registers (3 + MTW fragments read for
+// 9*MTW products; reading both operands for every tap cost 12 for 10, and the
+// LDS reads, not the matrix cores, bounded the kernel).  The next tile's
+// global loads are in flight meanwhile; off-image pixels are loaded from the
+// image's first pixel and stored as zeros, so no load depends on a branch.
+// Measured against tiles stored transposed and the shifts realigned in
+// registers, without the loads ahead: 16 x 32 x 32, 128 -> 128 channels 26.8 ->
+// 15.3 us; the launches of a training step of 16 windows of 256^2 81 -> 37 us on
+// average, and 22 launches of the bias kernels less.
+constexpr int kWgTW = 32, kWgTH = 4, kWgPix = kWgTW * kWgTH;
+constexpr int kWgXW = kWgTW + 2, kWgXPix = kWgXW * (kWgTH + 2);
+// Blocks of a launch: two per CU, which all run at once (64 output channels
+// per block fit two).  Training step, us per launch of blocks of 64 / of 32
+// channels / of the partials' sum: 256 blocks' worth of partials 42 / 42 / 6.1,
+// 512 29 / 43 / 6.8, 768 35 / 43 / 8.1, 1024 35 / 47 / 9.0.
+constexpr int kWgBlocks = 512;
+constexpr int kWgXS = 32 + 8;  // halfwords per pixel of X; 16 pixels cover the banks evenly
 
 struct WgArgs {
   const __bf16* __restrict__ x;
   const __bf16* __restrict__ g;
-  float* part;  // [splits][Cout][K]
+  float* part;  // [splits][Cout*K (+ Cout with bias)]
   int N, H, W, Cin, Cout, K;
+  int bias;
   int tiles_x, tiles_y, tiles;
   int tiles_per_split;
 };
 
-template <int MT>
+// 8 pixels of one channel: p = this lane's 4 channels of its pixel of the
+// first four, stride halfwords per pixel
+__device__ inline bf16x8 read_pixels8(const __bf16* p, int stride) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * stride));
+  return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+template <int MTW>
 __global__ void __launch_bounds__(256) wgrad_lds_kernel(WgArgs a) {
-  constexpr int NCO = 16 * MT;
-  constexpr int GS = kWgPix + 8;  // G^T row (pixels) with padding
-  __shared__ __bf16 gt[NCO * GS];
-  __shared__ __bf16 xt[32 * (kWgTH + 2) * kXR];
+  constexpr int NCO = 32 * MTW;
+  constexpr int GS = NCO + 8;
+  constexpr int RG = kWgPix * (NCO / 8) / 256, RX = (kWgXPix * 4 + 255) / 256;
+  __shared__ __align__(16) __bf16 gt[kWgPix * GS];
+  __shared__ __align__(16) __bf16 xt[kWgXPix * kWgXS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int cb = blockIdx.x * NCO, ci0 = blockIdx.y * 32;
   const int t_begin = blockIdx.z * a.tiles_per_split;
   const int t_end = min(a.tiles, t_begin + a.tiles_per_split);
   const int Cin = a.Cin, Cout = a.Cout;
-  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-  f32x4 acc[MT][5];
+  const bool bias = a.bias && ci0 == 0 && (wave & 1) == 0;  // uniform over the wave
+  f32x4 acc[9][MTW], accb[MTW];
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int m = 0; m < MTW; ++m) {
+    accb[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int j = 0; j < 5; ++j) acc[m][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int t = t_begin; t < t_end; ++t) {
+    for (int t = 0; t < 9; ++t) acc[t][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  bf16x8 rg[RG], rx[RX];
+  uint32_t okg = 0, okx = 0;
+  auto gload = [&](int t) {
     const int tx = t % a.tiles_x, ty = (t / a.tiles_x) % a.tiles_y;
     const int n = t / (a.tiles_x * a.tiles_y);
     const int x0 = tx * kWgTW, y0 = ty * kWgTH;
-    // G^T: task = (4 pixels of a row, 8 channels); pixels off the image are 0
-    for (int task = threadIdx.x; task < (kWgPix / 4) * (NCO / 8); task += 256) {
-      const int pq = task % (kWgPix / 4), cq = task / (kWgPix / 4);
-      const int pix = pq * 4, row = pix / kWgTW, col = pix % kWgTW;
-      bf16x8 v[4];
+    const __bf16* gi = a.g + (size_t)n * a.H * a.W * Cout + cb;
+    const __bf16* xi = a.x + (size_t)n * a.H * a.W * Cin + ci0;
+    okg = okx = 0;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int gy = y0 + row, gx = x0 + col + u;
-        v[u] = zero8();
-        if (gy < a.H && gx < a.W)
-          v[u] = load8(a.g + ((size_t)(n * a.H + gy) * a.W + gx) * Cout + cb + cq * 8);
-      }
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        bf16x4 w4 = {v[0][c], v[1][c], v[2][c], v[3][c]};
-        *reinterpret_cast<bf16x4*>(&gt[(cq * 8 + c) * GS + pix]) = w4;
-      }
+    for (int j = 0; j < RG; ++j) {
+      const int v = threadIdx.x + 256 * j, pix = v / (NCO / 8), q = v % (NCO / 8);
+      const int gy = y0 + pix / kWgTW, gx = x0 + pix % kWgTW;
+      const bool ok = gy < a.H && gx < a.W;
+      okg |= ok ? 1u << j : 0u;
+      rg[j] = load8(gi + (ok ? ((size_t)gy * a.W + gx) * Cout : 0) + q * 8);
     }
-    // X^T: task = (row of the halo tile, 4 halo columns, 8 channels)
-    for (int task = threadIdx.x; task < (kWgTH + 2) * 5 * 4; task += 256) {
-      const int r = task % (kWgTH + 2), rest = task / (kWgTH + 2);
-      const int cg = rest % 5, cq = rest / 5;
-      bf16x8 v[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int hc = cg * 4 + u;  // halo column 0..19 (18, 19 are padding)
-        const int gy = y0 + r - 1, gx = x0 + hc - 1;
-        v[u] = zero8();
-        if (hc < kWgTW + 2 && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W)
-          v[u] = load8(a.x + ((size_t)(n * a.H + gy) * a.W + gx) * Cin + ci0 + cq * 8);
-      }
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        bf16x4 w4 = {v[0][c], v[1][c], v[2][c], v[3][c]};
-        *reinterpret_cast<bf16x4*>(&xt[((cq * 8 + c) * (kWgTH + 2) + r) * kXR + cg * 4]) = w4;
-      }
+    for (int j = 0; j < RX; ++j) {
+      const int v = threadIdx.x + 256 * j, pix = v >> 2, q = v & 3;
+      const int gy = y0 + pix / kWgXW - 1, gx = x0 + pix % kWgXW - 1;
+      const bool ok = v < kWgXPix * 4 && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W;
+      okx |= ok ? 1u << j : 0u;
+      rx[j] = load8(xi + (ok ? ((size_t)gy * a.W + gx) * Cin : 0) + q * 8);
     }
+  };
+  auto lstore = [&]() {
+#pragma unroll
+    for (int j = 0; j < RG; ++j) {
+      const int v = threadIdx.x + 256 * j, pix = v / (NCO / 8), q = v % (NCO / 8);
+      *reinterpret_cast<bf16x8*>(&gt[pix * GS + q * 8]) = okg >> j & 1 ? rg[j] : zero8();
+    }
+#pragma unroll
+    for (int j = 0; j < RX; ++j) {
+      const int v = threadIdx.x + 256 * j;
+      if (v < kWgXPix * 4)
+        *reinterpret_cast<bf16x8*>(&xt[(v >> 2) * kWgXS + (v & 3) * 8]) =
+            okx >> j & 1 ? rx[j] : zero8();
+    }
+  };
+  // this lane's pixel of a row's first 4 of 8 (k group lane/16) and its 4 channels
+  const int pix0 = (lane >> 4) * 8 + ((lane & 15) >> 2), ch0 = (lane & 3) * 4;
+  const __bf16* gl = &gt[pix0 * GS + (wave >> 1) * 16 * MTW + ch0];
+  const __bf16* xl = &xt[pix0 * kWgXS + (wave & 1) * 16 + ch0];
+  bf16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+  gload(t_begin);
+  for (int t = t_begin; t < t_end; ++t) {
+    lstore();
     __syncthreads();
-    // 4 k-steps of 32 pixels (tile rows 2s, 2s+1)
+    if (t + 1 < t_end) gload(t + 1);
+    bf16x8 A[3][MTW];
 #pragma unroll
-    for (int s = 0; s < kWgPix / 32; ++s) {
-      const int grp = lane >> 4;  // 8-pixel group of this lane
-      const int R = 2 * s + (grp >> 1), c0 = (grp & 1) * 8;
-      bf16x8 A[MT];
+    for (int j = 0; j < kWgTH + 2; ++j) {
+      if (j < kWgTH) {
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-        A[m] = *reinterpret_cast<const bf16x8*>(&gt[(m * 16 + (lane & 15)) * GS + R * kWgTW + c0]);
+        for (int m = 0; m < MTW; ++m)
+          A[j % 3][m] = read_pixels8(gl + j * kWgTW * GS + m * 16, GS);
+        if (bias)
 #pragma unroll
-      for (int j = 0; j < 5; ++j) {
-        const int nt = wave + 4 * j;  // N tile: tap nt/2, channels 16*(nt%2) + 0..15
-        if (nt >= 18) continue;
-        const int tap = nt >> 1, dy = tap / 3, dx = tap % 3;
-        const int ci = (nt & 1) * 16 + (lane & 15);
-        const __bf16* row = &xt[(ci * (kWgTH + 2) + R + dy) * kXR + c0];
-        const bf16x8 lo = *reinterpret_cast<const bf16x8*>(row);
-        const bf16x8 hi = *reinterpret_cast<const bf16x8*>(row + 8);
-        const bf16x8 B = shift_pixels(lo, hi, dx);
+          for (int m = 0; m < MTW; ++m) accb[m] = mfma(A[j % 3][m], ones, accb[m]);
+      }
+      bf16x8 B[3];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m][j] = mfma(A[m], B, acc[m][j]);
+      for (int dx = 0; dx < 3; ++dx)
+        B[dx] = read_pixels8(xl + (j * kWgXW + dx) * kWgXS, kWgXS);
+      // X row j (image row y0 - 1 + j) under tap row dy meets G row j - dy
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy) {
+        if (j - dy < 0 || j - dy >= kWgTH) continue;
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+          for (int m = 0; m < MTW; ++m)
+            acc[dy * 3 + dx][m] = mfma(A[(j - dy) % 3][m], B[dx], acc[dy * 3 + dx][m]);
       }
     }
     __syncthreads();
   }
-  float* out = a.part + (size_t)blockIdx.z * Cout * a.K;
+  const size_t per = (size_t)Cout * a.K + (a.bias ? Cout : 0);
+  float* out = a.part + (size_t)blockIdx.z * per;
+  const int co0 = cb + (wave >> 1) * 16 * MTW + (lane >> 4) * 4;
+  const int k0 = ci0 + (wave & 1) * 16 + (lane & 15);
 #pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    const int nt = wave + 4 * j;
-    if (nt >= 18) continue;
-    const int k = (nt >> 1) * Cin + ci0 + (nt & 1) * 16 + (lane & 15);
+  for (int t = 0; t < 9; ++t)
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MTW; ++m)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int co = cb + m * 16 + (lane >> 4) * 4 + i;
-        out[(size_t)co * a.K + k] = acc[m][j][i];
-      }
-  }
+      for (int i = 0; i < 4; ++i)
+        out[(size_t)(co0 + m * 16 + i) * a.K + t * Cin + k0] = acc[t][m][i];
+  if (bias && (lane & 15) == 0)
+#pragma unroll
+    for (int m = 0; m < MTW; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[(size_t)Cout * a.K + co0 + m * 16 + i] = accb[m][i];
 }
 
 // dW[i] = sum over splits of part[k][i] in a fixed order (deterministic):
@@ -915,7 +946,8 @@ __global__ void __launch_bounds__(256) wgrad_lds_kernel(WgArgs a) {
 constexpr int kRedSlices = 8;
 
 __global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float* __restrict__ part,
-                                                           float* dw, int n, int splits) {
+                                                           float* dw, float* db, int nw, int n,
+                                                           int splits) {
   __shared__ float acc[kRedSlices][32];
   const int e = threadIdx.x & 31, sl = threadIdx.x >> 5;
   const int i = blockIdx.x * 32 + e;
@@ -938,7 +970,10 @@ __global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float* __restri
     float t = 0.0f;
 #pragma unroll
     for (int q = 0; q < kRedSlices; ++q) t += acc[q][e];
-    dw[i] = t;
+    if (i < nw)
+      dw[i] = t;
+    else
+      db[i - nw] = t;
   }
 }
 
@@ -1592,40 +1627,49 @@ int shy_nn_flip_weights(const void* w, void* wf, int Cin, int Cout, int taps, vo
   return nn_check("flip_weights");
 }
 
+// The weight gradient by wgrad_lds_kernel, and with db the bias gradient of
+// the same pass; part holds cap floats.
+static int wgrad_lds(const void* x, const void* g, float* dw, float* db, float* part, size_t cap,
+                     int N, int H, int W, int Cin, int Cout, hipStream_t s) {
+  WgArgs b;
+  b.x = (const __bf16*)x;
+  b.g = (const __bf16*)g;
+  b.part = part;
+  b.N = N; b.H = H; b.W = W; b.Cin = Cin; b.Cout = Cout; b.K = 9 * Cin;
+  b.bias = db != nullptr;
+  b.tiles_x = (W + kWgTW - 1) / kWgTW;
+  b.tiles_y = (H + kWgTH - 1) / kWgTH;
+  const long long tiles = (long long)N * b.tiles_x * b.tiles_y;
+  if (tiles > INT32_MAX) return nn_fail("conv_wgrad: too many tiles");
+  b.tiles = (int)tiles;
+  const int mtw = Cout % 64 == 0 ? 2 : 1;
+  const int bxy = (Cout / (32 * mtw)) * (Cin / 32);
+  const int nw = Cout * b.K, n = nw + (db ? Cout : 0);
+  // about kWgBlocks blocks, as many partials as part holds, at least one tile
+  // each: fewer partials to sum afterwards
+  long long splits =
+      std::max(1LL, std::min<long long>((kWgBlocks + bxy - 1) / bxy, tiles));
+  splits = std::min<long long>(splits, (long long)(cap / (size_t)n));
+  b.tiles_per_split = (int)((tiles + splits - 1) / splits);
+  splits = (tiles + b.tiles_per_split - 1) / b.tiles_per_split;
+  dim3 grid((unsigned)(Cout / (32 * mtw)), (unsigned)(Cin / 32), (unsigned)splits);
+  if (mtw == 2)
+    wgrad_lds_kernel<2><<<grid, 256, 0, s>>>(b);
+  else
+    wgrad_lds_kernel<1><<<grid, 256, 0, s>>>(b);
+  if (int r = nn_check("conv_wgrad")) return r;
+  wgrad_reduce_kernel<<<(n + 31) / 32, 256, 0, s>>>(part, dw, db, nw, n, (int)splits);
+  return nn_check("wgrad_reduce");
+}
+
 int shy_nn_conv_wgrad(const void* x, const void* g, float* dw, float* part, int part_splits,
                       int N, int H, int W, int Cin, int Cout, int taps, void* stream) {
   if (!x || !g || !dw || !part || part_splits < 1) return nn_fail("conv_wgrad: bad pointers");
   if (Cin % 8 || Cout % 8 || (taps != 9 && taps != 1)) return nn_fail("conv_wgrad: channels must be multiples of 8");
   const long long P = (long long)N * H * W;
-  if (taps == 9 && Cin % 32 == 0 && Cout % 32 == 0) {
-    WgArgs b;
-    b.x = (const __bf16*)x;
-    b.g = (const __bf16*)g;
-    b.part = part;
-    b.N = N; b.H = H; b.W = W; b.Cin = Cin; b.Cout = Cout; b.K = 9 * Cin;
-    b.tiles_x = (W + kWgTW - 1) / kWgTW;
-    b.tiles_y = (H + kWgTH - 1) / kWgTH;
-    const long long tiles = (long long)N * b.tiles_x * b.tiles_y;
-    if (tiles > INT32_MAX) return nn_fail("conv_wgrad: too many tiles");
-    b.tiles = (int)tiles;
-    // 32 output channels per block, as in the forward (64-channel blocks
-    // ran at two waves per SIMD: training step 4.538 -> 4.513 ms)
-    const int mt = 2;
-    const int bxy = (Cout / (16 * mt)) * (Cin / 32);
-    // about 1024 blocks (4 waves per CU), at most part_splits partials, at
-    // least one tile each: fewer partials to sum afterwards
-    long long splits = std::max(1LL, std::min<long long>((1024 + bxy - 1) / bxy, tiles));
-    splits = std::min<long long>(splits, part_splits);
-    b.tiles_per_split = (int)((tiles + splits - 1) / splits);
-    splits = (tiles + b.tiles_per_split - 1) / b.tiles_per_split;
-    hipStream_t s = (hipStream_t)stream;
-    dim3 grid((unsigned)(Cout / (16 * mt)), (unsigned)(Cin / 32), (unsigned)splits);
-    wgrad_lds_kernel<2><<<grid, 256, 0, s>>>(b);
-    if (int r = nn_check("conv_wgrad")) return r;
-    const int n = Cout * b.K;
-    wgrad_reduce_kernel<<<(n + 31) / 32, 256, 0, s>>>(part, dw, n, (int)splits);
-    return nn_check("wgrad_reduce");
-  }
+  if (taps == 9 && Cin % 32 == 0 && Cout % 32 == 0)
+    return wgrad_lds(x, g, dw, nullptr, part, (size_t)part_splits * Cout * 9 * Cin, N, H, W, Cin,
+                     Cout, (hipStream_t)stream);
   int chunk = (int)((P + part_splits - 1) / part_splits);
 
   chunk = (chunk + 31) / 32 * 32;
@@ -1641,7 +1685,7 @@ int shy_nn_conv_wgrad(const void* x, const void* g, float* dw, float* part, int 
   conv_wgrad_kernel<<<grid, 64, 0, s>>>(a);
   if (int r = nn_check("conv_wgrad")) return r;
   const int n = Cout * a.K;
-  wgrad_reduce_kernel<<<(n + 31) / 32, 256, 0, s>>>(part, dw, n, splits);
+  wgrad_reduce_kernel<<<(n + 31) / 32, 256, 0, s>>>(part, dw, nullptr, n, n, splits);
   return nn_check("wgrad_reduce");
 }
 
@@ -1679,8 +1723,23 @@ int shy_nn_bias_grad(const void* g, float* db, float* part, int part_rows, int P
   const int nb = (P + rows - 1) / rows;
   bias_grad_kernel<<<nb, 256, 0, s>>>((const __bf16*)g, part, P, C, rows);
   if (int r = nn_check("bias_grad")) return r;
-  wgrad_reduce_kernel<<<(C + 31) / 32, 256, 0, s>>>(part, db, C, nb);
+  wgrad_reduce_kernel<<<(C + 31) / 32, 256, 0, s>>>(part, db, nullptr, C, C, nb);
   return nn_check("bias_grad_reduce");
+}
+
+int shy_nn_conv_wgrad_bias(const void* x, const void* g, float* dw, float* db, float* part,
+                           int part_splits, float* bias_part, int bias_rows, int N, int H, int W,
+                           int Cin, int Cout, int taps, void* stream) {
+  // one pass over g gives both where the weight gradient stages it by tiles and
+  // part has room for the bias sums beside the weights'
+  if (x && g && dw && db && part && part_splits > 1 && taps == 9 && Cin > 0 && Cout > 0 &&
+      Cout <= 1024 &&  // as shy_nn_bias_grad
+      Cin % 32 == 0 && Cout % 32 == 0)
+    return wgrad_lds(x, g, dw, db, part, (size_t)part_splits * Cout * 9 * Cin, N, H, W, Cin, Cout,
+                     (hipStream_t)stream);
+  if (int r = shy_nn_conv_wgrad(x, g, dw, part, part_splits, N, H, W, Cin, Cout, taps, stream))
+    return r;
+  return shy_nn_bias_grad(g, db, bias_part, bias_rows, N * H * W, Cout, stream);
 }
 
 inline bool a16(const void* p) { return ((uintptr_t)p & 15) == 0; }

@@ -51,6 +51,8 @@ def nn():
             "shy_nn_flip_weights": (i32, [vp, vp, i32, i32, i32, vp]),
             "shy_nn_conv_wgrad": (i32, [vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, vp]),
             "shy_nn_conv_wgrad_noalloc": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
+            "shy_nn_conv_wgrad_bias": (i32, [vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32,
+                                             i32, i32, vp]),
             "shy_nn_bias_grad": (i32, [vp, vp, vp, i32, i32, i32, vp]),
             "shy_nn_relu_bwd": (i32, [vp, vp, vp, sz, vp]),
             "shy_nn_pool2": (i32, [vp, vp, i32, i32, i32, i32, i32, vp]),
@@ -219,10 +221,9 @@ class Conv:
         N, H, W = shape
         P = N * H * W
         part, splits = scratch.part_for(self, P)
-        _ck(nn().shy_nn_conv_wgrad(_p(x), _p(g), _p(self.dw), _p(part), splits, N, H, W,
-                                   self.cin, self.cout, self.taps, _stream()))
-        _ck(nn().shy_nn_bias_grad(_p(g), _p(self.db), _p(scratch.bias_part), scratch.bias_rows,
-                                  P, self.cout, _stream()))
+        _ck(nn().shy_nn_conv_wgrad_bias(_p(x), _p(g), _p(self.dw), _p(self.db), _p(part), splits,
+                                        _p(scratch.bias_part), scratch.bias_rows, N, H, W,
+                                        self.cin, self.cout, self.taps, _stream()))
         if not need_dx:
             return None
         if self._wf_of != (self.w_bf.data_ptr(), self.w_bf._version):
@@ -265,10 +266,12 @@ class Scratch:
         self.bias_part = torch.empty(self.bias_rows * 1024, dtype=torch.float32, device=device)
 
     def part_for(self, conv, P):
+        fit = self.part.numel() // (conv.cout * conv.taps * conv.cin)
+        if conv.taps == 9 and conv.cin % 32 == 0 and conv.cout % 32 == 0:
+            return self.part, max(1, fit)  # an upper bound: the library splits by its grid
         tiles = ((conv.cout + 31) // 32) * ((conv.taps * conv.cin + 31) // 32)
         splits = max(1, min(P // 512, -(-4096 // tiles)))
-        splits = min(splits, self.part.numel() // (conv.cout * conv.taps * conv.cin))
-        return self.part, max(1, splits)
+        return self.part, max(1, min(splits, fit))
 
 
 def _relu_bwd(y, g):
