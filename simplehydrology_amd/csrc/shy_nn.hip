@@ -108,11 +108,8 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 // One lane's 4 consecutive output channels co..co+3 of output element o:
 // bias, residual (before rounding), ReLU, then the store, FP32 or BF16 (with
-// the backward-pass residual and mask after rounding).  Returns the stored
-// BF16 values (zeros for an FP32 output); with HEAD a null y_bf stores
-// nothing.
-template <bool HEAD>
-__device__ inline bf16x4 store_out4(const ConvArgs& a, size_t o, int co, const f32x4& acc) {
+// the backward-pass residual and mask after rounding).
+__device__ inline void store_out4(const ConvArgs& a, size_t o, int co, const f32x4& acc) {
   float v[4];
   // the lane's 4 biases in one load: co is a multiple of 4 and the entry
   // points require a 16-byte aligned bias
@@ -130,12 +127,10 @@ __device__ inline bf16x4 store_out4(const ConvArgs& a, size_t o, int co, const f
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
   }
-  bf16x4 q;
   if (a.y_f) {
     *reinterpret_cast<float4*>(a.y_f + o) = make_float4(v[0], v[1], v[2], v[3]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q[i] = (__bf16)0.0f;
   } else {
+    bf16x4 q;
 #pragma unroll
     for (int i = 0; i < 4; ++i) q[i] = (__bf16)v[i];
     if (a.gres) {
@@ -146,9 +141,8 @@ __device__ inline bf16x4 store_out4(const ConvArgs& a, size_t o, int co, const f
 #pragma unroll
       for (int i = 0; i < 4; ++i) q[i] = (float)a.mask[o + i] > 0.0f ? q[i] : (__bf16)0.0f;
     }
-    if (!HEAD || a.y_bf) *reinterpret_cast<bf16x4*>(a.y_bf + o) = q;
+    *reinterpret_cast<bf16x4*>(a.y_bf + o) = q;
   }
-  return q;
 }
 
 // The 1x1 head on a tile's rounded 32-channel output q (ConvArgs::head_w),
@@ -197,29 +191,11 @@ __device__ inline void conv_head(const ConvArgs& a, const bf16x4 (&q)[2][NT], in
   }
 }
 
-// The epilogue of a block's tile: lane holds channels cb + 16m + 4(lane/16)
-// + i of pixel (y0 + NT wave + t, x0 + lane%16).  HEAD: then the 1x1 head
-// (its own instantiation: the rounded outputs it keeps cost registers).
-template <int MT, int NT, bool HEAD = false, bool POOL = false>
-__device__ inline void conv_epilogue(const ConvArgs& a, const f32x4 (&acc)[MT][NT], int n, int y0,
-                                     int x0, int cb, int wave, int lane) {
-  static_assert(!POOL || NT % 2 == 0, "the pool pairs a wave's rows");
-  static_assert(!HEAD || MT == 2, "the head reads a block's 32 output channels");
+// What follows a tile's rounded outputs q: the 1x1 head, the 2x2 pool.
+template <int MT, int NT, bool HEAD, bool POOL>
+__device__ inline void conv_after(const ConvArgs& a, const bf16x4 (&q)[MT][NT], int n, int y0,
+                                  int x0, int cb, int wave, int lane) {
   const int gx = x0 + (lane & 15);
-  bf16x4 q[MT][NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int gy = y0 + wave * NT + t;
-    const size_t p = (size_t)(n * a.H + gy) * a.W + gx;
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const int co = cb + m * 16 + (lane >> 4) * 4;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) q[m][t][i] = (__bf16)0.0f;
-      if (gy < a.H && gx < a.W && co < a.Cout)
-        q[m][t] = store_out4<HEAD>(a, p * a.Cout + co, co, acc[m][t]);
-    }
-  }
   if constexpr (HEAD) conv_head<NT>(a, q, n, y0, x0, wave, lane);
   if constexpr (POOL) {
     // Rows y0 + NT wave + t pair as (t, t + 1) for even t (y0 and NT wave
@@ -254,6 +230,24 @@ __device__ inline void conv_epilogue(const ConvArgs& a, const f32x4 (&acc)[MT][N
           *reinterpret_cast<bf16x4*>(a.pool_y + pp + co) = o;
         }
       }
+    }
+  }
+}
+
+// The epilogue of a block's tile: lane holds channels cb + 16m + 4(lane/16)
+// + i of pixel (y0 + NT wave + t, x0 + lane%16).
+template <int MT, int NT>
+__device__ inline void conv_epilogue(const ConvArgs& a, const f32x4 (&acc)[MT][NT], int n, int y0,
+                                     int x0, int cb, int wave, int lane) {
+  const int gx = x0 + (lane & 15);
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int gy = y0 + wave * NT + t;
+    const size_t p = (size_t)(n * a.H + gy) * a.W + gx;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int co = cb + m * 16 + (lane >> 4) * 4;
+      if (gy < a.H && gx < a.W && co < a.Cout) store_out4(a, p * a.Cout + co, co, acc[m][t]);
     }
   }
 }
@@ -485,21 +479,56 @@ __global__ void __launch_bounds__(256, 2) conv_pf_kernel(ConvArgs a) {
 // leaves every block waiting for its patch.  A single-chunk layer loads its
 // weights once per block.  Three blocks per compute unit with 32 output
 // channels per block (MT = 2): at most 168 VGPRs and 45 KB of LDS each.
+//
+// The address work is kept off the vector units, which issue it in the shadow
+// of nothing (a step of 72 MFMAs per wave came with 460 other vector
+// instructions and a branch per load and bounds check; level-0 layers spent
+// as long issuing as waiting for memory): every access goes through a buffer
+// whose base the scalar unit sets per tile, with a lane offset that never
+// changes.  A row above the image gives an offset that wraps and a row below
+// one past the buffer's end; both read zeros and store nothing, as the
+// hardware checks each offset against the buffer's size, so only the tiles at
+// the left and right edge compare columns.  The rows of one tile must span
+// less than 2^31 bytes (tile_rows_fit).  A tile's residual (kEpiRes) or the
+// backward pass's residual and mask (kEpiGrad) are on their way while the next
+// tile goes to LDS.
+// Measured against the same loop with an address, a bounds check and a branch
+// per load (us, at batch 16): 256^2, 32 -> 32 channels 40.1 -> 28.9 (4.6 TB/s),
+// with residual and pool 65.2 -> 41.9; 128^2, 64 -> 64 38.2 -> 32.1; 64^2,
+// 96 -> 96 21.3 -> 18.6; 256^2, [up2, skip] 96 -> 32 85.1 -> 73.9.
 constexpr int kTileBlocksPerCU = 3;
 
-template <int TAPS, int MT, int NT, bool UPCAT = false, bool HEAD = false, bool POOL = false>
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// offset past the end of every buffer, also with a tile's offset added
+constexpr uint32_t kOffNone = 0x80000000u;
+
+// [base, base + bytes): reads past it give 0, writes past it are dropped
+__device__ inline __amdgpu_buffer_rsrc_t tile_buffer(const void* base, long long bytes) {
+  const int n = bytes < 0x7fffffffLL ? (int)bytes : 0x7fffffff;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, n, 0x00020000);
+}
+
+inline bool tile_rows_fit(const ConvArgs& a) {
+  const long long c = std::max(a.Cin, 2 * a.Cout);  // an FP32 output counts twice
+  return (long long)a.W * c * 2 * 20 < 0x7fffffffLL;
+}
+
+enum { kEpiPlain, kEpiRes, kEpiGrad };
+
+template <int MT, int NT, bool UPCAT, bool HEAD, bool POOL, int EPI>
 __global__ void __launch_bounds__(256, kTileBlocksPerCU) conv_tiles_kernel(ConvArgs a) {
   static_assert(MT == 2, "three blocks per CU fit 32 output channels per block");
+  static_assert(!POOL || NT % 2 == 0, "the pool pairs a wave's rows");
   constexpr int kTH = 4 * NT;
-  constexpr int HALO = TAPS == 9 ? 1 : 0;
-  constexpr int PW = kTW + 2 * HALO, PH = kTH + 2 * HALO;
-  constexpr int WS = TAPS * 32 + 8;  // LDS bf16 per output channel of the weight chunk
-  constexpr int NPV = PH * PW * 4;             // 16-byte patch vectors per chunk
-  constexpr int NWV = MT * 16 * TAPS * 4;      // 16-byte weight vectors per chunk
+  constexpr int PW = kTW + 2, PH = kTH + 2;
+  constexpr int WS = 9 * 32 + 8;          // LDS bf16 per output channel of the weight chunk
+  constexpr int NPV = PH * PW * 4;        // 16-byte patch vectors per chunk
+  constexpr int NWV = MT * 16 * 9 * 4;    // 16-byte weight vectors per chunk
   constexpr int RP = (NPV + 255) / 256, RW = (NWV + 255) / 256;
-  constexpr int NS = 2 * HALO + 1;             // column (and row) shifts
-  __shared__ __bf16 patch[PH * PW * kPS];
-  __shared__ __bf16 wl[MT * 16 * WS];
+  __shared__ __align__(16) __bf16 patch[PH * PW * kPS];
+  __shared__ __align__(16) __bf16 wl[MT * 16 * WS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tiles_x = (a.W + kTW - 1) / kTW, tiles_y = (a.H + kTH - 1) / kTH;
   const int total = a.N * tiles_x * tiles_y;
@@ -508,92 +537,115 @@ __global__ void __launch_bounds__(256, kTileBlocksPerCU) conv_tiles_kernel(ConvA
   const int cb = blockIdx.y * MT * 16;
   const int Cin = a.Cin, K = a.K;
   const bool reload_w = Cin > 32;  // one chunk: its weights stay in LDS
-  bf16x8 rp[RP], rw[RW];
+  // this thread's patch and weight vectors, in bytes from the tile's first
+  // halo pixel (UPCAT: of the second input, and poh of the half-size first one)
+  const int CS = UPCAT ? Cin - a.C1 : Cin, Wh = a.W >> 1;
+  uint32_t po[RP], poh[RP], wo[RW];
+#pragma unroll
+  for (int j = 0; j < RP; ++j) {
+    const int v = threadIdx.x + 256 * j, pix = v >> 2, py = pix / PW, px = pix % PW;
+    po[j] = v < NPV ? (uint32_t)((py * a.W + px) * CS * 2 + (v & 3) * 16) : kOffNone;
+    if (UPCAT)
+      poh[j] = v < NPV ? (uint32_t)((((py + 1) >> 1) * Wh + ((px + 1) >> 1)) * a.C1 * 2 + (v & 3) * 16)
+                       : kOffNone;
+  }
+#pragma unroll
+  for (int j = 0; j < RW; ++j) {
+    const int v = threadIdx.x + 256 * j, co = v / 36, r = v % 36;
+    wo[j] = v < NWV ? (uint32_t)((co * K + (r >> 2) * Cin) * 2 + (r & 3) * 16) : kOffNone;
+  }
+  const __amdgpu_buffer_rsrc_t wbuf =
+      tile_buffer(a.w + (size_t)cb * K, (long long)MT * 16 * K * 2);
+  u32x4 rp[RP], rw[RW];
   auto gload = [&](int t, int ci0, bool wts) {
     const int tx = t % tiles_x, r = t / tiles_x;
     const int x0 = tx * kTW, y0 = (r % tiles_y) * kTH, n = r / tiles_y;
+    const bool edge = x0 == 0 || x0 + kTW >= a.W;
+    const bool half = UPCAT && ci0 < a.C1;
+    // the buffer: the image's rows from the patch's first one on
+    const int C = half ? a.C1 : CS, w = half ? Wh : a.W, h = half ? a.H >> 1 : a.H;
+    const int sx = half ? x0 >> 1 : x0, sy = half ? y0 >> 1 : y0, c0 = UPCAT && !half ? ci0 - a.C1 : ci0;
+    const int row0 = sy > 0 ? sy - 1 : 0;
+    const __bf16* src = UPCAT && !half ? a.x2 : a.x;
+    const long long row_bytes = (long long)w * C * 2;
+    const __amdgpu_buffer_rsrc_t buf =
+        tile_buffer(src + ((size_t)n * h + row0) * w * C, (h - row0) * row_bytes);
+    const uint32_t toff =
+        (uint32_t)((sy - 1 - row0) * (int)row_bytes + (sx - 1) * C * 2 + c0 * 2);
 #pragma unroll
     for (int j = 0; j < RP; ++j) {
-      const int v = threadIdx.x + 256 * j;
-      bf16x8 val = zero8();
-      if (v < NPV) {
-        const int pix = v >> 2, q = v & 3;
-        const int py = pix / PW, px = pix % PW;
-        const int gy = y0 + py - HALO, gx = x0 + px - HALO;
-        if (gy >= 0 && gy < a.H && gx >= 0 && gx < a.W) {
-          const __bf16* src;
-          if (!UPCAT)
-            src = a.x + ((size_t)(n * a.H + gy) * a.W + gx) * Cin + ci0;
-          else if (ci0 < a.C1)  // upsampled half: pixel (gy/2, gx/2) of x
-            src = a.x + ((size_t)(n * (a.H >> 1) + (gy >> 1)) * (a.W >> 1) + (gx >> 1)) * a.C1 + ci0;
-          else
-            src = a.x2 + ((size_t)(n * a.H + gy) * a.W + gx) * (Cin - a.C1) + (ci0 - a.C1);
-          val = load8(src + q * 8);
-        }
+      uint32_t o = (half ? poh[j] : po[j]) + toff;
+      if (edge) {
+        const int px = ((threadIdx.x + 256 * j) >> 2) % PW;
+        if ((uint32_t)(x0 - 1 + px) >= (uint32_t)a.W) o = kOffNone;
       }
-      rp[j] = val;
+      rp[j] = __builtin_amdgcn_raw_buffer_load_b128(buf, o, 0, 0);
     }
     if (wts) {
 #pragma unroll
-      for (int j = 0; j < RW; ++j) {
-        const int v = threadIdx.x + 256 * j;
-        bf16x8 val = zero8();
-        if (v < NWV) {
-          const int co = v / (TAPS * 4), r2 = v % (TAPS * 4);
-          const int tap = r2 >> 2, q = r2 & 3;
-          if (cb + co < a.Cout) val = load8(a.w + (size_t)(cb + co) * K + tap * Cin + ci0 + q * 8);
-        }
-        rw[j] = val;
-      }
+      for (int j = 0; j < RW; ++j)
+        rw[j] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, wo[j] + (uint32_t)ci0 * 2, 0, 0);
     }
   };
   auto lstore = [&](bool wts) {
 #pragma unroll
     for (int j = 0; j < RP; ++j) {
       const int v = threadIdx.x + 256 * j;
-      if (v < NPV)
-        *reinterpret_cast<bf16x8*>(&patch[(v >> 2) * kPS + (v & 3) * 8]) = rp[j];
+      if (v < NPV) *reinterpret_cast<u32x4*>(&patch[(v >> 2) * kPS + (v & 3) * 8]) = rp[j];
     }
     if (wts) {
 #pragma unroll
       for (int j = 0; j < RW; ++j) {
         const int v = threadIdx.x + 256 * j;
         if (v < NWV) {
-          const int co = v / (TAPS * 4), r2 = v % (TAPS * 4);
-          *reinterpret_cast<bf16x8*>(&wl[co * WS + (r2 >> 2) * 32 + (r2 & 3) * 8]) = rw[j];
+          const int co = v / 36, r2 = v % 36;
+          *reinterpret_cast<u32x4*>(&wl[co * WS + (r2 >> 2) * 32 + (r2 & 3) * 8]) = rw[j];
         }
       }
     }
   };
+  // this lane's outputs, in bytes (BF16) from the tile's first pixel
+  const uint32_t lane_out =
+      (uint32_t)((wave * NT * a.W + (lane & 15)) * a.Cout * 2 + (lane >> 4) * 8);
   gload(tile, 0, true);
   lstore(true);
   __syncthreads();
   for (;;) {
+    const int tx = tile % tiles_x, r = tile / tiles_x;
+    const int n = r / tiles_y, y0 = (r % tiles_y) * kTH, x0 = tx * kTW;
+    const size_t out0 = (((size_t)n * a.H + y0) * a.W + x0) * a.Cout + cb;
+    const long long out_bytes = (((long long)(a.H - y0)) * a.W - x0) * a.Cout * 2 - cb * 2;
+    const uint32_t lo = x0 + (lane & 15) < a.W ? lane_out : kOffNone;
     f32x4 acc[MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int ci0 = 0; ci0 < Cin; ci0 += 32) {
+    auto load_out = [&](const __bf16* p, u32x2 (&e)[MT][NT]) {
+      const __amdgpu_buffer_rsrc_t buf = tile_buffer(p + out0, p ? out_bytes : 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          e[m][t] = __builtin_amdgcn_raw_buffer_load_b64(
+              buf, lo + (uint32_t)(t * a.W * a.Cout * 2) + m * 32, 0, 0);
+    };
+    for (int ci0 = 0;; ci0 += 32) {
       // the next (tile, chunk) of this block
-      int nt = tile, nc = ci0 + 32;
-      if (nc >= Cin) {
-        nt = tile + (int)gridDim.x;
-        nc = 0;
-      }
-      const bool more = nt < total;
-      if (more) gload(nt, nc, reload_w);
+      const bool last = ci0 + 32 >= Cin;
+      const int nt = last ? tile + (int)gridDim.x : tile;
+      if (nt < total) gload(nt, last ? 0 : ci0 + 32, reload_w);
 #pragma unroll
-      for (int dx = 0; dx < NS; ++dx) {
-        bf16x8 B[NT + 2 * HALO];
+      for (int dx = 0; dx < 3; ++dx) {
+        bf16x8 B[NT + 2];
 #pragma unroll
-        for (int r = 0; r < NT + 2 * HALO; ++r) {
+        for (int r = 0; r < NT + 2; ++r) {
           const int row = wave * NT + r, col = (lane & 15) + dx;
           B[r] = *reinterpret_cast<const bf16x8*>(&patch[(row * PW + col) * kPS + (lane >> 4) * 8]);
         }
 #pragma unroll
-        for (int dy = 0; dy < NS; ++dy) {
-          const int tap = dy * NS + dx;
+        for (int dy = 0; dy < 3; ++dy) {
+          const int tap = dy * 3 + dx;
           bf16x8 A[MT];
 #pragma unroll
           for (int m = 0; m < MT; ++m)
@@ -605,15 +657,73 @@ __global__ void __launch_bounds__(256, kTileBlocksPerCU) conv_tiles_kernel(ConvA
             for (int t = 0; t < NT; ++t) acc[m][t] = mfma(A[m], B[t + dy], acc[m][t]);
         }
       }
+      if (last) break;
       __syncthreads();
-      if (more) {
-        lstore(reload_w);
-        __syncthreads();
+      lstore(reload_w);
+      __syncthreads();
+    }
+    u32x2 e0[MT][NT], e1[MT][NT];
+    if (EPI == kEpiRes) load_out(a.res, e0);
+    if (EPI == kEpiGrad) {
+      load_out(a.gres, e0);
+      load_out(a.mask, e1);
+    }
+    if (tile + (int)gridDim.x < total) {
+      __syncthreads();
+      lstore(reload_w);
+      __syncthreads();
+    }
+    // store_out4's steps
+    bf16x4 q[MT][NT];
+    float4 bias[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      bias[m] = a.bias ? *reinterpret_cast<const float4*>(a.bias + cb + m * 16 + (lane >> 4) * 4)
+                       : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const bool bf_out = !a.y_f && (!HEAD || a.y_bf);
+    const __amdgpu_buffer_rsrc_t ybuf = tile_buffer(a.y_bf + out0, bf_out ? out_bytes : 0);
+    const __amdgpu_buffer_rsrc_t fbuf = tile_buffer(a.y_f + out0, a.y_f ? 2 * out_bytes : 0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const uint32_t o = lo + (uint32_t)(t * a.W * a.Cout * 2) + m * 32;
+        float v[4] = {acc[m][t][0] + bias[m].x, acc[m][t][1] + bias[m].y,
+                      acc[m][t][2] + bias[m].z, acc[m][t][3] + bias[m].w};
+        if (EPI == kEpiRes) {
+          const bf16x4 res = __builtin_bit_cast(bf16x4, e0[m][t]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] += (float)res[i];
+        }
+        if (a.relu) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[m][t][i] = (__bf16)v[i];
+        if (EPI == kEpiGrad) {
+          const bf16x4 gr = __builtin_bit_cast(bf16x4, e0[m][t]);
+          const bf16x4 mk = __builtin_bit_cast(bf16x4, e1[m][t]);
+          if (a.gres) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) q[m][t][i] = (__bf16)((float)q[m][t][i] + (float)gr[i]);
+          }
+          if (a.mask) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              q[m][t][i] = (float)mk[i] > 0.0f ? q[m][t][i] : (__bf16)0.0f;
+          }
+        }
+        if (bf_out)
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, q[m][t]), ybuf, o, 0, 0);
+        if (a.y_f) {
+          const float4 f = make_float4(v[0], v[1], v[2], v[3]);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f), fbuf,
+                                                 lo == kOffNone ? kOffNone : 2 * o, 0, 0);
+        }
       }
     }
-    const int tx = tile % tiles_x, r = tile / tiles_x;
-    conv_epilogue<MT, NT, HEAD, POOL>(a, acc, r / tiles_y, (r % tiles_y) * kTH, tx * kTW, cb,
-                                      wave, lane);
+    conv_after<MT, NT, HEAD, POOL>(a, q, n, y0, x0, cb, wave, lane);
     tile += (int)gridDim.x;
     if (tile >= total) break;
   }
@@ -1383,10 +1493,22 @@ int launch_tiles(const ConvArgs& a, hipStream_t s, const char* what) {
   const int gy = a.Cout / (16 * MT);
   const long long cap = std::max(1LL, (long long)kTileBlocksPerCU * device_cus() / gy);
   const dim3 g((unsigned)std::min(tiles, cap), (unsigned)gy);
-  if (a.x2) conv_tiles_kernel<9, MT, NT, true, false><<<g, 256, 0, s>>>(a);
-  else if (a.head_w) conv_tiles_kernel<9, MT, NT, false, true><<<g, 256, 0, s>>>(a);
-  else if (a.pool_y) conv_tiles_kernel<9, MT, NT, false, false, true><<<g, 256, 0, s>>>(a);
-  else conv_tiles_kernel<9, MT, NT, false, false><<<g, 256, 0, s>>>(a);
+  const bool grad = a.gres || a.mask;
+  if (a.x2) {
+    if (a.res) conv_tiles_kernel<MT, NT, true, false, false, kEpiRes><<<g, 256, 0, s>>>(a);
+    else conv_tiles_kernel<MT, NT, true, false, false, kEpiPlain><<<g, 256, 0, s>>>(a);
+  } else if (a.head_w) {
+    if (a.res) conv_tiles_kernel<MT, NT, false, true, false, kEpiRes><<<g, 256, 0, s>>>(a);
+    else conv_tiles_kernel<MT, NT, false, true, false, kEpiPlain><<<g, 256, 0, s>>>(a);
+  } else if (a.pool_y) {
+    if (a.res) conv_tiles_kernel<MT, NT, false, false, true, kEpiRes><<<g, 256, 0, s>>>(a);
+    else conv_tiles_kernel<MT, NT, false, false, true, kEpiPlain><<<g, 256, 0, s>>>(a);
+  } else if (grad) {
+    conv_tiles_kernel<MT, NT, false, false, false, kEpiGrad><<<g, 256, 0, s>>>(a);
+  } else {
+    if (a.res) conv_tiles_kernel<MT, NT, false, false, false, kEpiRes><<<g, 256, 0, s>>>(a);
+    else conv_tiles_kernel<MT, NT, false, false, false, kEpiPlain><<<g, 256, 0, s>>>(a);
+  }
   return nn_check(what);
 }
 
@@ -1401,7 +1523,7 @@ int launch_pf(const ConvArgs& a, int taps, hipStream_t s, const char* what) {
   // blocks below: 32->32 at 256^2 50.7 -> 43.4 us, [up2, skip] 96->32 at
   // 256^2 105 -> 83 us, 96->96 at 64^2 23.0 -> 21.5 us; at 32^2, 64 tiles,
   // the one-tile blocks' 16x8 tiles are faster)
-  if (taps == 9 && tiles16 >= device_cus()) return launch_tiles(a, s, what);
+  if (taps == 9 && tiles16 >= device_cus() && tile_rows_fit(a)) return launch_tiles(a, s, what);
   const unsigned gy = (unsigned)(a.Cout / 32);
   const long long tiles8 = (long long)a.N * ((a.H + 7) / 8) * ((a.W + kTW - 1) / kTW);
   if (tiles8 > INT32_MAX) return nn_fail(std::string(what) + ": too many tiles");
@@ -1529,6 +1651,13 @@ int shy_nn_conv_fwd_head(const void* x, const void* w, const float* bias, const 
   a.head_b = head_b;
   a.head_y = head_y;
   a.head_c = head_c;
+  if (!tile_rows_fit(a)) {  // rows beyond the tile loop's offsets: two passes
+    if (!y_bf16) return nn_fail("conv_fwd_head: rows too long without an output for y");
+    if (int r = shy_nn_conv_fwd(x, w, bias, res, y_bf16, nullptr, N, H, W, Cin, 32, 9, relu, stream))
+      return r;
+    return shy_nn_conv_fwd(y_bf16, head_w, head_b, nullptr, nullptr, head_y, N, H, W, 32, head_c, 1,
+                           0, stream);
+  }
   return launch_tiles(a, (hipStream_t)stream, "conv_fwd_head");
 }
 
@@ -1569,14 +1698,15 @@ int shy_nn_conv_fwd_pool(const void* x, const void* w, const float* bias, const 
     return nn_fail("conv_fwd_pool: need H, W even and Cin, Cout multiples of 32");
   if ((long long)N * H * W > INT32_MAX / 2) return nn_fail("conv_fwd_pool: too many pixels");
   const long long tiles16 = (long long)N * ((H + 15) / 16) * ((W + kTW - 1) / kTW);
-  if (tiles16 < device_cus()) {
+  ConvArgs a;
+  a.W = W; a.Cin = Cin; a.Cout = Cout;
+  if (tiles16 < device_cus() || !tile_rows_fit(a)) {
     // layers the tile loop does not take: the convolution, then the pool
     if (int r = shy_nn_conv_fwd(x, w, bias, res, y_bf16, nullptr, N, H, W, Cin, Cout, 9, relu,
                                 stream))
       return r;
     return shy_nn_pool2(y_bf16, pool_y, N, H, W, Cout, 0, stream);
   }
-  ConvArgs a;
   a.x = (const __bf16*)x;
   a.w = (const __bf16*)w;
   a.bias = bias;
