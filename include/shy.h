@@ -126,8 +126,10 @@ typedef struct shy_terrain_desc {
    walk_grid   0: one lane per drop; > 0: a persistent grid of that many blocks
                walking the wave's drops grid-stride
    tile        cascade/blend stencil tile: 0 = 32x8, 1 = 64x4, 2 = 16x16 cells
-   With the default walk_block (256) and walk_grid (0), cycles of at most 4096
-   drops run one wave per drop instead of one lane per drop. */
+   With the default walk_block (256) and walk_grid (0), cycles of at most 2560
+   drops (6144 on maps of up to 65536 cells) run one wave per drop instead of
+   one lane per drop, and cycles of at most 16384 (32768) drops use blocks of
+   64 (128) threads. */
 typedef struct shy_tuning {
   int walk_block;
   int walk_grid;

@@ -159,20 +159,37 @@ bool ordered(const shy_ctx* c) {
 }
 constexpr int kReplayBlock = 256;
 // Drops (with padding) up to which a cycle runs one wave per drop
-// (walk_solo_kernel), and the map sides it takes (its window needs unit steps
-// to move a position by at most two cells).  A cycle, one wave per drop
-// against one lane per drop and the partition: 128^2 with 512 drops 104
-// against 260 us; 256^2 with 1024 228 / 634, with 4096 280 / 544; 512^2 with
-// 512 238 / 679, with 4096 572 / 666, with 6144 726 / 655; 1024^2 with 1024
-// 286 / 759, with 4096 634 / 782, with 6144 885 / 796.
-// A launch shape or drop order that the caller asked for is one of the walk
-// with a lane per drop, and keeps that walk.
-constexpr int kSoloMaxDrops = 4096;
+// (walk_solo_kernel) on maps of up to / more than kSoloSmallCells cells (whose
+// drops soon leave a small map, so their waves end early), and the map sides it
+// takes (its window needs unit steps to move a position by at most two cells).
+// A cycle in us, one wave per drop / one lane per drop and the partition:
+// 128^2 with 1024 drops 103 / 214; 192^2 with 4096 249 / 336; 256^2 with 1024
+// 245 / 459, 4096 314 / 409, 6144 360 / 405, 8192 397 / 399; 384^2 with 2048
+// 376 / 467, 3072 486 / 465; 512^2 with 1024 258 / 478, 2048 367 / 480, 3072
+// 482 / 481, 4096 606 / 484; 1024^2 with 2048 392 / 524, 3072 507 / 528, 4096
+// 635 / 536.  A launch shape or drop order that the caller asked for is one of
+// the walk with a lane per drop, and keeps that walk.
+constexpr int kSoloMaxDropsSmall = 6144, kSoloMaxDrops = 2560;
+constexpr size_t kSoloSmallCells = 65536;
 constexpr int kSoloMaxSide = 1 << 22;
 constexpr int kWalkBlock = 256;  // default threads per block of the walk
 
+// Threads per walk block, which are a partition block's drops too: unless the
+// caller asked for a shape, the width that gives every CU one block where a
+// cycle has fewer drops than 256 CUs x 256.  The partition's chain of rounds is as
+// long as a block is wide, and waves that share a CU share its vector cache,
+// where the replay's gathers evict each other's lines.  701 x 1103 x 9973 drops,
+// us with 256 / 64 threads: walk 314 / 304, partition 179 / 89, replay 141 /
+// 62.  With 64 / 128 / 256 (and the replay's blocks at 256): cycles of 24000
+// drops on 1024^2 818 / 815 / 872, 32768 872 / 872 / 917, 48000 1007 / 1030 /
+// 1016, 65536 1136 / 1144 / 1123.
+int walk_block(const shy_ctx* c) {
+  if (c->tune.walk_block != kWalkBlock || c->tune.walk_grid != 0) return c->tune.walk_block;
+  return c->total_drops <= 64 * 256 ? 64 : c->total_drops <= 128 * 256 ? 128 : kWalkBlock;
+}
 bool solo_cycle(const shy_ctx* c) {
-  if (c->total_drops < 1 || c->total_drops > kSoloMaxDrops) return false;
+  const int most = c->n <= kSoloSmallCells ? kSoloMaxDropsSmall : kSoloMaxDrops;
+  if (c->total_drops < 1 || c->total_drops > most) return false;
   if (c->tune.walk_block != kWalkBlock || c->tune.walk_grid != 0 || c->drop_order > 0) return false;
   for (const Terrain& t : c->ter)
     if (t.nx > kSoloMaxSide || t.ny > kSoloMaxSide) return false;
@@ -404,7 +421,7 @@ int ensure_wave(shy_ctx* c) {
   // persistent grid), blocks inside one terrain (one terrain, or a block
   // size dividing the padded drop ranges), every terrain's tiles in its LDS
   // and count matrices of modest size.
-  const int bs = c->tune.walk_block;
+  const int bs = walk_block(c);
   int nb = 0, window = 0;
   const bool fit = c->ter.size() == 1 || kDropAlign % bs == 0;
   const bool walk_counts = c->total_drops > 0 && c->tune.walk_grid == 0 && fit &&
@@ -627,7 +644,7 @@ int launch_stencil(shy_ctx* c, int p) {
 // commit replay.  ensure_wave(c) must have sized the wave buffers.
 int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
   WaveArgs w = wave_args(c, p);
-  const int bs = c->tune.walk_block;
+  const int bs = walk_block(c);
   const int need = (c->total_drops + bs - 1) / bs;
   const int grid = c->tune.walk_grid > 0 ? std::min(c->tune.walk_grid, need) : need;
   const size_t n = c->n;
@@ -746,11 +763,12 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
   HIPCHK(c, hipGetLastError());
   if (ev) HIPCHK(c, hipEventRecord(ev[2], c->stream));
   if (walk) {
-    const unsigned nb = (unsigned)((c->total_drops + kReplayBlock - 1) / kReplayBlock);
+    const int rbs = std::min(bs, kReplayBlock);
+    const unsigned nb = (unsigned)((c->total_drops + rbs - 1) / rbs);
     if (root)
-      replay_kernel<true><<<nb, kReplayBlock, 0, c->stream>>>(w);
+      replay_kernel<true><<<nb, rbs, 0, c->stream>>>(w);
     else
-      replay_kernel<false><<<nb, kReplayBlock, 0, c->stream>>>(w);
+      replay_kernel<false><<<nb, rbs, 0, c->stream>>>(w);
     HIPCHK(c, hipGetLastError());
   }
   if (ev) HIPCHK(c, hipEventRecord(ev[3], c->stream));

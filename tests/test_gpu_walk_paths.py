@@ -90,8 +90,10 @@ def test_flat_cells(shy, orc, block):
     (1, 1, 64, dict()),                        # every step leaves the map
     (2, 300, 65, dict()),                      # windows clamped on both sides of an axis
     (64, 64, 256, dict()),
-    (130, 67, 4096, dict()),                   # the most drops of one wave each
-    (130, 67, 4097, dict()),                   # the first that are not
+    (130, 67, 6144, dict()),                   # the most drops of one wave each
+    (130, 67, 6145, dict()),                   # the first that are not
+    (300, 220, 2560, dict()),                  # the same on a map of over 65536 cells
+    (300, 220, 2561, dict()),
     (96, 80, 200, dict(maxAge=0.0)),           # one step
     (96, 80, 200, dict(maxAge=62.0)),          # 63 steps: a batch less one
     (96, 80, 200, dict(maxAge=63.0)),          # 64: a whole batch
@@ -119,8 +121,8 @@ def test_few_and_many_drops_alternate(shy, orc):
     w = shy.World(n, n, seed=seed)
     w.upload("height", h)
     P = orc.Params.default()
-    for c, (drops, graph) in enumerate([(300, False), (6000, False), (300, True), (300, True),
-                                        (5000, True), (5000, True), (128, False)]):
+    for c, (drops, graph) in enumerate([(300, False), (7000, False), (300, True), (300, True),
+                                        (6200, True), (6200, True), (128, False)]):
         w.erode_cycles(1, drops, graph=graph)
         orc.wave_cycle(h, d, mx, my, root, erfd, P, seed, c, drops)
         for name, ref in (("height", h), ("discharge", d), ("momentumx", mx), ("momentumy", my)):
@@ -159,9 +161,9 @@ def test_few_drops_ensemble(shy, orc):
 
 
 @pytest.mark.parametrize("nx,ny,drops,kw", [
-    (64, 64, 5000, dict()),                   # every step in one tile: all parts are its
-    (70, 64, 4200, dict(maxAge=3.0)),         # two tiles, fewer entries than one part's least
-    (200, 136, 5000, dict(maxAge=120.0)),     # tiles of one part beside tiles of several
+    (64, 64, 6200, dict()),                   # every step in one tile: all parts are its
+    (70, 64, 6200, dict(maxAge=3.0)),         # two tiles, fewer entries than one part's least
+    (200, 136, 6200, dict(maxAge=120.0)),     # tiles of one part beside tiles of several
     (4400, 1000, 4500, dict(maxAge=30.0)),    # more tiles than the block listing them has threads
 ])
 def test_tile_parts(shy, orc, nx, ny, drops, kw):
@@ -171,3 +173,10 @@ def test_tile_parts(shy, orc, nx, ny, drops, kw):
     # valleys, so that some tiles hold most of the steps
     h = (0.5 + 2e-4 * (np.abs(x % 97 - 48) + np.abs(y % 89 - 44))).astype(np.float32)
     check_cycles(shy, orc, h, drops, 2, kw)
+
+
+@pytest.mark.parametrize("drops", [16384, 16385, 32768, 32769])
+def test_walk_block_widths(shy, orc, drops):
+    """Blocks of 64 threads up to 16384 drops, of 128 up to 32768, then 256."""
+    h = orc.fbm(8, 200, 144)
+    check_cycles(shy, orc, h, drops, 2, dict(maxAge=60.0))
