@@ -157,7 +157,21 @@ constexpr int kOrderMinDrops = 262144;
 bool ordered(const shy_ctx* c) {
   return c->drop_order < 0 ? c->total_drops >= kOrderMinDrops : c->drop_order != 0;
 }
-constexpr int kReplayBlock = 256;
+// Unused LDS of a block of the walk in drop order, so that a CU holds eight
+// waves: the lanes of a wave read neighbouring records, and the waves of more
+// blocks evict them from its vector cache.  us with as many blocks of 256 threads
+// as the registers hold / 3 / 2 per CU: 64 maps of 512^2 x 16384 drops 6360 /
+// 5270 / 5300, 2048^2 x 262144 1297 / 1415 / 1174, 4096^2 x 524288 3430 / 3380 /
+// 3230.  Without the order the waves share nothing (2048^2 x 196608 1718 / 1717 /
+// 1750).
+constexpr int kWalkLds = 56 * 1024;
+// The replay's blocks are single waves, three of which take a CU's LDS (unused):
+// the gathers of more waves evict each other's lines from its vector cache.
+// us with as many waves as the registers hold / 4 / 3 / 2 / 1 per CU: 65536 drops
+// on 1024^2 200 / 254 / 186 / 186 / 243, 262144 on 2048^2 796 / 775 / 707 / 706 /
+// 934; one or two waves per CU take 65 and 92 for 16384 and 32768 drops.
+constexpr int kReplayBlock = 64;
+constexpr int kReplayLds = 52 * 1024;
 // Drops (with padding) up to which a cycle runs one wave per drop
 // (walk_solo_kernel) on maps of up to / more than kSoloSmallCells cells (whose
 // drops soon leave a small map, so their waves end early), and the map sides it
@@ -688,10 +702,11 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
     // the record prefetch pays where every drop runs at once (the walk is
     // bound by its chain's latency): the same waves the drop order leaves off
     const bool pf = !ordered(c);
+    const int lds = pf ? 0 : kWalkLds;
     if (c->walk_counts)
-      (pf ? walk_kernel<true, true> : walk_kernel<true, false>)<<<grid, bs, 0, c->stream>>>(w);
+      (pf ? walk_kernel<true, true> : walk_kernel<true, false>)<<<grid, bs, lds, c->stream>>>(w);
     else
-      (pf ? walk_kernel<false, true> : walk_kernel<false, false>)<<<grid, bs, 0, c->stream>>>(w);
+      (pf ? walk_kernel<false, true> : walk_kernel<false, false>)<<<grid, bs, lds, c->stream>>>(w);
     HIPCHK(c, hipGetLastError());
     c->dlog_valid = true;
   }
@@ -763,12 +778,11 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
   HIPCHK(c, hipGetLastError());
   if (ev) HIPCHK(c, hipEventRecord(ev[2], c->stream));
   if (walk) {
-    const int rbs = std::min(bs, kReplayBlock);
-    const unsigned nb = (unsigned)((c->total_drops + rbs - 1) / rbs);
+    const unsigned nb = (unsigned)((c->total_drops + kReplayBlock - 1) / kReplayBlock);
     if (root)
-      replay_kernel<true><<<nb, rbs, 0, c->stream>>>(w);
+      replay_kernel<true><<<nb, kReplayBlock, kReplayLds, c->stream>>>(w);
     else
-      replay_kernel<false><<<nb, rbs, 0, c->stream>>>(w);
+      replay_kernel<false><<<nb, kReplayBlock, kReplayLds, c->stream>>>(w);
     HIPCHK(c, hipGetLastError());
   }
   if (ev) HIPCHK(c, hipEventRecord(ev[3], c->stream));
