@@ -320,7 +320,7 @@ int shy_get_tuning(const shy_ctx* ctx, shy_tuning* t);
    cycle assigns drops to walk threads by the position of their spawn cell,
    so that each XCD walks drops of one region and consecutive blocks walk
    neighbouring drops; on = 0: thread g walks drop g; on = -1 (the default):
-   ordered when a cycle has at least 262144 drops (more walk threads than
+   ordered when a cycle has at least 40960 drops (three and more waves per
    the GPU runs at once, where the order shortens the walk), else not.
    Results are bit-identical either way. */
 int shy_set_drop_order(shy_ctx* ctx, int on);

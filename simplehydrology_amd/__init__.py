@@ -508,7 +508,7 @@ class World:
 
     def set_drop_order(self, on):
         """Spatial drop order of the count walk: True, False or None (automatic,
-        the default: on from 262144 drops per cycle); bit-identical results."""
+        the default: on from 40960 drops per cycle); bit-identical results."""
         _check(self._ctx, lib().shy_set_drop_order(self._ctx, -1 if on is None else int(bool(on))))
 
     def tuning(self) -> dict:

@@ -110,10 +110,13 @@ struct shy_ctx {
   int32_t* scnt = nullptr;  // [cell] its step counts then, zero between cycles
   int4* dlog = nullptr;  // [drop] how each walk ended
   bool dlog_valid = false;  // dlog holds a cycle of the current wave geometry
-  int32_t* dperm = nullptr;  // [drop] the terrain's drop each walk thread takes (order_kernel)
+  int32_t* dperm = nullptr;  // [drop] the terrain's drop each walk thread takes (order_place_kernel)
+  uint32_t* okey = nullptr;  // [drop] its bin and rank (order_rank_kernel)
+  int32_t* ocnt = nullptr;   // [chunk][kOrderBins] drops per bin
+  int ocnt_chunks = 0;       // chunks ocnt holds
   long long pack_recs = 0;   // packed walk records over all terrains (pack_records)
   int drop_order = -1;       // assign drops to walk threads by spawn position: 1, 0, -1 auto
-  int order_chunks = 0;      // blocks of order_kernel
+  int order_chunks = 0;      // chunks of the drop order
   int32_t* wsteps = nullptr;  // [drop] steps of each walk
   float4* pack = nullptr;  // per cell, 2 x float4: the count walk's record
   size_t dlog_cap = 0;
@@ -149,10 +152,13 @@ constexpr int kWaveDrops = 64;  // drop ranges are padded to whole wave64s
 // drop ranges of an ensemble are padded to 256 drops: walk blocks of 64, 128
 // or 256 threads then never span terrains
 constexpr int kDropAlign = 256;
-// drops from which the automatic drop order is on: more walk threads than
-// the GPU runs at once, so the walk's blocks run in sequence and neighbouring
-// blocks share the L2 when their drops start near each other
-constexpr int kOrderMinDrops = 262144;
+// drops from which the automatic drop order is on: three and more waves per
+// CU, whose lanes' records share lines when their drops start near each other,
+// and beyond 65536 walk blocks that run in sequence.  Cycles in us without /
+// with the order: 32768 drops on 724^2 767 / 765; on 1024^2 40960 971 / 950,
+// 49152 1028 / 991, 65536 1175 / 1092; 98304 on 1448^2 2072 / 1658; on 2048^2
+// 131072 2839 / 2218, 262144 5560 / 4090
+constexpr int kOrderMinDrops = 40960;
 
 bool ordered(const shy_ctx* c) {
   return c->drop_order < 0 ? c->total_drops >= kOrderMinDrops : c->drop_order != 0;
@@ -462,6 +468,15 @@ int ensure_wave(shy_ctx* c) {
   c->part_window = window;
   c->part_maxw = 0;
   for (const Terrain& t : c->ter) c->part_maxw = std::max(c->part_maxw, t.part_dwidth);
+  if (c->order_chunks > c->ocnt_chunks) {
+    drop_graph(c);
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (c->ocnt) hipFree(c->ocnt);
+    c->ocnt = nullptr;
+    c->ocnt_chunks = 0;
+    HIPCHK(c, hipMalloc(&c->ocnt, (size_t)c->order_chunks * kOrderBins * sizeof(int32_t)));
+    c->ocnt_chunks = c->order_chunks;
+  }
   const size_t hist_need = entries + 1;
   const int qstride =
       ((rows + kReplayDepth - 1) / kReplayDepth * kReplayDepth + 31) / 32 * 32;
@@ -562,13 +577,16 @@ int ensure_wave(shy_ctx* c) {
     if (c->dlog) hipFree(c->dlog);
     if (c->wsteps) hipFree(c->wsteps);
     if (c->dperm) hipFree(c->dperm);
+    if (c->okey) hipFree(c->okey);
     c->dlog = nullptr;
     c->wsteps = nullptr;
     c->dperm = nullptr;
+    c->okey = nullptr;
     c->dlog_cap = 0;
     HIPCHK(c, hipMalloc(&c->dlog, need_d * sizeof(int4)));
     HIPCHK(c, hipMalloc(&c->wsteps, need_d * sizeof(int32_t)));
     HIPCHK(c, hipMalloc(&c->dperm, need_d * sizeof(int32_t)));
+    HIPCHK(c, hipMalloc(&c->okey, need_d * sizeof(uint32_t)));
     c->dlog_cap = need_d;
   }
   if (hist_need > c->hist_cap) {
@@ -666,14 +684,20 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
   const bool walk = c->total_drops > 0;
   if (walk) {
     const size_t nrec = (size_t)c->pack_recs;
+    const bool order = ordered(c) && !c->solo;
     pack_kernel<<<(unsigned)((nrec + 255) / 256), 256, 0, c->stream>>>(c->d_ter, nter, nrec,
                                                                         c->h[p], c->fld, c->pack,
                                                                         c->gflag,
                                                                         c->solo ? c->dh : nullptr,
-                                                                        c->trk, n);
-    if (ordered(c) && !c->solo)
-      order_kernel<<<c->order_chunks, 1024, 0, c->stream>>>(c->d_ter, nter, c->total_drops, bs, c->state,
-                                                 c->dperm);
+                                                                        c->trk, n, c->ocnt,
+                                                                        order ? (size_t)c->order_chunks * kOrderBins : 0);
+    if (order) {
+      const unsigned nb = (unsigned)c->order_chunks * (kOrderChunk / 1024);
+      order_rank_kernel<<<nb, 1024, 0, c->stream>>>(c->d_ter, nter, c->total_drops, c->state,
+                                                    c->ocnt, c->okey);
+      order_place_kernel<<<nb, 1024, 0, c->stream>>>(c->d_ter, nter, c->total_drops, bs, c->ocnt,
+                                                     c->okey, c->dperm);
+    }
     HIPCHK(c, hipGetLastError());
   }
   if (ev) HIPCHK(c, hipEventRecord(ev[0], c->stream));
@@ -983,7 +1007,7 @@ int shy_destroy(shy_ctx* c) {
   void* ptrs[] = {c->h[0], c->h[1], c->fld, c->root, c->visit[0], c->visit[1], c->first,
                   c->sr, c->dh, c->trk, c->deposit, c->slog, c->strk, c->qb, c->ent, c->gflag,
                   c->vq, c->vt, c->scnt, c->rootp, c->tparts, c->tlist, c->tmulti, c->tcount,
-                  c->tsum, c->hist, c->hbsum, c->tstart, c->dlog, c->wsteps, c->dperm, c->tsteps, c->veg_px, c->veg_py, c->veg_alive, c->veg_cflag,
+                  c->tsum, c->hist, c->hbsum, c->tstart, c->dlog, c->wsteps, c->dperm, c->okey, c->ocnt, c->tsteps, c->veg_px, c->veg_py, c->veg_alive, c->veg_cflag,
                   c->veg_cx, c->veg_cy, c->veg_units, c->veg_st, c->veg_size, c->pack, c->d_ter, c->state, c->erf_a, c->part, c->perms, c->trace_buf,
                   c->trace_n, c->drop_buf};
   for (void* q : ptrs)

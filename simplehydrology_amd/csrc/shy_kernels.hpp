@@ -6,7 +6,8 @@
 //  pack_kernel           one 32-byte record per cell of what a walk step reads
 //                        there, the cell's normal precomputed, in 2x2 cell
 //                        blocks (four records per 128-byte line)
-//  order_kernel          (many drops) which drop each walk thread takes
+//  order_rank_kernel, order_place_kernel  (many drops) which drop each walk
+//                        thread takes
 //  walk_kernel           one drop per lane walks its trajectory; for every
 //                        step it logs, coalesced as [step][drop], 16 bytes
 //                        {start cell, c_eq} + {tracks} of what the
@@ -163,7 +164,7 @@ struct WaveArgs {
   int vt_rows;
   int32_t* steps;     // [drop] steps of the walk (the log rows it filled)
   int32_t* hist;      // per-terrain [tile][walk block] step counts, when the walk counts them
-  const int32_t* __restrict__ perm;  // [drop] the terrain's drop a thread walks (order_kernel), or null
+  const int32_t* __restrict__ perm;  // [drop] the terrain's drop a thread walks (order_place_kernel), or null
   const float4* __restrict__ pack;  // per cell 32 B: what one walk step reads (pack_kernel), 2x2 cell blocks (pack_rec)
   int32_t* deposit;
   uint8_t* visit;
@@ -688,8 +689,9 @@ __device__ int walk_short(const WalkArgs& a, const float2* __restrict__ vt, int 
 __global__ void pack_kernel(const Terrain* __restrict__ ter, int nter, size_t nrec,
                             const float* __restrict__ h, const float4* __restrict__ fld,
                             float4* pack, int* gflag, int32_t* clear_dh, long long* clear_trk,
-                            size_t clear_n) {
+                            size_t clear_n, int32_t* clear_order, size_t order_n) {
   const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (size_t j = g; j < order_n; j += (size_t)gridDim.x * blockDim.x) clear_order[j] = 0;
   if (g >= nrec) return;
   const int t = find_terrain(nter, (long long)g, [&](int q) { return ter[q].pack_off; });
   const Terrain& T = ter[t];
@@ -1515,7 +1517,7 @@ __device__ inline void block_scan_runs(const int* v, int* out, int m, int* wsum)
 // starting near each other on one XCD share its L2.  Drops are independent
 // within a cycle, every log is indexed by the thread that walked it and
 // every per-cell result is an integer sum, so any assignment of drops to
-// threads gives the same results.  order_kernel assigns them spatially, per
+// threads gives the same results.  order_rank_kernel and order_place_kernel assign them spatially, per
 // chunk of kOrderChunk threads of a terrain (one block each): the chunk's
 // drops sorted by the Morton code of their spawn cell on a grid of at most
 // 64 x 64 bins, and the sorted list laid onto the chunk's walk blocks class
@@ -1552,43 +1554,74 @@ __device__ inline int morton_bin(uint32_t cid, int ny, int sx, int sy) {
   return (int)m;
 }
 
-// One block of 1024 threads per chunk; Terrain::order_first numbers the
-// chunks of the terrains.  The second pass recomputes each drop's bin (a
-// global round trip per drop costs more at one block per CU).
-__global__ void __launch_bounds__(1024) order_kernel(const Terrain* __restrict__ ter, int nter,
-                                                     int total_drops, int bs,
-                                                     const DeviceState* __restrict__ state,
-                                                     int32_t* perm) {
-  __shared__ int cnt[4096];
-  __shared__ int off[4096];
-  __shared__ int wsum[16];
-  const int t = find_terrain(nter, (long long)blockIdx.x,
-                             [&](int q) { return (long long)ter[q].order_first; });
-  const Terrain& T = ter[t];
-  const int end = t + 1 < nter ? ter[t + 1].drop_off : total_drops;
+// Two passes over the drops, 1024 per block: each takes a rank in its bin of
+// its chunk (kOrderBins counters, cleared by pack_kernel), then, with the
+// counters scanned by every block for itself, its position.  (One block per
+// chunk sorting all of its drops in LDS took 100 us a chunk; these take 12 us
+// for one chunk and 18 for four.)
+// Terrain::order_first numbers the chunks of the terrains.
+constexpr int kOrderBins = 4096;
+
+// the terrain and chunk of a block's 1024 threads
+struct OrderBlock {
+  int t, chunk;  // chunk over all terrains
+  int c0, c1;    // the chunk's threads of the terrain
+  int i;         // this thread
+};
+
+__device__ inline OrderBlock order_block(const Terrain* __restrict__ ter, int nter,
+                                         int total_drops) {
+  constexpr int kBlocks = kOrderChunk / 1024;
+  OrderBlock o;
+  o.chunk = (int)blockIdx.x / kBlocks;
+  o.t = find_terrain(nter, (long long)o.chunk, [&](int q) { return (long long)ter[q].order_first; });
+  const Terrain& T = ter[o.t];
+  const int end = o.t + 1 < nter ? ter[o.t + 1].drop_off : total_drops;
   const int P = end - T.drop_off;  // the terrain's padded drops
-  const int c0 = ((int)blockIdx.x - T.order_first) * kOrderChunk;
-  const int c1 = c0 + kOrderChunk < P ? c0 + kOrderChunk : P;
-  const int r1 = c1 < T.drops ? c1 : T.drops;  // real drops of the chunk: [c0, r1)
-  const int nbl = (c1 - c0) / bs, b0 = (T.drop_off + c0) / bs;
-  const uint32_t ncell = (uint32_t)T.nx * (uint32_t)T.ny;
-  const uint64_t key = cycle_key(T.seed, T.id, state->cycle);
+  o.c0 = (o.chunk - T.order_first) * kOrderChunk;
+  o.c1 = o.c0 + kOrderChunk < P ? o.c0 + kOrderChunk : P;
+  o.i = o.c0 + ((int)blockIdx.x % kBlocks) * 1024 + (int)threadIdx.x;
+  return o;
+}
+
+// key[g] = bin << 16 | rank of real drop g - drop_off
+__global__ void __launch_bounds__(1024) order_rank_kernel(const Terrain* __restrict__ ter, int nter,
+                                                          int total_drops,
+                                                          const DeviceState* __restrict__ state,
+                                                          int32_t* cnt, uint32_t* key) {
+  const OrderBlock o = order_block(ter, nter, total_drops);
+  const Terrain& T = ter[o.t];
+  if (o.i >= o.c1 || o.i >= T.drops) return;
   int sx = 0, sy = 0;
   while (((T.nx - 1) >> sx) >= 64) ++sx;
   while (((T.ny - 1) >> sy) >= 64) ++sy;
-  for (int b = threadIdx.x; b < 4096; b += 1024) cnt[b] = 0;
+  const uint64_t ck = cycle_key(T.seed, T.id, state->cycle);
+  const int bin = morton_bin(spawn_cell(ck, (uint32_t)o.i, (uint32_t)T.nx * (uint32_t)T.ny), T.ny,
+                             sx, sy);
+  const int r = atomicAdd(&cnt[(size_t)o.chunk * kOrderBins + bin], 1);
+  key[T.drop_off + o.i] = (uint32_t)bin << 16 | (uint32_t)r;
+}
+
+__global__ void __launch_bounds__(1024) order_place_kernel(const Terrain* __restrict__ ter,
+                                                           int nter, int total_drops, int bs,
+                                                           const int32_t* __restrict__ cnt,
+                                                           const uint32_t* __restrict__ key,
+                                                           int32_t* perm) {
+  __shared__ int off[kOrderBins];
+  __shared__ int wsum[16];
+  const OrderBlock o = order_block(ter, nter, total_drops);
+  if (o.i - (int)threadIdx.x >= o.c1) return;  // uniform over the block
+  const Terrain& T = ter[o.t];
+  block_scan_runs(cnt + (size_t)o.chunk * kOrderBins, off, kOrderBins, wsum);
   __syncthreads();
-  for (int i = c0 + (int)threadIdx.x; i < r1; i += 1024)
-    atomicAdd(&cnt[morton_bin(spawn_cell(key, (uint32_t)i, ncell), T.ny, sx, sy)], 1);
-  __syncthreads();
-  block_scan_runs(cnt, off, 4096, wsum);
-  __syncthreads();
-  for (int i = c0 + (int)threadIdx.x; i < r1; i += 1024) {
-    const int s = atomicAdd(&off[morton_bin(spawn_cell(key, (uint32_t)i, ncell), T.ny, sx, sy)], 1);
-    perm[T.drop_off + c0 + order_position(s, bs, nbl, b0)] = i;
+  if (o.i >= o.c1) return;
+  const int nbl = (o.c1 - o.c0) / bs, b0 = (T.drop_off + o.c0) / bs;
+  int s = o.i - o.c0;  // a padding thread keeps its place behind the real drops
+  if (o.i < T.drops) {
+    const uint32_t kk = key[T.drop_off + o.i];
+    s = off[kk >> 16] + (int)(kk & 0xffffu);
   }
-  for (int s = (r1 > c0 ? r1 : c0) - c0 + (int)threadIdx.x; s < c1 - c0; s += 1024)
-    perm[T.drop_off + c0 + order_position(s, bs, nbl, b0)] = c0 + s;
+  perm[T.drop_off + o.c0 + order_position(s, bs, nbl, b0)] = o.i;
 }
 
 // The scatter with its writes grouped: each round of RS slots is ranked per

@@ -180,3 +180,25 @@ def test_walk_block_widths(shy, orc, drops):
     """Blocks of 64 threads up to 16384 drops, of 128 up to 32768, then 256."""
     h = orc.fbm(8, 200, 144)
     check_cycles(shy, orc, h, drops, 2, dict(maxAge=60.0))
+
+
+@pytest.mark.parametrize("nx,ny,drops", [
+    (60, 70, 1), (60, 70, 1023), (60, 70, 1025),  # blocks of 1024 drops
+    (300, 9, 65536), (90, 130, 65537),            # one chunk and one drop more
+    (1, 4097, 5000),                              # all bins along one axis
+])
+def test_drop_order_chunks(shy, nx, ny, drops):
+    """The drop order is a permutation: no field and no count depends on it."""
+    got = []
+    for on in (True, False):
+        w = shy.World(nx, ny, seed=4, params=shy.Params(maxAge=40.0))
+        w.upload("height", plane(nx, ny))
+        w.set_drop_order(on)
+        say("order", on, nx, ny, drops)
+        w.erode(drops)
+        w.erode_cycles(4, drops)
+        got.append([bits(w.field(f)) for f in ("height", "discharge", "momentumx", "momentumy")] +
+                   [w.stats()])
+        w.close()
+    assert all(np.array_equal(a, b) for a, b in zip(got[0][:4], got[1][:4]))
+    assert got[0][4] == got[1][4]
