@@ -361,9 +361,6 @@ constexpr int kPartMaxBlocks = 512;
 // cells).
 constexpr int kTileParts = 512;
 constexpr int kPartMin = 16384;
-// partition blocks up to which each takes a CU's whole LDS (the scatter's
-// rounds of 8192 entries): no more blocks than CUs
-constexpr int kBigRoundBlocks = 256;
 
 // The partition geometry: per terrain its tiles, its blocks of dwidth drops
 // (dwidth = walk_block when the walk counts, else enough drops for at most
@@ -762,18 +759,17 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
     scan_top_kernel<<<1, kScanBlock, 0, c->stream>>>(c->hbsum, nbh);
     scan_apply_kernel<<<nbh, kScanBlock, 0, c->stream>>>(c->hist, c->hbsum, nh);
     const int mw = c->part_maxw;
-    if (c->part_window <= 1024 && nb <= kBigRoundBlocks) {
-      if (mw <= scatter_lds_drops<1024, 8192>())
+    // rounds of 8192 slots fill a CU's LDS with one block; two blocks per CU with
+    // rounds of 4096 write shorter runs (64 maps of 512^2 x 16384 drops 4590 -> 4490
+    // us and the sums that read the runs 2890 -> 2730, 2048^2 x 262144 1060 -> 980
+    // and 590 -> 570), so they are left to terrains of more than 1024 tiles
+    if (c->part_window <= 1024) {
+      if (mw <= kScatterLdsDrops)
         part_scatter_staged_kernel<1024, 8192, true><<<nb, 1024, 0, c->stream>>>(pa);
       else
         part_scatter_staged_kernel<1024, 8192, false><<<nb, 1024, 0, c->stream>>>(pa);
-    } else if (c->part_window <= 1024) {
-      if (mw <= scatter_lds_drops<1024, 4096>())
-        part_scatter_staged_kernel<1024, 4096, true><<<nb, 1024, 0, c->stream>>>(pa);
-      else
-        part_scatter_staged_kernel<1024, 4096, false><<<nb, 1024, 0, c->stream>>>(pa);
     } else if (c->part_window <= 4096) {
-      if (mw <= scatter_lds_drops<4096, 4096>())
+      if (mw <= kScatterLdsDrops)
         part_scatter_staged_kernel<4096, 4096, true><<<nb, 1024, 0, c->stream>>>(pa);
       else
         part_scatter_staged_kernel<4096, 4096, false><<<nb, 1024, 0, c->stream>>>(pa);

@@ -1628,24 +1628,18 @@ __global__ void __launch_bounds__(1024) order_place_kernel(const Terrain* __rest
 // tile in LDS, staged in tile order and written out so that the round's
 // entries of one tile go to consecutive addresses.  LDS holds the block's
 // terrain's tiles (at most MAXT, which the host checks) and RS entries.
-template <int MAXT, int RS>
-constexpr int scatter_lds_drops() {
-  return (MAXT <= 1024 && RS <= 4096) ? 1008 : 4096;
-}
+constexpr int kScatterLdsDrops = 4096;
 
 // LDSW: the block's step counts are staged in LDS (every block width at most
-// scatter_lds_drops, which the host checks); else they are read from memory.
+// kScatterLdsDrops, which the host checks); else they are read from memory.
 // The choice is made at compile time: a pointer that may address either
 // makes every read of it a flat access, whose wait covers all memory loads
 // in flight, and so would serialise the next round's loads.
 template <int MAXT, int RS, bool LDSW>
-// (rounds of 4096: two blocks of 1024 threads per CU, at most 64 VGPRs;
-// rounds of 8192 fill the LDS of a CU with one block)
-__global__ void __launch_bounds__(1024, RS <= 4096 ? 8 : 4) part_scatter_staged_kernel(PartArgs a) {
+// (the LDS of a CU holds one block)
+__global__ void __launch_bounds__(1024) part_scatter_staged_kernel(PartArgs a) {
   constexpr int PER = RS / 1024;
-  // drops whose step counts the block keeps in LDS: with 1024 tiles and 4096
-  // staged entries the block stays within 80 KB, two blocks per CU
-  constexpr int kMaxW = LDSW ? scatter_lds_drops<MAXT, RS>() : 1;
+  constexpr int kMaxW = LDSW ? kScatterLdsDrops : 1;
   __shared__ int cur[MAXT];  // next entry of each tile of the block's terrain
   __shared__ int cnt[MAXT];  // the round's entries per tile
   __shared__ int off[MAXT];  // their exclusive offsets in the stage
