@@ -97,6 +97,13 @@ int shy_nn_bias_grad(const void* g, float* db, float* part, int part_rows, int P
 int shy_nn_conv_wgrad_bias(const void* x, const void* g, float* dw, float* db, float* part,
                            int part_splits, float* bias_part, int bias_rows, int N, int H, int W,
                            int Cin, int Cout, int taps, void* stream);
+/* The same of a convolution of [up2(x_half), skip] along channels (C1 + C2),
+   read from the two tensors (shy_nn_conv_fwd_upcat's input).  H, W even; C1,
+   C2, Cout multiples of 32; part holds part_splits*Cout*9*(C1+C2) floats,
+   part_splits > 1. */
+int shy_nn_conv_wgrad_bias_upcat(const void* x_half, const void* skip, const void* g, float* dw,
+                                 float* db, float* part, int part_splits, int N, int H, int W,
+                                 int C1, int C2, int Cout, void* stream);
 int shy_nn_relu_bwd(const void* y, const void* g, void* out, size_t n, void* stream);
 /* 2x2 average pool (backward: x = dy, y = dx at full size) */
 int shy_nn_pool2(const void* x, void* y, int N, int H, int W, int C, int backward, void* stream);
@@ -104,6 +111,17 @@ int shy_nn_pool2(const void* x, void* y, int N, int H, int W, int C, int backwar
    y [N][2H][2W][Cy]; backward sums the 4 children back */
 int shy_nn_up2(const void* x, void* y, int N, int H, int W, int C, int Cy, int c_off,
                int backward, void* stream);
+/* shy_nn_up2's backward, zeroed where y [N][H][W][C] (what was upsampled) is
+   not positive; C, Cy, c_off multiples of 8 */
+int shy_nn_up2_bwd_relu(const void* gy, const void* y, void* gx, int N, int H, int W, int C, int Cy,
+                        int c_off, void* stream);
+/* out [N][H][W][C] = the backward of the 2x2 average pool (gp
+   [N][H/2][W/2][C]) plus channels [c_off, c_off+C) of gu [N][H][W][Cu], zeroed
+   where y is not positive: shy_nn_pool2, shy_nn_channels, shy_nn_add and
+   shy_nn_relu_bwd with the same roundings.  H, W even, C, Cu, c_off multiples
+   of 8 */
+int shy_nn_skip_bwd(const void* gp, const void* gu, const void* y, void* out, int N, int H, int W,
+                    int C, int Cu, int c_off, void* stream);
 /* dir 0: copy src [P][C] into channels [c_off, c_off+C) of dst [P][Cy];
    dir 1: the reverse */
 int shy_nn_channels(const void* src, void* dst, size_t P, int C, int Cy, int c_off, int dir,

@@ -911,7 +911,11 @@ constexpr int kWgBlocks = 512;
 constexpr int kWgXS = 32 + 8;  // halfwords per pixel of X; 16 pixels cover the banks evenly
 
 struct WgArgs {
+  // the input: x [N][H][W][Cin], or (C1 > 0) its channels below C1 from x
+  // [N][H/2][W/2][C1], read at (y/2, x/2), and the others from x2
   const __bf16* __restrict__ x;
+  const __bf16* __restrict__ x2;
+  int C1;
   const __bf16* __restrict__ g;
   float* part;  // [splits][Cout*K (+ Cout with bias)]
   int N, H, W, Cin, Cout, K;
@@ -944,6 +948,11 @@ __global__ void __launch_bounds__(256) wgrad_lds_kernel(WgArgs a) {
   const int t_end = min(a.tiles, t_begin + a.tiles_per_split);
   const int Cin = a.Cin, Cout = a.Cout;
   const bool bias = a.bias && ci0 == 0 && (wave & 1) == 0;  // uniform over the wave
+  // where this block's input channels lie
+  const int up = ci0 < a.C1 ? 1 : 0;
+  const __bf16* src = a.C1 > 0 && !up ? a.x2 : a.x;
+  const int srcH = a.H >> up, srcW = a.W >> up;
+  const int srcC = up ? a.C1 : Cin - a.C1, srcc = up ? ci0 : ci0 - a.C1;
   f32x4 acc[9][MTW], accb[MTW];
 #pragma unroll
   for (int m = 0; m < MTW; ++m) {
@@ -958,7 +967,7 @@ __global__ void __launch_bounds__(256) wgrad_lds_kernel(WgArgs a) {
     const int n = t / (a.tiles_x * a.tiles_y);
     const int x0 = tx * kWgTW, y0 = ty * kWgTH;
     const __bf16* gi = a.g + (size_t)n * a.H * a.W * Cout + cb;
-    const __bf16* xi = a.x + (size_t)n * a.H * a.W * Cin + ci0;
+    const __bf16* xi = src + (size_t)n * srcH * srcW * srcC + srcc;
     okg = okx = 0;
 #pragma unroll
     for (int j = 0; j < RG; ++j) {
@@ -974,7 +983,7 @@ __global__ void __launch_bounds__(256) wgrad_lds_kernel(WgArgs a) {
       const int gy = y0 + pix / kWgXW - 1, gx = x0 + pix % kWgXW - 1;
       const bool ok = v < kWgXPix * 4 && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W;
       okx |= ok ? 1u << j : 0u;
-      rx[j] = load8(xi + (ok ? ((size_t)gy * a.W + gx) * Cin : 0) + q * 8);
+      rx[j] = load8(xi + (ok ? ((size_t)(gy >> up) * srcW + (gx >> up)) * srcC : 0) + q * 8);
     }
   };
   auto lstore = [&]() {
@@ -1362,8 +1371,11 @@ __global__ void up2_fwd_v8_kernel(const __bf16* __restrict__ x, __bf16* y, int N
   store8(y + q * Cy + c_off + c, load8(x + ((size_t)(nn * H + yo / 2) * W + xo / 2) * C + c));
 }
 
-__global__ void up2_bwd_v8_kernel(const __bf16* __restrict__ gy, __bf16* gx, int N, int H, int W,
-                                  int C, int Cy, int c_off) {
+// gate (or null): the result is zeroed where it is not positive (ReLU's
+// backward on what was upsampled)
+__global__ void up2_bwd_v8_kernel(const __bf16* __restrict__ gy, __bf16* gx,
+                                  const __bf16* __restrict__ gate, int N, int H, int W, int C,
+                                  int Cy, int c_off) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int C8 = C / 8;
   if (i >= (size_t)N * H * W * C8) return;
@@ -1378,7 +1390,39 @@ __global__ void up2_bwd_v8_kernel(const __bf16* __restrict__ gy, __bf16* gx, int
 #pragma unroll
   for (int k = 0; k < 8; ++k)
     r[k] = (__bf16)((float)v0[k] + (float)v1[k] + (float)v2[k] + (float)v3[k]);
+  if (gate) {
+    const bf16x8 y = load8(gate + q * C + c);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) r[k] = (float)y[k] > 0.0f ? r[k] : (__bf16)0.0f;
+  }
   store8(gx + q * C + c, r);
+}
+
+// The gradient of an encoder stage's output y [N][H][W][C], before its ReLU:
+// the pooled path's gp [N][H/2][W/2][C] spread over 2x2, plus the decoder's
+// channels [c_off, c_off + C) of gu [N][H][W][Cu], zeroed where y is not
+// positive.  The roundings of the four passes it replaces (pool, channel
+// copy, sum, ReLU), which moved 2.6 times the bytes: memory bound, and at 16 x
+// 256^2 x 32 channels 46 us against 128.
+__global__ void skip_bwd_v8_kernel(const __bf16* __restrict__ gp, const __bf16* __restrict__ gu,
+                                   const __bf16* __restrict__ y, __bf16* out, int N, int H, int W,
+                                   int C, int Cu, int c_off) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int C8 = C / 8;
+  if (i >= (size_t)N * H * W * C8) return;
+  const int c = (int)(i % C8) * 8;
+  const size_t q = i / C8;
+  const int px = (int)(q % W), py = (int)((q / W) % H), nn = (int)(q / ((size_t)W * H));
+  const bf16x8 a = load8(gp + ((size_t)(nn * (H / 2) + py / 2) * (W / 2) + px / 2) * C + c);
+  const bf16x8 b = load8(gu + q * Cu + c_off + c), v = load8(y + q * C + c);
+  bf16x8 r;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const __bf16 p = (__bf16)(0.25f * (float)a[k]);
+    const __bf16 s = (__bf16)((float)p + (float)b[k]);
+    r[k] = (float)v[k] > 0.0f ? s : (__bf16)0.0f;
+  }
+  store8(out + q * C + c, r);
 }
 
 __global__ void channels_copy_v8_kernel(const __bf16* __restrict__ src, __bf16* dst, size_t P,
@@ -1759,10 +1803,13 @@ int shy_nn_flip_weights(const void* w, void* wf, int Cin, int Cout, int taps, vo
 
 // The weight gradient by wgrad_lds_kernel, and with db the bias gradient of
 // the same pass; part holds cap floats.
-static int wgrad_lds(const void* x, const void* g, float* dw, float* db, float* part, size_t cap,
-                     int N, int H, int W, int Cin, int Cout, hipStream_t s) {
+static int wgrad_lds(const void* x, const void* x2, int C1, const void* g, float* dw, float* db,
+                     float* part, size_t cap, int N, int H, int W, int Cin, int Cout,
+                     hipStream_t s) {
   WgArgs b;
   b.x = (const __bf16*)x;
+  b.x2 = (const __bf16*)x2;
+  b.C1 = C1;
   b.g = (const __bf16*)g;
   b.part = part;
   b.N = N; b.H = H; b.W = W; b.Cin = Cin; b.Cout = Cout; b.K = 9 * Cin;
@@ -1798,7 +1845,7 @@ int shy_nn_conv_wgrad(const void* x, const void* g, float* dw, float* part, int 
   if (Cin % 8 || Cout % 8 || (taps != 9 && taps != 1)) return nn_fail("conv_wgrad: channels must be multiples of 8");
   const long long P = (long long)N * H * W;
   if (taps == 9 && Cin % 32 == 0 && Cout % 32 == 0)
-    return wgrad_lds(x, g, dw, nullptr, part, (size_t)part_splits * Cout * 9 * Cin, N, H, W, Cin,
+    return wgrad_lds(x, nullptr, 0, g, dw, nullptr, part, (size_t)part_splits * Cout * 9 * Cin, N, H, W, Cin,
                      Cout, (hipStream_t)stream);
   int chunk = (int)((P + part_splits - 1) / part_splits);
 
@@ -1865,11 +1912,23 @@ int shy_nn_conv_wgrad_bias(const void* x, const void* g, float* dw, float* db, f
   if (x && g && dw && db && part && part_splits > 1 && taps == 9 && Cin > 0 && Cout > 0 &&
       Cout <= 1024 &&  // as shy_nn_bias_grad
       Cin % 32 == 0 && Cout % 32 == 0)
-    return wgrad_lds(x, g, dw, db, part, (size_t)part_splits * Cout * 9 * Cin, N, H, W, Cin, Cout,
-                     (hipStream_t)stream);
+    return wgrad_lds(x, nullptr, 0, g, dw, db, part, (size_t)part_splits * Cout * 9 * Cin, N, H, W,
+                     Cin, Cout, (hipStream_t)stream);
   if (int r = shy_nn_conv_wgrad(x, g, dw, part, part_splits, N, H, W, Cin, Cout, taps, stream))
     return r;
   return shy_nn_bias_grad(g, db, bias_part, bias_rows, N * H * W, Cout, stream);
+}
+
+int shy_nn_conv_wgrad_bias_upcat(const void* x_half, const void* skip, const void* g, float* dw,
+                                 float* db, float* part, int part_splits, int N, int H, int W,
+                                 int C1, int C2, int Cout, void* stream) {
+  if (!x_half || !skip || !g || !dw || !db || !part || part_splits < 2)
+    return nn_fail("conv_wgrad_bias_upcat: bad pointers, or fewer than two partials");
+  if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || C1 < 32 || C1 % 32 || C2 < 32 || C2 % 32 ||
+      Cout < 32 || Cout % 32 || Cout > 1024)
+    return nn_fail("conv_wgrad_bias_upcat: need H, W even and C1, C2, Cout multiples of 32");
+  return wgrad_lds(x_half, skip, C1, g, dw, db, part, (size_t)part_splits * Cout * 9 * (C1 + C2), N,
+                   H, W, C1 + C2, Cout, (hipStream_t)stream);
 }
 
 inline bool a16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -1913,7 +1972,7 @@ int shy_nn_up2(const void* x, void* y, int N, int H, int W, int C, int Cy, int c
         (const __bf16*)x, (__bf16*)y, N, H, W, C, Cy, c_off);
   else if (v8)
     up2_bwd_v8_kernel<<<blocks((size_t)N * H * W * C / 8), 256, 0, s>>>(
-        (const __bf16*)x, (__bf16*)y, N, H, W, C, Cy, c_off);
+        (const __bf16*)x, (__bf16*)y, nullptr, N, H, W, C, Cy, c_off);
   else if (!backward)
     up2_fwd_kernel<<<blocks((size_t)N * 4 * H * W * C), 256, 0, s>>>(
         (const __bf16*)x, (__bf16*)y, N, H, W, C, Cy, c_off);
@@ -1921,6 +1980,30 @@ int shy_nn_up2(const void* x, void* y, int N, int H, int W, int C, int Cy, int c
     up2_bwd_kernel<<<blocks((size_t)N * H * W * C), 256, 0, s>>>((const __bf16*)x, (__bf16*)y, N, H,
                                                                  W, C, Cy, c_off);
   return nn_check("up2");
+}
+
+int shy_nn_up2_bwd_relu(const void* gy, const void* y, void* gx, int N, int H, int W, int C, int Cy,
+                        int c_off, void* stream) {
+  if (!gy || !y || !gx) return nn_fail("up2_bwd_relu: bad pointers");
+  if (N < 1 || H < 1 || W < 1 || C < 8 || C % 8 || Cy % 8 || c_off % 8 || c_off < 0 ||
+      c_off + C > Cy || !a16(gy) || !a16(y) || !a16(gx))
+    return nn_fail("up2_bwd_relu: need channels in multiples of 8, inside the target, 16-byte "
+                   "aligned tensors");
+  up2_bwd_v8_kernel<<<blocks((size_t)N * H * W * C / 8), 256, 0, (hipStream_t)stream>>>(
+      (const __bf16*)gy, (__bf16*)gx, (const __bf16*)y, N, H, W, C, Cy, c_off);
+  return nn_check("up2_bwd_relu");
+}
+
+int shy_nn_skip_bwd(const void* gp, const void* gu, const void* y, void* out, int N, int H, int W,
+                    int C, int Cu, int c_off, void* stream) {
+  if (!gp || !gu || !y || !out) return nn_fail("skip_bwd: bad pointers");
+  if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || C < 8 || C % 8 || Cu % 8 || c_off % 8 ||
+      c_off < 0 || c_off + C > Cu || !a16(gp) || !a16(gu) || !a16(y) || !a16(out))
+    return nn_fail("skip_bwd: need H, W even, channels in multiples of 8, inside the source, "
+                   "16-byte aligned tensors");
+  skip_bwd_v8_kernel<<<blocks((size_t)N * H * W * C / 8), 256, 0, (hipStream_t)stream>>>(
+      (const __bf16*)gp, (const __bf16*)gu, (const __bf16*)y, (__bf16*)out, N, H, W, C, Cu, c_off);
+  return nn_check("skip_bwd");
 }
 
 int shy_nn_channels(const void* src, void* dst, size_t P, int C, int Cy, int c_off, int dir,

@@ -53,6 +53,10 @@ def nn():
             "shy_nn_conv_wgrad_noalloc": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
             "shy_nn_conv_wgrad_bias": (i32, [vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32,
                                              i32, i32, vp]),
+            "shy_nn_conv_wgrad_bias_upcat": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32,
+                                                   i32, i32, vp]),
+            "shy_nn_up2_bwd_relu": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
+            "shy_nn_skip_bwd": (i32, [vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
             "shy_nn_bias_grad": (i32, [vp, vp, vp, i32, i32, i32, vp]),
             "shy_nn_relu_bwd": (i32, [vp, vp, vp, sz, vp]),
             "shy_nn_pool2": (i32, [vp, vp, i32, i32, i32, i32, i32, vp]),
@@ -216,14 +220,22 @@ class Conv:
     def backward(self, x, g, shape, scratch, need_dx=True, gres=None, mask=None):
         """g: gradient of the pre-activation output (bf16). Returns dx (bf16);
         with ``gres`` and ``mask`` (32-channel multiples) dx + gres, zeroed
-        where mask <= 0, from the data-gradient kernel's epilogue."""
+        where mask <= 0, from the data-gradient kernel's epilogue.  x is the
+        convolution's input, or the (xh, skip) of :meth:`forward_upcat`."""
         import torch
         N, H, W = shape
         P = N * H * W
         part, splits = scratch.part_for(self, P)
-        _ck(nn().shy_nn_conv_wgrad_bias(_p(x), _p(g), _p(self.dw), _p(self.db), _p(part), splits,
-                                        _p(scratch.bias_part), scratch.bias_rows, N, H, W,
-                                        self.cin, self.cout, self.taps, _stream()))
+        if isinstance(x, tuple):
+            xh, skip = x
+            _ck(nn().shy_nn_conv_wgrad_bias_upcat(_p(xh), _p(skip), _p(g), _p(self.dw),
+                                                  _p(self.db), _p(part), splits, N, H, W,
+                                                  xh.shape[-1], skip.shape[-1], self.cout,
+                                                  _stream()))
+        else:
+            _ck(nn().shy_nn_conv_wgrad_bias(_p(x), _p(g), _p(self.dw), _p(self.db), _p(part),
+                                            splits, _p(scratch.bias_part), scratch.bias_rows, N, H,
+                                            W, self.cin, self.cout, self.taps, _stream()))
         if not need_dx:
             return None
         if self._wf_of != (self.w_bf.data_ptr(), self.w_bf._version):
@@ -296,12 +308,15 @@ class ResStage:
         self.b = Conv(c, c, 9, gen, device)
         self.c = Conv(c, c, 9, gen, device)
 
-    def forward(self, x, shape, skip=None, head=None, pool=False):
+    def forward(self, x, shape, skip=None, head=None, pool=False, keep=None):
         """With ``skip`` the stage's input is [up2(x), skip] along channels,
-        read without building it (inference: nothing is kept for backward).
-        With ``head`` (a 1x1 Conv) returns (output or None with ``skip``,
-        head applied to it) from the last convolution's one pass.  With
-        ``pool`` returns (output, its 2x2 average pool), also from one pass."""
+        read without building it.  ``keep`` (default: without ``skip``) keeps
+        what :meth:`backward` needs.  With ``head`` (a 1x1 Conv) returns
+        (output or None without ``keep``, head applied to it) from the last
+        convolution's one pass.  With ``pool`` returns (output, its 2x2
+        average pool), also from one pass."""
+        if keep is None:
+            keep = skip is None
         if skip is None:
             ya = self.a.forward(x, shape)
         else:
@@ -313,15 +328,17 @@ class ResStage:
         elif head is None:
             yc = self.c.forward(yb, shape, res=ya)
         else:
-            yc, out = self.c.forward_head(yb, shape, head, res=ya, keep=skip is None)
-        self.saved = (x, ya, yb, yc) if skip is None else None
+            yc, out = self.c.forward_head(yb, shape, head, res=ya, keep=keep)
+        self.saved = (x if skip is None else (x, skip), ya, yb, yc) if keep else None
         if pool:
             return yc, pooled
         return yc if head is None else (yc, out)
 
-    def backward(self, g, shape, scratch, need_dx=True):
+    def backward(self, g, shape, scratch, need_dx=True, gated=False):
+        """g: gradient of the stage's output, with ``gated`` already zeroed
+        where that is not positive."""
         x, ya, yb, yc = self.saved
-        gc = _relu_bwd(yc, g)
+        gc = g if gated else _relu_bwd(yc, g)
         # relu_bwd(yb, dgrad_c) and relu_bwd(ya, gc + dgrad_b) in the
         # data-gradient epilogues (the same bits as the separate passes)
         gb = self.c.backward(yb, gc, shape, scratch, mask=yb)
@@ -372,10 +389,9 @@ class UNet:
 
     def forward(self, x, keep=True):
         """x: [N, H, W, 8] bf16 (H, W multiples of 8). Returns [N, H, W, 8] f32.
-        ``keep`` saves what :meth:`backward` needs; without it (inference) the
-        decoder stages read their upsampled-and-concatenated input straight
-        from the two tensors, with the same bits."""
-        import torch
+        ``keep`` saves what :meth:`backward` needs.  The decoder stages read
+        their upsampled-and-concatenated input straight from the two
+        tensors."""
         N, H, W, _ = x.shape
         self.shapes = [(N, H >> k, W >> k) for k in range(4)]
         self.kept = keep
@@ -392,19 +408,10 @@ class UNet:
                 h = self.e[k].forward(h, self.shapes[k])
         self.cat = []
         for k in (2, 1, 0):
-            n, hh, ww = self.shapes[k]
-            cu, cs = h.shape[-1], skips[k].shape[-1]
+            self.cat.append((h.shape[-1], skips[k].shape[-1]))
             # the last stage's last convolution applies the head in its own pass
-            head = self.head if k == 0 else None
-            if not keep:
-                h = self.d[k].forward(h, self.shapes[k], skip=skips[k], head=head)
-                continue
-            u = torch.empty(n, hh, ww, cu + cs, dtype=torch.bfloat16, device=x.device)
-            _ck(nn().shy_nn_up2(_p(h), _p(u), n, hh // 2, ww // 2, cu, cu + cs, 0, 0, _stream()))
-            _ck(nn().shy_nn_channels(_p(skips[k]), _p(u), n * hh * ww, cs, cu + cs, cu, 0,
-                                     _stream()))
-            self.cat.append((cu, cs))
-            h = self.d[k].forward(u, self.shapes[k], head=head)
+            h = self.d[k].forward(h, self.shapes[k], skip=skips[k],
+                                  head=self.head if k == 0 else None, keep=keep)
         self.h0, out = h
         return out
 
@@ -414,24 +421,27 @@ class UNet:
         if not self.kept:
             raise RuntimeError("backward needs a forward(..., keep=True)")
         g = self.head.backward(self.h0, gy, self.shapes[0], self.scratch)
-        gskip = [None, None, None]
+        gus = []
         for k, (cu, cs) in zip((0, 1, 2), reversed(self.cat)):
             n, hh, ww = self.shapes[k]
-            gu = self.d[k].backward(g, self.shapes[k], self.scratch)
-            gs = torch.empty(n, hh, ww, cs, dtype=torch.bfloat16, device=gy.device)
-            _ck(nn().shy_nn_channels(_p(gu), _p(gs), n * hh * ww, cs, cu + cs, cu, 1, _stream()))
-            gskip[k] = gs
+            gu = self.d[k].backward(g, self.shapes[k], self.scratch, gated=k > 0)
+            gus.append(gu)
+            # through the upsampling and the ReLU of the stage below
+            below = self.d[k + 1] if k < 2 else self.e[3]
             g = torch.empty(n, hh // 2, ww // 2, cu, dtype=torch.bfloat16, device=gy.device)
-            _ck(nn().shy_nn_up2(_p(gu), _p(g), n, hh // 2, ww // 2, cu, cu + cs, 0, 1, _stream()))
+            _ck(nn().shy_nn_up2_bwd_relu(_p(gu), _p(below.saved[3]), _p(g), n, hh // 2, ww // 2,
+                                         cu, cu + cs, 0, _stream()))
         for k in (3, 2, 1, 0):
-            gx = self.e[k].backward(g, self.shapes[k], self.scratch, need_dx=k > 0)
+            gx = self.e[k].backward(g, self.shapes[k], self.scratch, need_dx=k > 0, gated=True)
             if k == 0:
                 break
+            # the pooled path, the decoder's share and the ReLU of the stage above
             n, hh, ww = self.shapes[k - 1]
             c = gx.shape[-1]
-            gp = torch.empty(n, hh, ww, c, dtype=torch.bfloat16, device=gy.device)
-            _ck(nn().shy_nn_pool2(_p(gx), _p(gp), n, hh, ww, c, 1, _stream()))
-            g = _add(gp, gskip[k - 1])
+            cu, cs = self.cat[3 - k]
+            g = torch.empty(n, hh, ww, c, dtype=torch.bfloat16, device=gy.device)
+            _ck(nn().shy_nn_skip_bwd(_p(gx), _p(gus[k - 1]), _p(self.e[k - 1].saved[3]), _p(g), n,
+                                     hh, ww, c, cu + cs, cu, _stream()))
 
     def step(self, lr, wd=0.0):
         self.t += 1

@@ -47,3 +47,50 @@ def test_wgrad_and_bias_at_tile_edges(shy, N, H, W, cin, cout, splits):
                              N, H, W, cin, cout, 9, s)
     assert rc == 0, L.shy_nn_last_error()
     assert float((dw2.cpu().double() - ref).norm()) <= 1e-5 * float(ref.norm())
+
+
+@pytest.mark.parametrize("N,H,W,c1,c2,cout", [(1, 2, 2, 32, 32, 32), (2, 6, 34, 64, 32, 32),
+                                              (1, 18, 64, 32, 64, 64)])
+def test_wgrad_of_upsampled_input(shy, N, H, W, c1, c2, cout):
+    """The gradients of a convolution of [up2(xh), skip], read from the two
+    tensors: the bits of the ones from the concatenated input."""
+    from simplehydrology_amd import surrogate as sg
+    print("wgrad upcat", N, H, W, c1, c2, cout, flush=True)
+    gen = torch.Generator().manual_seed(H * W + cout)
+    xh, sk, g = (torch.randn(*s, generator=gen).to(torch.bfloat16).cuda()
+                 for s in ((N, H // 2, W // 2, c1), (N, H, W, c2), (N, H, W, cout)))
+    x = torch.cat([xh.repeat_interleave(2, 1).repeat_interleave(2, 2), sk], -1).contiguous()
+    conv = sg.Conv(c1 + c2, cout, 9, np.random.default_rng(0), "cuda:0")
+    scratch = sg.Scratch("cuda:0")
+    got = []
+    for inp in (x, (xh, sk)):
+        conv.dw.fill_(float("nan"))
+        conv.db.fill_(float("nan"))
+        conv.backward(inp, g, (N, H, W), scratch, need_dx=False)
+        got.append((conv.dw.clone(), conv.db.clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("N,H,W,c,cu,off", [(1, 2, 2, 8, 8, 0), (2, 6, 10, 32, 96, 64),
+                                            (3, 14, 6, 64, 160, 96)])
+def test_fused_skip_gradients(shy, N, H, W, c, cu, off):
+    """The passes between two stages of the backward in one kernel each: the
+    separate passes' bits."""
+    from simplehydrology_amd import surrogate as sg
+    print("skip", N, H, W, c, cu, off, flush=True)
+    L, s = sg.nn(), torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator().manual_seed(c)
+    gp, gu, y = (torch.randn(*d, generator=gen).to(torch.bfloat16).cuda()
+                 for d in ((N, H // 2, W // 2, c), (N, H, W, cu), (N, H, W, c)))
+    spread, share, out = (torch.empty_like(y) for _ in range(3))
+    assert L.shy_nn_pool2(gp.data_ptr(), spread.data_ptr(), N, H, W, c, 1, s) == 0
+    assert L.shy_nn_channels(gu.data_ptr(), share.data_ptr(), N * H * W, c, cu, off, 1, s) == 0
+    assert L.shy_nn_skip_bwd(gp.data_ptr(), gu.data_ptr(), y.data_ptr(), out.data_ptr(), N, H, W, c,
+                             cu, off, s) == 0
+    assert torch.equal(out, sg._relu_bwd(y, sg._add(spread, share)))
+    down, gated = torch.empty_like(gp), torch.empty_like(gp)
+    yh = torch.randn(N, H // 2, W // 2, c, generator=gen).to(torch.bfloat16).cuda()
+    assert L.shy_nn_up2(gu.data_ptr(), down.data_ptr(), N, H // 2, W // 2, c, cu, off, 1, s) == 0
+    assert L.shy_nn_up2_bwd_relu(gu.data_ptr(), yh.data_ptr(), gated.data_ptr(), N, H // 2, W // 2,
+                                 c, cu, off, s) == 0
+    assert torch.equal(gated, sg._relu_bwd(yh, down))
