@@ -140,6 +140,12 @@ int shy_nn_adam(float* w, const float* g, float* m, float* v, void* w_bf16, size
 int shy_nn_adam_conv(float* w, const float* g, float* m, float* v, void* w_bf16, void* wf_bf16,
                      int Cin, int Cout, int taps, float lr, float b1, float b2, float eps, int step,
                      float weight_decay, void* stream);
+/* The same, and shy_nn_adam without weight decay on the bias b[Cout], in one
+   launch (b null: the weights only) */
+int shy_nn_adam_conv_bias(float* w, const float* g, float* m, float* v, void* w_bf16,
+                          void* wf_bf16, int Cin, int Cout, int taps, float* b, const float* bg,
+                          float* bm, float* bv, float lr, float b1, float b2, float eps, int step,
+                          float weight_decay, void* stream);
 int shy_nn_cast(const void* src, void* dst, size_t n, int to_bf16, void* stream);
 
 #ifdef __cplusplus

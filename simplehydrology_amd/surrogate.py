@@ -67,6 +67,8 @@ def nn():
             "shy_nn_adam": (i32, [vp, vp, vp, vp, vp, sz, f32, f32, f32, f32, i32, f32, vp]),
             "shy_nn_adam_conv": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, f32, f32, f32, f32,
                                        i32, f32, vp]),
+            "shy_nn_adam_conv_bias": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, vp,
+                                            f32, f32, f32, f32, i32, f32, vp]),
             "shy_nn_cast": (i32, [vp, vp, sz, i32, vp]),
         }
         for name, (res, args) in sig.items():
@@ -257,12 +259,11 @@ class Conv:
         s = _stream()
         # the kernel writes w_bf and its flipped copy wf_bf (torch's version
         # counter of w_bf does not move: it counts writes made through torch)
-        _ck(nn().shy_nn_adam_conv(_p(self.w), _p(self.dw), _p(self.m[0]), _p(self.v[0]),
-                                  _p(self.w_bf), _p(self.wf_bf), self.cin, self.cout, self.taps,
-                                  lr, 0.9, 0.999, 1e-8, t, wd, s))
+        _ck(nn().shy_nn_adam_conv_bias(_p(self.w), _p(self.dw), _p(self.m[0]), _p(self.v[0]),
+                                       _p(self.w_bf), _p(self.wf_bf), self.cin, self.cout,
+                                       self.taps, _p(self.b), _p(self.db), _p(self.m[1]),
+                                       _p(self.v[1]), lr, 0.9, 0.999, 1e-8, t, wd, s))
         self._wf_of = (self.w_bf.data_ptr(), self.w_bf._version)
-        _ck(nn().shy_nn_adam(_p(self.b), _p(self.db), _p(self.m[1]), _p(self.v[1]), None,
-                             self.b.numel(), lr, 0.9, 0.999, 1e-8, t, 0.0, s))
 
     def params(self):
         return [self.w, self.b]
