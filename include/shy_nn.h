@@ -146,6 +146,26 @@ int shy_nn_adam_conv_bias(float* w, const float* g, float* m, float* v, void* w_
                           void* wf_bf16, int Cin, int Cout, int taps, float* b, const float* bg,
                           float* bm, float* bv, float lr, float b1, float b2, float eps, int step,
                           float weight_decay, void* stream);
+/* Tiled inference (no reference counterpart).  feats [X][Y][8] FP32 of a map:
+   height, its central differences x slope, log1p(discharge) x scale, signed
+   log1p(momentum) x scale, two zeros.  strides: {x, y} in elements of h, d,
+   mx, my. */
+int shy_nn_flow_features(const float* h, const float* d, const float* mx, const float* my,
+                         const long long* strides, float* feats, int X, int Y, float slope,
+                         float scale, void* stream);
+/* n <= 32 windows of tile x tile cells, jobs {wx, cx, lx, wy, cy, ly} each
+   (host memory): the window's first cell, its core's first cell and length,
+   along x and y.  out [n][tile][tile][8] = the windows of feats. */
+int shy_nn_window_copy(const float* feats, const int* jobs, int n, float* out, int X, int Y,
+                       int tile, void* stream);
+/* the windows in bf16, channel 0 as (height - mean[window]) x scale */
+int shy_nn_window_input(const float* xs, const float* mean, void* out, int n, int tile, float scale,
+                        void* stream);
+/* the cores of the network's outputs y [n][tile][tile][8], decoded (the
+   inverse of the features' encoding, exponents capped at 20), into d, mx, my
+   [X][Y] */
+int shy_nn_window_output(const float* y, const int* jobs, int n, float* d, float* mx, float* my,
+                         int X, int Y, int tile, float scale, void* stream);
 int shy_nn_cast(const void* src, void* dst, size_t n, int to_bf16, void* stream);
 
 #ifdef __cplusplus

@@ -69,6 +69,10 @@ def nn():
                                        i32, f32, vp]),
             "shy_nn_adam_conv_bias": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, vp,
                                             f32, f32, f32, f32, i32, f32, vp]),
+            "shy_nn_flow_features": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, f32, f32, vp]),
+            "shy_nn_window_copy": (i32, [vp, vp, i32, vp, i32, i32, i32, vp]),
+            "shy_nn_window_input": (i32, [vp, vp, vp, i32, i32, f32, vp]),
+            "shy_nn_window_output": (i32, [vp, vp, i32, vp, vp, vp, i32, i32, i32, f32, vp]),
             "shy_nn_cast": (i32, [vp, vp, sz, i32, vp]),
         }
         for name, (res, args) in sig.items():
@@ -500,13 +504,38 @@ def predict_tiled(net, h, d, mx, my, tile=256, halo=32, batch=16):
     X, Y = h.shape
     if X < tile or Y < tile:
         raise ValueError(f"map {X}x{Y} is smaller than one {tile}x{tile} window")
-    feats = features(h, d, mx, my)
-    out = torch.empty(X, Y, 3, dtype=torch.float32, device=h.device)
     jobs = [(wx, cx, lx, wy, cy, ly) for wx, cx, lx in _tile_starts(X, tile, halo)
             for wy, cy, ly in _tile_starts(Y, tile, halo)]
+    maps = (h, d, mx, my)
+    if any(t.dtype != torch.float32 or t.shape != h.shape or t.device != h.device
+           for t in maps) or not h.is_cuda or tile > 32767:
+        feats = features(h, d, mx, my)
+        out = torch.empty(X, Y, 3, dtype=torch.float32, device=h.device)
+        for b0 in range(0, len(jobs), batch):
+            js = jobs[b0:b0 + batch]
+            y = net.forward(window_batch(feats, [(j[0], j[3]) for j in js], tile), keep=False)
+            for k, (wx, cx, lx, wy, cy, ly) in enumerate(js):
+                out[cx:cx + lx, cy:cy + ly] = y[k, cx - wx:cx - wx + lx, cy - wy:cy - wy + ly, :3]
+        return decode_flow(out)
+    # features, windows, crops and decoding in one launch each
+    strides = (C.c_longlong * 8)(*(s for t in maps for s in t.stride()))
+    feats = torch.empty(X, Y, 8, dtype=torch.float32, device=h.device)
+    _ck(nn().shy_nn_flow_features(_p(h), _p(d), _p(mx), _p(my), strides, _p(feats), X, Y,
+                                  SLOPE_SCALE, 1.0 / D_SCALE, _stream()))
+    out = [torch.empty(X, Y, dtype=torch.float32, device=h.device) for _ in range(3)]
     for b0 in range(0, len(jobs), batch):
         js = jobs[b0:b0 + batch]
-        y = net.forward(window_batch(feats, [(j[0], j[3]) for j in js], tile), keep=False)
-        for k, (wx, cx, lx, wy, cy, ly) in enumerate(js):
-            out[cx:cx + lx, cy:cy + ly] = y[k, cx - wx:cx - wx + lx, cy - wy:cy - wy + ly, :3]
-    return decode_flow(out)
+        n = len(js)
+        xs = torch.empty(n, tile, tile, 8, dtype=torch.float32, device=h.device)
+        parts = [(k, min(32, n - k), (C.c_int * (6 * min(32, n - k)))(
+            *(v for j in js[k:k + 32] for v in j))) for k in range(0, n, 32)]
+        for k, m, table in parts:
+            _ck(nn().shy_nn_window_copy(_p(feats), table, m, _p(xs[k]), X, Y, tile, _stream()))
+        mean = xs[..., 0].mean(dim=(1, 2))
+        x = torch.empty(n, tile, tile, 8, dtype=torch.bfloat16, device=h.device)
+        _ck(nn().shy_nn_window_input(_p(xs), _p(mean), _p(x), n, tile, H_SCALE, _stream()))
+        y = net.forward(x, keep=False)
+        for k, m, table in parts:
+            _ck(nn().shy_nn_window_output(_p(y[k]), table, m, _p(out[0]), _p(out[1]), _p(out[2]),
+                                          X, Y, tile, D_SCALE, _stream()))
+    return tuple(out)

@@ -85,3 +85,26 @@ def test_upsampled_input(shy, N, H, W, c1, c2, cout):
                                        r.data_ptr() if r is not None else None, y.data_ptr(), None,
                                        N, H, W, c1, c2, cout, 0, s) == 0
         close(y, ref if r is None else ref + res.double(), 2 ** -8)
+
+
+@pytest.mark.parametrize("X,Y,tile,halo,batch", [(64, 64, 64, 8, 4), (65, 97, 64, 8, 3),
+                                                 (40, 300, 32, 4, 40), (33, 32, 32, 4, 16)])
+def test_tiled_inference_passes(shy, X, Y, tile, halo, batch):
+    """Features, windows, crops and decoding of the tiled inference against
+    the element-wise passes, on strided maps with values below zero.  The math
+    library's log1p and expm1 differ by at most 2 ulp each, which BF16 inputs
+    pass on as half an ulp of theirs at most: the network's output moves by
+    less than 2^-8 of its norm."""
+    from simplehydrology_amd import surrogate as sg
+    print("tiled", X, Y, tile, flush=True)
+    g = torch.Generator().manual_seed(X)
+    a = torch.randn(X, Y, 4, generator=g).cuda()
+    a[..., 1:] *= 30.0
+    h, d, mx, my = (a[..., k] for k in range(4))
+    net = sg.UNet(seed=1)
+    got = sg.predict_tiled(net, h, d, mx, my, tile=tile, halo=halo, batch=batch)
+    # float64 maps take the element-wise passes; features() keeps float32
+    want = sg.predict_tiled(net, h.double(), d, mx, my, tile=tile, halo=halo, batch=batch)
+    for u, v in zip(got, want):
+        assert u.shape == v.shape and u.dtype == torch.float32 and u.is_contiguous()
+        assert float((u - v).norm()) <= 2 ** -8 * float(v.norm())
