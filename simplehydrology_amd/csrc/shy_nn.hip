@@ -490,7 +490,7 @@ __global__ void __launch_bounds__(256, 2) conv_pf_kernel(ConvArgs a) {
 // hardware checks each offset against the buffer's size, so only the tiles at
 // the left and right edge compare columns.  The rows of one tile must span
 // less than 2^31 bytes (tile_rows_fit).  A tile's residual (kEpiRes) or the
-// backward pass's residual and mask (kEpiGrad) are on their way while the next
+// backward pass's residual and mask (kEpiGrad, kEpiMask) are on their way while the next
 // tile goes to LDS.
 // Measured against the same loop with an address, a bounds check and a branch
 // per load (us, at batch 16): 256^2, 32 -> 32 channels 40.1 -> 28.9 (4.6 TB/s),
@@ -515,7 +515,7 @@ inline bool tile_rows_fit(const ConvArgs& a) {
   return (long long)a.W * c * 2 * 20 < 0x7fffffffLL;
 }
 
-enum { kEpiPlain, kEpiRes, kEpiGrad };
+enum { kEpiPlain, kEpiRes, kEpiMask, kEpiGrad };  // + nothing, res, mask, gres (and mask)
 
 template <int MT, int NT, bool UPCAT, bool HEAD, bool POOL, int EPI>
 __global__ void __launch_bounds__(256, kTileBlocksPerCU) conv_tiles_kernel(ConvArgs a) {
@@ -664,10 +664,8 @@ __global__ void __launch_bounds__(256, kTileBlocksPerCU) conv_tiles_kernel(ConvA
     }
     u32x2 e0[MT][NT], e1[MT][NT];
     if (EPI == kEpiRes) load_out(a.res, e0);
-    if (EPI == kEpiGrad) {
-      load_out(a.gres, e0);
-      load_out(a.mask, e1);
-    }
+    if (EPI == kEpiGrad) load_out(a.gres, e0);
+    if (EPI == kEpiGrad || EPI == kEpiMask) load_out(a.mask, e1);
     if (tile + (int)gridDim.x < total) {
       __syncthreads();
       lstore(reload_w);
@@ -703,12 +701,12 @@ __global__ void __launch_bounds__(256, kTileBlocksPerCU) conv_tiles_kernel(ConvA
         for (int i = 0; i < 4; ++i) q[m][t][i] = (__bf16)v[i];
         if (EPI == kEpiGrad) {
           const bf16x4 gr = __builtin_bit_cast(bf16x4, e0[m][t]);
-          const bf16x4 mk = __builtin_bit_cast(bf16x4, e1[m][t]);
-          if (a.gres) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) q[m][t][i] = (__bf16)((float)q[m][t][i] + (float)gr[i]);
-          }
-          if (a.mask) {
+          for (int i = 0; i < 4; ++i) q[m][t][i] = (__bf16)((float)q[m][t][i] + (float)gr[i]);
+        }
+        if (EPI == kEpiGrad || EPI == kEpiMask) {
+          const bf16x4 mk = __builtin_bit_cast(bf16x4, e1[m][t]);
+          if (EPI == kEpiMask || a.mask) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
               q[m][t][i] = (float)mk[i] > 0.0f ? q[m][t][i] : (__bf16)0.0f;
@@ -1664,7 +1662,6 @@ int launch_tiles(const ConvArgs& a, hipStream_t s, const char* what) {
   const int gy = a.Cout / (16 * MT);
   const long long cap = std::max(1LL, (long long)kTileBlocksPerCU * device_cus() / gy);
   const dim3 g((unsigned)std::min(tiles, cap), (unsigned)gy);
-  const bool grad = a.gres || a.mask;
   if (a.x2) {
     if (a.res) conv_tiles_kernel<MT, NT, true, false, false, kEpiRes><<<g, 256, 0, s>>>(a);
     else conv_tiles_kernel<MT, NT, true, false, false, kEpiPlain><<<g, 256, 0, s>>>(a);
@@ -1674,8 +1671,10 @@ int launch_tiles(const ConvArgs& a, hipStream_t s, const char* what) {
   } else if (a.pool_y) {
     if (a.res) conv_tiles_kernel<MT, NT, false, false, true, kEpiRes><<<g, 256, 0, s>>>(a);
     else conv_tiles_kernel<MT, NT, false, false, true, kEpiPlain><<<g, 256, 0, s>>>(a);
-  } else if (grad) {
+  } else if (a.gres) {
     conv_tiles_kernel<MT, NT, false, false, false, kEpiGrad><<<g, 256, 0, s>>>(a);
+  } else if (a.mask) {
+    conv_tiles_kernel<MT, NT, false, false, false, kEpiMask><<<g, 256, 0, s>>>(a);
   } else {
     if (a.res) conv_tiles_kernel<MT, NT, false, false, false, kEpiRes><<<g, 256, 0, s>>>(a);
     else conv_tiles_kernel<MT, NT, false, false, false, kEpiPlain><<<g, 256, 0, s>>>(a);
