@@ -1833,16 +1833,21 @@ int shy_get_stats(shy_ctx* c, shy_stats* out) {
   DeviceState st;
   HIPCHK(c, hipMemcpyAsync(&st, c->state, sizeof(st), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  out->steps = st.stats[ST_STEPS];
-  out->walked = st.stats[ST_WALKED];
-  out->skipped = st.stats[ST_SKIPPED];
-  out->exits = st.stats[ST_EXITS];
-  out->ends_age = st.stats[ST_ENDS_AGE];
-  out->ends_vol = st.stats[ST_ENDS_VOL];
-  out->export40 = st.stats[ST_EXPORT40];
-  out->gain40 = st.stats[ST_GAIN40];
-  out->walk_dh = st.stats[ST_WALK_DH];
-  out->casc_moves = st.stats[ST_CASC_MOVES];
+  unsigned long long u[ST_COUNT] = {};
+  for (const auto& slot : st.stats)
+    for (int k = 0; k < ST_COUNT; ++k) u[k] += (unsigned long long)slot[k];
+  long long sum[ST_COUNT];
+  for (int k = 0; k < ST_COUNT; ++k) sum[k] = (long long)u[k];
+  out->steps = sum[ST_STEPS];
+  out->walked = sum[ST_WALKED];
+  out->skipped = sum[ST_SKIPPED];
+  out->exits = sum[ST_EXITS];
+  out->ends_age = sum[ST_ENDS_AGE];
+  out->ends_vol = sum[ST_ENDS_VOL];
+  out->export40 = sum[ST_EXPORT40];
+  out->gain40 = sum[ST_GAIN40];
+  out->walk_dh = sum[ST_WALK_DH];
+  out->casc_moves = sum[ST_CASC_MOVES];
   return SHY_OK;
 }
 
