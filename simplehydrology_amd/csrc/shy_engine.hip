@@ -170,7 +170,8 @@ bool ordered(const shy_ctx* c) {
 // 5270 / 5300, 2048^2 x 262144 1297 / 1415 / 1174, 4096^2 x 524288 3430 / 3380 /
 // 3230.  Without the order the waves share nothing (2048^2 x 196608 1718 / 1717 /
 // 1750).
-constexpr int kWalkLds = 56 * 1024;
+// A block of bs threads takes bs / 512 of the 160 KB, 16 KB of it the walk's own.
+int walk_lds(int bs) { return std::min(160 * 1024, 320 * bs) - 17 * 1024; }
 // The replay's blocks are single waves, three of which take a CU's LDS (unused):
 // the gathers of more waves evict each other's lines from its vector cache.
 // us with as many waves as the registers hold / 4 / 3 / 2 / 1 per CU: 65536 drops
@@ -723,7 +724,7 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
     // the record prefetch pays where every drop runs at once (the walk is
     // bound by its chain's latency): the same waves the drop order leaves off
     const bool pf = !ordered(c);
-    const int lds = pf ? 0 : kWalkLds;
+    const int lds = pf ? 0 : walk_lds(bs);
     if (c->walk_counts)
       (pf ? walk_kernel<true, true> : walk_kernel<true, false>)<<<grid, bs, lds, c->stream>>>(w);
     else
