@@ -45,7 +45,7 @@ int shy_nn_conv_fwd_upcat(const void* x_half, const void* skip, const void* w, c
    pass: head_y [N][H][W][head_c] (FP32) = head_b + head_w [head_c][32] . y,
    head_c in {4, 8, 12, 16}, Cin 32 or 64, head_w and head_b 16-byte
    aligned.  A network's last convolution and its output head without the
-   32-channel tensor round trip. */
+   32-channel tensor round trip.  W above 800000 needs y (two passes). */
 int shy_nn_conv_fwd_head(const void* x, const void* w, const float* bias, const void* res,
                          void* y_bf16, const void* head_w, const float* head_b, float* head_y,
                          int N, int H, int W, int Cin, int head_c, int relu, void* stream);
@@ -56,6 +56,17 @@ int shy_nn_conv_fwd_head(const void* x, const void* w, const float* bias, const 
 int shy_nn_conv_fwd_pool(const void* x, const void* w, const float* bias, const void* res,
                          void* y_bf16, void* pool_y, int N, int H, int W, int Cin, int Cout,
                          int relu, void* stream);
+/* The whole 4-level residual U-Net of surrogate.py, inference only: its 22
+   convolutions' weights w (BF16, the layouts above) and biases b in the order
+   encoder stages of levels 0..3, decoder stages of levels 0..2 (three each),
+   head; x [N][H][W][cin], ch[4] the levels' channels (ch[0] 32 or 64, a
+   multiple of 32 each), out [N][H][W][head_c] FP32.  H, W multiples of 8.  The
+   tables are read during the call.  work holds at least
+   shy_nn_unet_work_bytes(ch, N, H, W) bytes. */
+long long shy_nn_unet_work_bytes(const int* ch, int N, int H, int W);
+int shy_nn_unet_forward(const void* x, const void* const* w, const float* const* b, const int* ch,
+                        int cin, int head_c, void* work, long long work_bytes, float* out, int N,
+                        int H, int W, void* stream);
 /* The data gradient dx [N][H][W][Cin] (BF16) of a convolution from g
    [N][H][W][Cout] with the flipped weights wf of shy_nn_flip_weights, with
    the backward pass's next two element-wise steps in its epilogue: gres

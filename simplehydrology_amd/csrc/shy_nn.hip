@@ -1893,6 +1893,82 @@ int shy_nn_conv_fwd_pool(const void* x, const void* w, const float* bias, const 
   return launch_tiles(a, (hipStream_t)stream, "conv_fwd_pool");
 }
 
+// Work memory of shy_nn_unet_forward: per level three activations of its
+// channels (stage output and two between), the pooled input of the next level.
+static size_t unet_align(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
+long long shy_nn_unet_work_bytes(const int* ch, int N, int H, int W) {
+  if (!ch || N < 1 || H < 8 || W < 8 || H % 8 || W % 8) return -1;
+  size_t sum = 0;
+  for (int k = 0; k < 4; ++k) {
+    const size_t p = (size_t)N * (H >> k) * (W >> k) * 2;
+    sum += 3 * unet_align(p * ch[k]) + (k < 3 ? unet_align(p / 4 * ch[k]) : 0);
+  }
+  return (long long)sum;
+}
+
+int shy_nn_unet_forward(const void* x, const void* const* w, const float* const* b, const int* ch,
+                        int cin, int head_c, void* work, long long work_bytes, float* out, int N,
+                        int H, int W, void* stream) {
+  if (!x || !w || !b || !ch || !work || !out) return nn_fail("unet_forward: bad pointers");
+  const long long need = shy_nn_unet_work_bytes(ch, N, H, W);
+  if (need < 0) return nn_fail("unet_forward: H and W must be multiples of 8");
+  if (work_bytes < need) return nn_fail("unet_forward: work memory too small");
+  char* at = (char*)work;
+  auto take = [&](size_t bytes) {
+    void* p = at;
+    at += unet_align(bytes);
+    return p;
+  };
+  void *ya[4], *yb[4], *yc[4], *pool[3];
+  for (int k = 0; k < 4; ++k) {
+    const size_t p = (size_t)N * (H >> k) * (W >> k) * 2;
+    ya[k] = take(p * ch[k]);
+    yb[k] = take(p * ch[k]);
+    yc[k] = take(p * ch[k]);
+    if (k < 3) pool[k] = take(p / 4 * ch[k]);
+  }
+  int c = 0;  // convolution
+  auto conv = [&](const void* in, void* y, const void* res, int k, int ci) {
+    const int r = shy_nn_conv_fwd(in, w[c], b[c], res, y, nullptr, N, H >> k, W >> k, ci, ch[k], 9,
+                                  1, stream);
+    ++c;
+    return r;
+  };
+  const void* h = x;
+  for (int k = 0; k < 4; ++k) {
+    if (int r = conv(h, ya[k], nullptr, k, k == 0 ? cin : ch[k - 1])) return r;
+    if (int r = conv(ya[k], yb[k], nullptr, k, ch[k])) return r;
+    if (k == 3) {
+      if (int r = conv(yb[k], yc[k], ya[k], k, ch[k])) return r;
+    } else {
+      if (int r = shy_nn_conv_fwd_pool(yb[k], w[c], b[c], ya[k], yc[k], pool[k], N, H >> k, W >> k,
+                                       ch[k], ch[k], 1, stream))
+        return r;
+      ++c;
+      h = pool[k];
+    }
+  }
+  // decoder stages take the encoder's ya, yb and, but for the last, write over
+  // its skip after reading it
+  for (int k = 2; k >= 0; --k) {
+    // w and b list the decoder stages from level 0 on
+    c = 12 + 3 * k;
+    if (int r = shy_nn_conv_fwd_upcat(yc[k + 1], yc[k], w[c], b[c], nullptr, ya[k], nullptr, N,
+                                      H >> k, W >> k, ch[k + 1], ch[k], ch[k], 1, stream))
+      return r;
+    ++c;
+    if (int r = conv(ya[k], yb[k], nullptr, k, ch[k])) return r;
+    if (k > 0) {
+      if (int r = conv(yb[k], yc[k], ya[k], k, ch[k])) return r;
+    } else if (int r = shy_nn_conv_fwd_head(yb[k], w[c], b[c], ya[k], nullptr, w[21], b[21], out, N,
+                                            H, W, ch[0], head_c, 1, stream)) {
+      return r;
+    }
+  }
+  return 0;
+}
+
 int shy_nn_conv_dgrad(const void* g, const void* wf, const void* gres, const void* mask,
                       void* dx_bf16, int N, int H, int W, int Cin, int Cout, int taps,
                       void* stream) {

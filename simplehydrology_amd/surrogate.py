@@ -43,6 +43,9 @@ def nn():
                                       vp]),
             "shy_nn_conv_fwd_upcat": (i32, [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32,
                                             i32, i32, vp]),
+            "shy_nn_unet_work_bytes": (C.c_longlong, [vp, i32, i32, i32]),
+            "shy_nn_unet_forward": (i32, [vp, vp, vp, vp, i32, i32, vp, C.c_longlong, vp, i32, i32,
+                                          i32, vp]),
             "shy_nn_conv_dgrad": (i32, [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
             "shy_nn_conv_fwd_head": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32,
                                            i32, i32, vp]),
@@ -400,6 +403,8 @@ class UNet:
         N, H, W, _ = x.shape
         self.shapes = [(N, H >> k, W >> k) for k in range(4)]
         self.kept = keep
+        if not keep:
+            return self._infer(x, N, H, W)
         skips = []
         h = x
         for k in range(4):
@@ -418,6 +423,26 @@ class UNet:
             h = self.d[k].forward(h, self.shapes[k], skip=skips[k],
                                   head=self.head if k == 0 else None, keep=keep)
         self.h0, out = h
+        return out
+
+    def _infer(self, x, N, H, W):
+        """The forward without what backward needs, in one call: 21 launches
+        made one by one from here take 9 us of host time each, more than a
+        small batch's kernels."""
+        import torch
+        for s in self.e + self.d:
+            s.saved = None
+        cs = self.convs()
+        w = (C.c_void_p * len(cs))(*(c.w_bf.data_ptr() for c in cs))
+        b = (C.c_void_p * len(cs))(*(c.b.data_ptr() for c in cs))
+        ch = (C.c_int * 4)(*(s.a.cout for s in self.e))
+        size = nn().shy_nn_unet_work_bytes(ch, N, H, W)
+        if size < 0:
+            raise RuntimeError("shy_nn: unet_forward: H and W must be multiples of 8")
+        work = torch.empty(size, dtype=torch.uint8, device=x.device)
+        out = torch.empty(N, H, W, self.head.cout, dtype=torch.float32, device=x.device)
+        _ck(nn().shy_nn_unet_forward(_p(x), w, b, ch, cs[0].cin, self.head.cout, _p(work), size,
+                                     _p(out), N, H, W, _stream()))
         return out
 
     def backward(self, gy):
