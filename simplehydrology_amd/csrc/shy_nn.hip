@@ -8,9 +8,9 @@
 // that instruction (checked on the device): lane l holds A[l%16][(l/16)*8+i],
 // B[(l/16)*8+i][l%16] for i < 8 and C[(l/16)*4+i][l%16] for i < 4.
 //
-//   conv_tiles_kernel  3x3 forward / data gradient of every layer whose
-//                      16x16 pixel tiles give each CU at least one:
-//                      persistent blocks (three per CU, 32 output channels
+//   conv_tiles_kernel  3x3 forward / data gradient of every layer of 32-channel
+//                      multiples, 16x16 pixel tiles (16x8 where those leave a
+//                      CU without any): persistent blocks (three per CU, 32 output channels
 //                      each) over the tiles, patch and weights staged in LDS,
 //                      the next chunk's patch loaded into registers during
 //                      the current chunk's MFMAs; decoder inputs read as
@@ -18,8 +18,8 @@
 //                      head on the rounded output, or its 2x2 average pool
 //                      (pairs of rows in a lane, pairs of columns across
 //                      lanes l and l ^ 1)
-//   conv_pf_kernel     the same arithmetic with one tile per block for the
-//                      smaller layers (16x8 tiles: more blocks)
+//   conv_pf_kernel     the same arithmetic with one tile per block, for 1x1
+//                      convolutions and rows beyond the tile loop's offsets
 //   conv_c8_kernel     the 8-channel first layer, four taps per MFMA k-step
 //   conv_fwd_kernel    direct-load convolution of the remaining shapes (the
 //                      head's data gradient)
@@ -29,11 +29,13 @@
 //                      by Adam) the residual gradient and the ReLU mask
 //   wgrad_lds_kernel   dW[co][k] = sum_p g[p][co] x[p + tap][ci]: K = pixels,
 //   conv_wgrad_kernel  staged through LDS (both operands need 8 consecutive
-//                      pixels per lane; the second loads directly), split
-//                      over pixel ranges into FP32 partials that
-//                      wgrad_reduce_kernel sums in a fixed order
+//                      pixels per lane: transposed LDS reads; the second loads
+//                      directly), split over pixel ranges into FP32 partials
+//                      that wgrad_reduce_kernel sums in a fixed order; the first
+//                      sums the bias gradient from the same tiles
 //   elementwise        ReLU backward, 2x2 average pool, nearest upsample,
-//                      channel concat/split, bias gradient, MSE loss, Adam
+//                      channel concat/split, the fused passes between two
+//                      stages of the backward, bias gradient, MSE loss, Adam
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -80,7 +82,7 @@ struct ConvArgs {
   float* y_f;
   int N, H, W, Cin, Cout, K;
   int relu;
-  // When x2 is set (conv_pf_kernel only), the input is the concatenation of
+  // When x2 is set (UPCAT instantiations), the input is the concatenation of
   // a nearest x2 upsample of x ([N][H/2][W/2][C1]) and x2 ([N][H][W][Cin-C1]).
   const __bf16* __restrict__ x2;
   int C1;
@@ -342,7 +344,7 @@ constexpr int kPS = 40;
 // read from LDS once per column shift dx and used for the three row shifts
 // dy (a wave's NT output rows need NT + 2 patch rows): per chunk and wave
 // 3 (NT + 2) B reads and 9 MT A reads feed 9 MT NT MFMAs.
-template <int TAPS, int MT, int NT, bool UPCAT = false, bool PF = true>
+template <int TAPS, int MT, int NT, bool UPCAT = false>
 __global__ void __launch_bounds__(256, 2) conv_pf_kernel(ConvArgs a) {
   constexpr int kTH = 4 * NT;
   constexpr int HALO = TAPS == 9 ? 1 : 0;
@@ -420,22 +422,12 @@ __global__ void __launch_bounds__(256, 2) conv_pf_kernel(ConvArgs a) {
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  // PF: the next chunk loads into registers during this chunk's MFMAs; else
-  // each chunk is loaded and staged before its MFMAs (fewer registers live
-  // across them, for single-chunk layers with larger tiles)
-  if constexpr (PF) {
-    gload(0);
-    lstore();
-    __syncthreads();
-  }
+  // the next chunk loads into registers during this chunk's MFMAs
+  gload(0);
+  lstore();
+  __syncthreads();
   for (int ci0 = 0; ci0 < Cin; ci0 += 32) {
-    if constexpr (!PF) {
-      if (ci0 > 0) __syncthreads();
-      gload(ci0);
-      lstore();
-      __syncthreads();
-    }
-    const bool more = PF && ci0 + 32 < Cin;
+    const bool more = ci0 + 32 < Cin;
     if (more) gload(ci0 + 32);
 #pragma unroll
     for (int dx = 0; dx < NS; ++dx) {
@@ -459,12 +451,10 @@ __global__ void __launch_bounds__(256, 2) conv_pf_kernel(ConvArgs a) {
           for (int t = 0; t < NT; ++t) acc[m][t] = mfma(A[m], B[t + dy], acc[m][t]);
       }
     }
-    if constexpr (PF) {
+    __syncthreads();
+    if (more) {
+      lstore();
       __syncthreads();
-      if (more) {
-        lstore();
-        __syncthreads();
-      }
     }
   }
   conv_epilogue<MT, NT>(a, acc, n, y0, x0, cb, wave, lane);
@@ -1655,8 +1645,9 @@ int device_cus() {
 // 64-channel layer takes two such blocks per tile: at 16 x 128^2, 32->64
 // 31.1 -> 27.8 us and 64->64 41.7 -> 40.7 us against one 64-channel block
 // at two blocks per CU (the 64-channel block needs 255 VGPRs).
-int launch_tiles(const ConvArgs& a, hipStream_t s, const char* what) {
-  constexpr int MT = 2, NT = 4;
+template <int NT>
+int launch_tiles_of(const ConvArgs& a, hipStream_t s, const char* what) {
+  constexpr int MT = 2;
   const long long tiles = (long long)a.N * ((a.H + 4 * NT - 1) / (4 * NT)) * ((a.W + kTW - 1) / kTW);
   if (tiles > INT32_MAX) return nn_fail(std::string(what) + ": too many tiles");
   const int gy = a.Cout / (16 * MT);
@@ -1682,40 +1673,33 @@ int launch_tiles(const ConvArgs& a, hipStream_t s, const char* what) {
   return nn_check(what);
 }
 
-// conv_pf_kernel for Cin and Cout multiples of 32, 32 output channels per
-// block (MT = 2; 64-channel blocks at 32^2 and 128^2 ran 4-16% slower: half
-// the blocks, and 210-256 VGPRs), 16x16 tiles (4 rows per wave) when they
-// still give >= 1024 blocks, else 16x8.
-int launch_pf(const ConvArgs& a, int taps, hipStream_t s, const char* what) {
+// 16 x 8 tiles where 16 x 16 ones leave a CU without any: twice the blocks,
+// each half as long (a whole forward, us with 16 x 16 blocks of one tile each,
+// an address and a check per load and a pool pass of its own / with these: one
+// window of 64^2 160 / 144, two of 128^2 170 / 149, four of 256^2 243 / 234)
+int launch_tiles(const ConvArgs& a, hipStream_t s, const char* what) {
   const long long tiles16 = (long long)a.N * ((a.H + 15) / 16) * ((a.W + kTW - 1) / kTW);
-  // 3x3 layers whose 16x16 tiles give every CU at least one: the persistent
-  // tile loop, decoder inputs included (at batch 16, against the one-tile
-  // blocks below: 32->32 at 256^2 50.7 -> 43.4 us, [up2, skip] 96->32 at
-  // 256^2 105 -> 83 us, 96->96 at 64^2 23.0 -> 21.5 us; at 32^2, 64 tiles,
-  // the one-tile blocks' 16x8 tiles are faster)
-  if (taps == 9 && tiles16 >= device_cus() && tile_rows_fit(a)) return launch_tiles(a, s, what);
+  return tiles16 >= device_cus() ? launch_tiles_of<4>(a, s, what) : launch_tiles_of<2>(a, s, what);
+}
+
+// Cin and Cout multiples of 32: the tile loop for 3x3 (against one tile per
+// block at batch 16: 32->32 at 256^2 50.7 -> 43.4 us, [up2, skip] 96->32 at 256^2
+// 105 -> 83 us before its buffer accesses); conv_pf_kernel, 32 output channels
+// per block (64-channel blocks ran 4-16% slower: half the blocks, and 210-256
+// VGPRs), for 1x1 and for rows beyond the tile loop's offsets, with 16x16 tiles
+// when they give >= 1024 blocks, else 16x8.
+int launch_pf(const ConvArgs& a, int taps, hipStream_t s, const char* what) {
+  if (taps == 9 && tile_rows_fit(a)) return launch_tiles(a, s, what);
+  const long long tiles16 = (long long)a.N * ((a.H + 15) / 16) * ((a.W + kTW - 1) / kTW);
   const unsigned gy = (unsigned)(a.Cout / 32);
   const long long tiles8 = (long long)a.N * ((a.H + 7) / 8) * ((a.W + kTW - 1) / kTW);
   if (tiles8 > INT32_MAX) return nn_fail(std::string(what) + ": too many tiles");
-  const bool big = tiles16 * gy >= 1024;
+  const bool big = taps == 9 || tiles16 * gy >= 1024;
   const dim3 g((unsigned)(big ? tiles16 : tiles8), gy);
-  const long long tiles32 = (long long)a.N * ((a.H + 31) / 32) * ((a.W + kTW - 1) / kTW);
-  if (!a.x2 && taps == 9 && a.Cin == 32 && tiles32 * gy >= 1024) {
-    // one input chunk: 16x32 tiles staged without prefetch, so each block
-    // reloads the layer's weights for twice the pixels
-    conv_pf_kernel<9, 2, 8, false, false><<<dim3((unsigned)tiles32, gy), 256, 0, s>>>(a);
-    return nn_check(what);
-  }
-  if (a.x2) {  // the input is [up2(x), x2] (taps 9)
-    if (big) conv_pf_kernel<9, 2, 4, true><<<g, 256, 0, s>>>(a);
-    else conv_pf_kernel<9, 2, 2, true><<<g, 256, 0, s>>>(a);
-  } else if (big) {
-    if (taps == 9) conv_pf_kernel<9, 2, 4><<<g, 256, 0, s>>>(a);
-    else conv_pf_kernel<1, 2, 4><<<g, 256, 0, s>>>(a);
-  } else {
-    if (taps == 9) conv_pf_kernel<9, 2, 2><<<g, 256, 0, s>>>(a);
-    else conv_pf_kernel<1, 2, 2><<<g, 256, 0, s>>>(a);
-  }
+  if (a.x2) conv_pf_kernel<9, 2, 4, true><<<g, 256, 0, s>>>(a);  // the input is [up2(x), x2]
+  else if (taps == 9) conv_pf_kernel<9, 2, 4><<<g, 256, 0, s>>>(a);
+  else if (big) conv_pf_kernel<1, 2, 4><<<g, 256, 0, s>>>(a);
+  else conv_pf_kernel<1, 2, 2><<<g, 256, 0, s>>>(a);
   return nn_check(what);
 }
 
@@ -1867,11 +1851,10 @@ int shy_nn_conv_fwd_pool(const void* x, const void* w, const float* bias, const 
   if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || Cin < 32 || Cin % 32 || Cout < 32 || Cout % 32)
     return nn_fail("conv_fwd_pool: need H, W even and Cin, Cout multiples of 32");
   if ((long long)N * H * W > INT32_MAX / 2) return nn_fail("conv_fwd_pool: too many pixels");
-  const long long tiles16 = (long long)N * ((H + 15) / 16) * ((W + kTW - 1) / kTW);
   ConvArgs a;
   a.W = W; a.Cin = Cin; a.Cout = Cout;
-  if (tiles16 < device_cus() || !tile_rows_fit(a)) {
-    // layers the tile loop does not take: the convolution, then the pool
+  if (!tile_rows_fit(a)) {
+    // rows the tile loop does not take: the convolution, then the pool
     if (int r = shy_nn_conv_fwd(x, w, bias, res, y_bf16, nullptr, N, H, W, Cin, Cout, 9, relu,
                                 stream))
       return r;
