@@ -357,10 +357,13 @@ size_t wave_steps(const shy_ctx* c) {
 // Partition blocks: at most kPartMaxBlocks, each a whole number of waves of
 // drops over all log rows (the [tile][block] matrix stays small).
 constexpr int kPartMaxBlocks = 512;
-// Parts that the tiles' entries are cut into (tile_parts_kernel): two per CU,
-// and at least kPartMin entries each (a part costs a pass over its tile's
-// cells).
-constexpr int kTileParts = 512;
+// Parts that the tiles' entries are cut into (tile_parts_kernel), and at least
+// kPartMin entries each (a part costs a pass over its tile's cells).  A part is
+// a block that fills a CU, and the tiles of one part are blocks too: with 256
+// CUs, cycles in us with 512 / 448 / 384 / 320 parts: 65536 drops on 1024^2 1056
+// / 1054 / 1030 / 1037, 32768 782 / 779 / 772 / 767; 131072 on 1536^2 1852 / 1855 /
+// 1876 / 1867; 262144 on 2048^2 3824 / 3764 / 3753 / 3749.
+constexpr int kTileParts = 320;
 constexpr int kPartMin = 16384;
 
 // The partition geometry: per terrain its tiles, its blocks of dwidth drops
