@@ -45,7 +45,7 @@ __host__ __device__ inline long long pack_records(int nx, int ny) {
 // The line at 1/16: an unused index costs the tile kernels what a cell costs.
 // Measured against the x-major order, kernel times of a cycle in us: 65536
 // drops on 1024^2: scatter 229 -> 211, replay 233 -> 196, sums 233 -> 203;
-// 64 maps of 512^2 with 16384 drops each: scatter 5364 -> 4655, sums 3580 -> 3690.
+// 64 maps of 128^2 to 1024^2, 1.5 M drops: scatter 5364 -> 4655, sums 3580 -> 3690.
 struct TileMap {
   int a, b;      // log2 of the block's sides
   int nyb;       // blocks along y (x-major order: ny)

@@ -166,7 +166,7 @@ bool ordered(const shy_ctx* c) {
 // Unused LDS of a block of the walk in drop order, so that a CU holds eight
 // waves: the lanes of a wave read neighbouring records, and the waves of more
 // blocks evict them from its vector cache.  us with as many blocks of 256 threads
-// as the registers hold / 3 / 2 per CU: 64 maps of 512^2 x 16384 drops 6360 /
+// as the registers hold / 3 / 2 per CU: 64 maps of 128^2 to 1024^2 6360 /
 // 5270 / 5300, 2048^2 x 262144 1297 / 1415 / 1174, 4096^2 x 524288 3430 / 3380 /
 // 3230.  Without the order the waves share nothing (2048^2 x 196608 1718 / 1717 /
 // 1750).
@@ -764,7 +764,7 @@ int launch_cycle(shy_ctx* c, int p, hipEvent_t* ev = nullptr) {
     scan_apply_kernel<<<nbh, kScanBlock, 0, c->stream>>>(c->hist, c->hbsum, nh);
     const int mw = c->part_maxw;
     // rounds of 8192 slots fill a CU's LDS with one block; two blocks per CU with
-    // rounds of 4096 write shorter runs (64 maps of 512^2 x 16384 drops 4590 -> 4490
+    // rounds of 4096 write shorter runs (64 maps of 128^2 to 1024^2 4590 -> 4490
     // us and the sums that read the runs 2890 -> 2730, 2048^2 x 262144 1060 -> 980
     // and 590 -> 570), so they are left to terrains of more than 1024 tiles
     if (c->part_window <= 1024) {

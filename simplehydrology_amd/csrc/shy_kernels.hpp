@@ -1718,7 +1718,7 @@ __global__ void __launch_bounds__(1024) part_scatter_staged_kernel(PartArgs a) {
     // a thread's records in one tile one after another take neighbouring ranks
     // (fewer atomics, and a drop's steps lie together, whose commits
     // tile_reduce_kernel gathers from one line: ranks taken step by step gave 3690
-    // us for those sums over 64 maps of 512^2 x 16384 drops, these 2890; 2048^2 x
+    // us for those sums over 64 maps of 128^2 to 1024^2, these 2890; 2048^2 x
     // 262144 drops 679 and 588)
     int run[PER];
 #pragma unroll
