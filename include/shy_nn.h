@@ -102,16 +102,21 @@ int shy_nn_conv_wgrad_noalloc(const void* x, const void* g, float* dw, int N, in
 /* db[c] = sum over pixels of g[p][c]; part holds part_rows*C floats */
 int shy_nn_bias_grad(const void* g, float* db, float* part, int part_rows, int P, int C,
                      void* stream);
-/* dw and db of one convolution (shy_nn_conv_wgrad and shy_nn_bias_grad), in
-   one pass over g where Cin and Cout are multiples of 32, taps = 9 and
-   part_splits > 1 */
+/* dw and db of one convolution: shy_nn_conv_wgrad and shy_nn_bias_grad, the
+   same bits, in two launches where Cin and Cout are multiples of 32 and taps = 9 */
 int shy_nn_conv_wgrad_bias(const void* x, const void* g, float* dw, float* db, float* part,
                            int part_splits, float* bias_part, int bias_rows, int N, int H, int W,
                            int Cin, int Cout, int taps, void* stream);
 /* The same of a convolution of [up2(x_half), skip] along channels (C1 + C2),
-   read from the two tensors (shy_nn_conv_fwd_upcat's input).  H, W even; C1,
-   C2, Cout multiples of 32; part holds part_splits*Cout*9*(C1+C2) floats,
-   part_splits > 1. */
+   read from the two tensors (shy_nn_conv_fwd_upcat's input): the bits of the
+   gradients of the concatenated input.  H, W even; C1, C2, Cout multiples of 32,
+   Cout <= 1024; part holds part_splits*Cout*9*(C1+C2) floats; g and bias_part
+   16-byte aligned. */
+int shy_nn_conv_wgrad_bias_cat(const void* x_half, const void* skip, const void* g, float* dw,
+                               float* db, float* part, int part_splits, float* bias_part,
+                               int bias_rows, int N, int H, int W, int C1, int C2, int Cout,
+                               void* stream);
+/* The same without bias_part: part serves for both, one after the other */
 int shy_nn_conv_wgrad_bias_upcat(const void* x_half, const void* skip, const void* g, float* dw,
                                  float* db, float* part, int part_splits, int N, int H, int W,
                                  int C1, int C2, int Cout, void* stream);

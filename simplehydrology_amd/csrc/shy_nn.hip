@@ -31,8 +31,8 @@
 //   conv_wgrad_kernel  staged through LDS (both operands need 8 consecutive
 //                      pixels per lane: transposed LDS reads; the second loads
 //                      directly), split over pixel ranges into FP32 partials
-//                      that wgrad_reduce_kernel sums in a fixed order; the first
-//                      sums the bias gradient from the same tiles
+//                      that wgrad_reduce_kernel sums in a fixed order; both
+//                      launches of the first take the bias gradient along
 //   elementwise        ReLU backward, 2x2 average pool, nearest upsample,
 //                      channel concat/split, the fused passes between two
 //                      stages of the backward, bias gradient, MSE loss, Adam
@@ -869,34 +869,40 @@ __global__ void __launch_bounds__(64) conv_wgrad_kernel(WgradArgs a) {
 }
 
 // Weight gradient for Cin and Cout multiples of 32, TAPS = 9, staged through
-// LDS: dW[co][tap*Cin + ci] = sum_p g[p][co] x[p + tap][ci], and with a.bias
-// the bias gradient sum_p g[p][co] from the same tiles (a product with ones).
+// LDS: dW[co][tap*Cin + ci] = sum_p g[p][co] x[p + tap][ci]; its last blocks
+// take the partials of the bias gradient sum_p g[p][co] (bias_partial).
 // The reduction runs over pixels, so both MFMA operands need 8 pixels of one
-// channel per lane, while the tiles lie pixel by pixel: G [4 rows][32 pixels][co]
-// and X [6 rows][34 pixels][32 ci] (the 1-pixel halo).  They are staged as they
-// lie, and ds_read_b64_tr_b16 transposes while reading: each 16 lanes give four
-// pixels x 16 channels, lane j receives channel j of the four.  A tap's shift is
-// then only an address, also for odd columns.
-// A block owns 32*MTW output channels x 32 input channels x all 9 taps; wave w
-// the input channels 16*(w%2).. and the output channels of half w/2.  It goes
-// down the rows of X: a row's three column shifts are read once and serve the
-// three rows of G around it, which stay in registers (3 + MTW fragments read for
-// 9*MTW products; reading both operands for every tap cost 12 for 10, and the
-// LDS reads, not the matrix cores, bounded the kernel).  The next tile's
-// global loads are in flight meanwhile; off-image pixels are loaded from the
-// image's first pixel and stored as zeros, so no load depends on a branch.
-// Measured against tiles stored transposed and the shifts realigned in
-// registers, without the loads ahead: 16 x 32 x 32, 128 -> 128 channels 26.8 ->
-// 15.3 us; the launches of a training step of 16 windows of 256^2 81 -> 37 us on
-// average, and 22 launches of the bias kernels less.
-constexpr int kWgTW = 32, kWgTH = 4, kWgPix = kWgTW * kWgTH;
+// channel per lane, while the tiles lie pixel by pixel: G [8 rows][16 pixels]
+// [32 co] and X [10 rows][18 pixels][32 ci] (the 1-pixel halo).  They are staged
+// as they lie, and ds_read_b64_tr_b16 transposes while reading: each 16 lanes
+// give four pixels x 16 channels, lane j receives channel j of the four.  A tap's
+// shift is then only an address, also for odd columns.
+// The order of the sums is part of the results: FP32 sums in another order are
+// as accurate, but Adam divides each gradient by its own size, so that from a
+// difference of 1e-7 a few steps of training lead to other BF16 weights.  An
+// element's products are added two rows of 16 pixels (one MFMA) after the other, tile
+// by tile of 16 x 8 pixels, over a range of tiles that follows from the shape and
+// the partials given; no tile shape, block shape or staging may change that.
+// A block owns 32 output channels x 32 input channels x all 9 taps; a wave the
+// taps of one column shift and 16 input channels.  It goes down the rows of X: the
+// two rows from row j on serve the taps (s, dy) with 2 s + dy = j, so every pair of
+// rows is read once (17 fragments for 24 products; a wave per 16 x 16 channels and
+// nine taps would read 31 for 36).  While a tile is multiplied, the next one comes
+// from memory into registers and from there into the other half of LDS: one
+// barrier a tile.  Off-image pixels are loaded from the image's first pixel and
+// stored as zeros, so no load depends on a branch.
+// A layer's launches, bias gradient and sums of the partials included, in us at
+// batch 16: tiles stored transposed, without loads ahead and with launches for
+// the bias / these with 3 waves of 32 input channels / 6 of 16 / 6 and two halves
+// of LDS: 256^2 32 -> 32 channels 95.8 / 53.1 / 48.8 / 49.8, 256^2 96 -> 32 264 / 117 / 105
+// / 102, 128^2 64 -> 64 101 / 48.7 / 46.8 / 41.1, 128^2 160 -> 64 221 / 98.7 / 91.6 /
+// 83.5, 64^2 224 -> 96 125 / 56.3 / 52.3 / 50.5, 32^2 128 -> 128 48.2 / 24.4 / 23.2 / 22.9.
+// (The bias blocks first in the grid: 128^2 64 -> 64 51.0.)
+constexpr int kWgTW = 16, kWgTH = 8, kWgPix = kWgTW * kWgTH;
 constexpr int kWgXW = kWgTW + 2, kWgXPix = kWgXW * (kWgTH + 2);
-// Blocks of a launch: two per CU, which all run at once (64 output channels
-// per block fit two).  Training step, us per launch of blocks of 64 / of 32
-// channels / of the partials' sum: 256 blocks' worth of partials 42 / 42 / 6.1,
-// 512 29 / 43 / 6.8, 768 35 / 43 / 8.1, 1024 35 / 47 / 9.0.
-constexpr int kWgBlocks = 512;
-constexpr int kWgXS = 32 + 8;  // halfwords per pixel of X; 16 pixels cover the banks evenly
+constexpr int kWgThreads = 384;  // a wave per column shift and 16 input channels
+constexpr int kWgS = 32 + 8;     // halfwords per pixel in LDS; 16 pixels cover the banks evenly
+constexpr int kWgHalf = (kWgPix + kWgXPix) * kWgS;  // a tile's, 24640 bytes
 
 struct WgArgs {
   // the input: x [N][H][W][Cin], or (C1 > 0) its channels below C1 from x
@@ -905,55 +911,101 @@ struct WgArgs {
   const __bf16* __restrict__ x2;
   int C1;
   const __bf16* __restrict__ g;
-  float* part;  // [splits][Cout*K (+ Cout with bias)]
+  float* part;  // [splits][Cout*K]
   int N, H, W, Cin, Cout, K;
-  int bias;
   int tiles_x, tiles_y, tiles;
   int tiles_per_split;
+  int blocks;            // of the weight gradient; those after it sum the bias gradient
+  float* bias_part;      // [ranges of bias_rows pixels][Cout]
+  int bias_rows;
 };
 
+// bias_grad_v8_kernel's partial of range b of rows_per_block pixels, 32 channels
+// from c0 on, by a block of NT threads: the same sums in the same order
+// (thread t takes the work of that kernel's threads t, t + NT, ... of these
+// channels).  acc: 8192 floats of LDS.
+template <int NT>
+__device__ inline void bias_partial(const __bf16* __restrict__ g, float* part, int P, int C,
+                                    int rows_per_block, int b, int c0, float* acc) {
+  const int groups = 1024 / (C / 8);
+  const int p0 = b * rows_per_block, p1 = min(P, p0 + rows_per_block);
+  for (int v = threadIdx.x; v < 4 * groups; v += NT) {
+    const int r = v >> 2;
+    const __bf16* gc = g + c0 + 8 * (v & 3);
+    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int p = p0 + r;
+    for (; p + 7 * groups < p1; p += 8 * groups) {
+      bf16x8 x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = load8(gc + (size_t)(p + u * groups) * C);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s[k] += (float)x[u][k];
+    }
+    for (; p < p1; p += groups) {
+      const bf16x8 x = load8(gc + (size_t)p * C);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s[k] += (float)x[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[v * 8 + k] = s[k];
+  }
+  __syncthreads();
+  for (int n = groups; n > 1;) {
+    const int h = (n + 1) / 2;
+    for (int i = threadIdx.x; i < (n - h) * 32; i += NT) acc[i] += acc[h * 32 + i];
+    __syncthreads();
+    n = h;
+  }
+  if (threadIdx.x < 32) part[(size_t)b * C + c0 + threadIdx.x] = acc[threadIdx.x];
+}
+
 // 8 pixels of one channel: p = this lane's 4 channels of its pixel of the
-// first four, stride halfwords per pixel
-__device__ inline bf16x8 read_pixels8(const __bf16* p, int stride) {
+// first four
+__device__ inline bf16x8 read_pixels8(const __bf16* p) {
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   typedef short s16x8 __attribute__((ext_vector_type(8)));
   typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
   const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * stride));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * kWgS));
   return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int MTW>
-__global__ void __launch_bounds__(256) wgrad_lds_kernel(WgArgs a) {
-  constexpr int NCO = 32 * MTW;
-  constexpr int GS = NCO + 8;
-  constexpr int RG = kWgPix * (NCO / 8) / 256, RX = (kWgXPix * 4 + 255) / 256;
-  __shared__ __align__(16) __bf16 gt[kWgPix * GS];
-  __shared__ __align__(16) __bf16 xt[kWgXPix * kWgXS];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+__global__ void __launch_bounds__(kWgThreads) wgrad_lds_kernel(WgArgs a) {
+  constexpr int NT = kWgThreads;
+  constexpr int RG = (kWgPix * 4 + NT - 1) / NT, RX = (kWgXPix * 4 + NT - 1) / NT;
+  __shared__ __align__(16) float lds[kWgHalf];  // two halves, or bias_partial's floats
+  static_assert(kWgHalf >= 8192, "bias_partial's floats");
+  __bf16* gt = reinterpret_cast<__bf16*>(lds);
+  __bf16* xt = gt + kWgPix * kWgS;
+  if ((int)blockIdx.x >= a.blocks) {
+    const int b = (int)blockIdx.x - a.blocks, nc = a.Cout / 32;
+    bias_partial<NT>(a.g, a.bias_part, a.N * a.H * a.W, a.Cout, a.bias_rows, b / nc, b % nc * 32,
+                     lds);
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, dx = wave % 3, cw = wave / 3 * 16;
   const int Cin = a.Cin, Cout = a.Cout;
   // Workgroups go round-robin over the 8 XCDs: the channel blocks of one
   // range of tiles, which read the same g and x, follow each other on one XCD
   // and share its L2 (training step: 96 -> 96 channels at 64^2 31 -> 23.5 us)
-  const int nco = Cout / NCO, nch = nco * (Cin / 32), seq = (int)blockIdx.x >> 3;
+  const int nco = Cout / 32, nch = nco * (Cin / 32), seq = (int)blockIdx.x >> 3;
   const int split = seq / nch * 8 + ((int)blockIdx.x & 7), ch = seq % nch;
-  const int cb = ch % nco * NCO, ci0 = ch / nco * 32;
+  const int cb = ch % nco * 32, ci0 = ch / nco * 32;
   const int t_begin = split * a.tiles_per_split;
   const int t_end = min(a.tiles, t_begin + a.tiles_per_split);
   if (t_begin >= t_end) return;  // uniform over the block
-  const bool bias = a.bias && ci0 == 0 && (wave & 1) == 0;  // uniform over the wave
   // where this block's input channels lie
   const int up = ci0 < a.C1 ? 1 : 0;
   const __bf16* src = a.C1 > 0 && !up ? a.x2 : a.x;
   const int srcH = a.H >> up, srcW = a.W >> up;
   const int srcC = up ? a.C1 : Cin - a.C1, srcc = up ? ci0 : ci0 - a.C1;
-  f32x4 acc[9][MTW], accb[MTW];
+  f32x4 acc[3][2];  // [tap row][half of the output channels]
 #pragma unroll
-  for (int m = 0; m < MTW; ++m) {
-    accb[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
-    for (int t = 0; t < 9; ++t) acc[t][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  }
+    for (int m = 0; m < 2; ++m) acc[dy][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   bf16x8 rg[RG], rx[RX];
   uint32_t okg = 0, okx = 0;
   auto gload = [&](int t) {
@@ -965,91 +1017,79 @@ __global__ void __launch_bounds__(256) wgrad_lds_kernel(WgArgs a) {
     okg = okx = 0;
 #pragma unroll
     for (int j = 0; j < RG; ++j) {
-      const int v = threadIdx.x + 256 * j, pix = v / (NCO / 8), q = v % (NCO / 8);
+      const int v = threadIdx.x + NT * j, pix = v >> 2, q = v & 3;
       const int gy = y0 + pix / kWgTW, gx = x0 + pix % kWgTW;
-      const bool ok = gy < a.H && gx < a.W;
+      const bool ok = v < kWgPix * 4 && gy < a.H && gx < a.W;
       okg |= ok ? 1u << j : 0u;
       rg[j] = load8(gi + (ok ? ((size_t)gy * a.W + gx) * Cout : 0) + q * 8);
     }
 #pragma unroll
     for (int j = 0; j < RX; ++j) {
-      const int v = threadIdx.x + 256 * j, pix = v >> 2, q = v & 3;
+      const int v = threadIdx.x + NT * j, pix = v >> 2, q = v & 3;
       const int gy = y0 + pix / kWgXW - 1, gx = x0 + pix % kWgXW - 1;
       const bool ok = v < kWgXPix * 4 && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W;
       okx |= ok ? 1u << j : 0u;
       rx[j] = load8(xi + (ok ? ((size_t)(gy >> up) * srcW + (gx >> up)) * srcC : 0) + q * 8);
     }
   };
-  auto lstore = [&]() {
+  // into the half of LDS from halfword o on
+  auto lstore = [&](int o) {
 #pragma unroll
     for (int j = 0; j < RG; ++j) {
-      const int v = threadIdx.x + 256 * j, pix = v / (NCO / 8), q = v % (NCO / 8);
-      *reinterpret_cast<bf16x8*>(&gt[pix * GS + q * 8]) = okg >> j & 1 ? rg[j] : zero8();
+      const int v = threadIdx.x + NT * j;
+      if (v < kWgPix * 4)
+        *reinterpret_cast<bf16x8*>(&gt[o + (v >> 2) * kWgS + (v & 3) * 8]) =
+            okg >> j & 1 ? rg[j] : zero8();
     }
 #pragma unroll
     for (int j = 0; j < RX; ++j) {
-      const int v = threadIdx.x + 256 * j;
+      const int v = threadIdx.x + NT * j;
       if (v < kWgXPix * 4)
-        *reinterpret_cast<bf16x8*>(&xt[(v >> 2) * kWgXS + (v & 3) * 8]) =
+        *reinterpret_cast<bf16x8*>(&xt[o + (v >> 2) * kWgS + (v & 3) * 8]) =
             okx >> j & 1 ? rx[j] : zero8();
     }
   };
-  // this lane's pixel of a row's first 4 of 8 (k group lane/16) and its 4 channels
-  const int pix0 = (lane >> 4) * 8 + ((lane & 15) >> 2), ch0 = (lane & 3) * 4;
-  const __bf16* gl = &gt[pix0 * GS + (wave >> 1) * 16 * MTW + ch0];
-  const __bf16* xl = &xt[pix0 * kWgXS + (wave & 1) * 16 + ch0];
-  bf16x8 ones;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.0f;
+  // An MFMA's 32 pixels are two rows of 16; lane group lane/16 holds 8 of them:
+  // row group/2, columns 8 (group % 2) on.  This lane's pixel of the first 4 of
+  // the 8, and its 4 channels:
+  const int grp = lane >> 4, p4 = (lane & 15) >> 2, ch0 = (lane & 3) * 4;
+  const __bf16* gl = &gt[(grp * 8 + p4) * kWgS + ch0];
+  const __bf16* xl = &xt[((grp >> 1) * kWgXW + (grp & 1) * 8 + p4 + dx) * kWgS + cw + ch0];
   gload(t_begin);
+  lstore(0);
+  int o = 0;
   for (int t = t_begin; t < t_end; ++t) {
-    lstore();
+    // tile t is in LDS, and the other half is no longer read
     __syncthreads();
     if (t + 1 < t_end) gload(t + 1);
-    bf16x8 A[3][MTW];
+    bf16x8 B[3];  // the pair of X rows from row 2 s + dy on
 #pragma unroll
-    for (int j = 0; j < kWgTH + 2; ++j) {
-      if (j < kWgTH) {
+    for (int s = 0; s < kWgTH / 2; ++s) {
+      bf16x8 A[2];
 #pragma unroll
-        for (int m = 0; m < MTW; ++m)
-          A[j % 3][m] = read_pixels8(gl + j * kWgTW * GS + m * 16, GS);
-        if (bias)
-#pragma unroll
-          for (int m = 0; m < MTW; ++m) accb[m] = mfma(A[j % 3][m], ones, accb[m]);
-      }
-      bf16x8 B[3];
-#pragma unroll
-      for (int dx = 0; dx < 3; ++dx)
-        B[dx] = read_pixels8(xl + (j * kWgXW + dx) * kWgXS, kWgXS);
-      // X row j (image row y0 - 1 + j) under tap row dy meets G row j - dy
+      for (int m = 0; m < 2; ++m) A[m] = read_pixels8(gl + o + s * 32 * kWgS + m * 16);
 #pragma unroll
       for (int dy = 0; dy < 3; ++dy) {
-        if (j - dy < 0 || j - dy >= kWgTH) continue;
+        if (s > 0 && dy == 0)
+          B[0] = B[2];  // read as the last pair of the step before
+        else
+          B[dy] = read_pixels8(xl + o + (2 * s + dy) * kWgXW * kWgS);
 #pragma unroll
-        for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-          for (int m = 0; m < MTW; ++m)
-            acc[dy * 3 + dx][m] = mfma(A[(j - dy) % 3][m], B[dx], acc[dy * 3 + dx][m]);
+        for (int m = 0; m < 2; ++m) acc[dy][m] = mfma(A[m], B[dy], acc[dy][m]);
       }
     }
-    __syncthreads();
+    o ^= kWgHalf;
+    if (t + 1 < t_end) lstore(o);
   }
-  const size_t per = (size_t)Cout * a.K + (a.bias ? Cout : 0);
-  float* out = a.part + (size_t)split * per;
-  const int co0 = cb + (wave >> 1) * 16 * MTW + (lane >> 4) * 4;
-  const int k0 = ci0 + (wave & 1) * 16 + (lane & 15);
+  float* out = a.part + (size_t)split * Cout * a.K;
+  const int co0 = cb + (lane >> 4) * 4, k0 = ci0 + cw + (lane & 15);
 #pragma unroll
-  for (int t = 0; t < 9; ++t)
+  for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
-    for (int m = 0; m < MTW; ++m)
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        out[(size_t)(co0 + m * 16 + i) * a.K + t * Cin + k0] = acc[t][m][i];
-  if (bias && (lane & 15) == 0)
-#pragma unroll
-    for (int m = 0; m < MTW; ++m)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) out[(size_t)Cout * a.K + co0 + m * 16 + i] = accb[m][i];
+        out[(size_t)(co0 + m * 16 + i) * a.K + (dy * 3 + dx) * Cin + k0] = acc[dy][m][i];
 }
 
 // dW[i] = sum over splits of part[k][i] in a fixed order (deterministic):
@@ -1058,10 +1098,43 @@ __global__ void __launch_bounds__(256) wgrad_lds_kernel(WgArgs a) {
 // and give every output 8 independent chains.
 constexpr int kRedSlices = 8;
 
+// db[c0 .. c0 + 7] from the bias partials part [nb][C], by a block of 256
+// threads: bias_reduce_kernel's sums in their order.  C >= 32.
+__device__ inline void bias_reduce8(const float* __restrict__ part, float* db, int C, int nb,
+                                    int c0) {
+  __shared__ float acc[256 * 8];
+  const int groups = 1024 / (C / 8), r = threadIdx.x;
+  if (r < groups) {
+    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int b = r; b < nb; b += groups) {
+      const float4* q = reinterpret_cast<const float4*>(part + (size_t)b * C + c0);
+      const float4 v0 = q[0], v1 = q[1];
+      s[0] += v0.x; s[1] += v0.y; s[2] += v0.z; s[3] += v0.w;
+      s[4] += v1.x; s[5] += v1.y; s[6] += v1.z; s[7] += v1.w;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc[r * 8 + k] = s[k];
+  }
+  __syncthreads();
+  for (int n = groups; n > 1;) {
+    const int h = (n + 1) / 2;
+    for (int i = r; i < (n - h) * 8; i += 256) acc[i] += acc[h * 8 + i];
+    __syncthreads();
+    n = h;
+  }
+  if (r < 8) db[c0 + r] = acc[r];
+}
+
 __global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float* __restrict__ part,
-                                                           float* dw, float* db, int nw, int n,
-                                                           int splits) {
+                                                           float* dw, int n, int splits,
+                                                           const float* __restrict__ bias_part,
+                                                           float* db, int C, int nb) {
   __shared__ float acc[kRedSlices][32];
+  const int blocks = (n + 31) / 32;  // the ones after them: 8 channels of db each
+  if ((int)blockIdx.x >= blocks) {
+    bias_reduce8(bias_part, db, C, nb, ((int)blockIdx.x - blocks) * 8);
+    return;
+  }
   const int e = threadIdx.x & 31, sl = threadIdx.x >> 5;
   const int i = blockIdx.x * 32 + e;
   float s = 0.0f;
@@ -1083,10 +1156,7 @@ __global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float* __restri
     float t = 0.0f;
 #pragma unroll
     for (int q = 0; q < kRedSlices; ++q) t += acc[q][e];
-    if (i < nw)
-      dw[i] = t;
-    else
-      db[i - nw] = t;
+    dw[i] = t;
   }
 }
 
@@ -1986,11 +2056,20 @@ int shy_nn_flip_weights(const void* w, void* wf, int Cin, int Cout, int taps, vo
   return nn_check("flip_weights");
 }
 
-// The weight gradient by wgrad_lds_kernel, and with db the bias gradient of
-// the same pass; part holds cap floats.
-static int wgrad_lds(const void* x, const void* x2, int C1, const void* g, float* dw, float* db,
-                     float* part, size_t cap, int N, int H, int W, int Cin, int Cout,
-                     hipStream_t s) {
+inline bool a16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// pixels per partial of shy_nn_bias_grad: at least 2048 (two 1024-thread blocks
+// per CU on the largest layers, eight rows in flight per thread)
+static int bias_rows_per_block(int P, int part_rows) {
+  return std::max((P + part_rows - 1) / part_rows, 2048);
+}
+
+// The weight gradient by wgrad_lds_kernel, of x or (C1 > 0) [up2(x), x2];
+// part holds part_splits partials.  With db the bias gradient too, bias_part
+// holding bias_rows partials.
+static int wgrad_lds(const void* x, const void* x2, int C1, const void* g, float* dw, float* part,
+                     int part_splits, float* db, float* bias_part, int bias_rows, int N, int H,
+                     int W, int Cin, int Cout, hipStream_t s) {
   WgArgs b;
   b.x = (const __bf16*)x;
   b.x2 = (const __bf16*)x2;
@@ -1998,29 +2077,32 @@ static int wgrad_lds(const void* x, const void* x2, int C1, const void* g, float
   b.g = (const __bf16*)g;
   b.part = part;
   b.N = N; b.H = H; b.W = W; b.Cin = Cin; b.Cout = Cout; b.K = 9 * Cin;
-  b.bias = db != nullptr;
   b.tiles_x = (W + kWgTW - 1) / kWgTW;
   b.tiles_y = (H + kWgTH - 1) / kWgTH;
   const long long tiles = (long long)N * b.tiles_x * b.tiles_y;
   if (tiles > INT32_MAX) return nn_fail("conv_wgrad: too many tiles");
   b.tiles = (int)tiles;
-  const int mtw = Cout % 64 == 0 ? 2 : 1;
-  const int bxy = (Cout / (32 * mtw)) * (Cin / 32);
-  const int nw = Cout * b.K, n = nw + (db ? Cout : 0);
-  // at most kWgBlocks blocks (one more is a second pass over the CUs: 520 blocks
-  // 94 us for 160 -> 64 channels at 128^2, 480 67) and equally many on every XCD, as many partials as part holds, at least one tile each
-  const int most = kWgBlocks / bxy;
-  long long splits = std::min<long long>(most >= 8 ? most / 8 * 8 : std::max(most, 1), tiles);
-  splits = std::min<long long>(splits, (long long)(cap / (size_t)n));
+  const int bxy = (Cout / 32) * (Cin / 32);
+  // about 1024 blocks, at most part_splits partials, at least one tile each;
+  // the ranges of tiles are part of the order of the sums (wgrad_lds_kernel)
+  long long splits = std::max(1LL, std::min<long long>((1024 + bxy - 1) / bxy, tiles));
+  splits = std::min<long long>(splits, part_splits);
   b.tiles_per_split = (int)((tiles + splits - 1) / splits);
   splits = (tiles + b.tiles_per_split - 1) / b.tiles_per_split;
-  const unsigned grid = (unsigned)((splits + 7) / 8 * 8 * bxy);
-  if (mtw == 2)
-    wgrad_lds_kernel<2><<<grid, 256, 0, s>>>(b);
-  else
-    wgrad_lds_kernel<1><<<grid, 256, 0, s>>>(b);
+  b.blocks = (int)((splits + 7) / 8 * 8 * bxy);  // equally many on every XCD
+  b.bias_part = bias_part;
+  b.bias_rows = 0;
+  int nb = 0;
+  if (db) {
+    const int P = N * H * W;
+    b.bias_rows = bias_rows_per_block(P, bias_rows);
+    nb = (P + b.bias_rows - 1) / b.bias_rows;
+  }
+  wgrad_lds_kernel<<<(unsigned)(b.blocks + nb * (Cout / 32)), kWgThreads, 0, s>>>(b);
   if (int r = nn_check("conv_wgrad")) return r;
-  wgrad_reduce_kernel<<<(n + 31) / 32, 256, 0, s>>>(part, dw, db, nw, n, (int)splits);
+  const int n = Cout * b.K;
+  wgrad_reduce_kernel<<<(n + 31) / 32 + (db ? Cout / 8 : 0), 256, 0, s>>>(
+      part, dw, n, (int)splits, bias_part, db, Cout, nb);
   return nn_check("wgrad_reduce");
 }
 
@@ -2030,7 +2112,7 @@ int shy_nn_conv_wgrad(const void* x, const void* g, float* dw, float* part, int 
   if (Cin % 8 || Cout % 8 || (taps != 9 && taps != 1)) return nn_fail("conv_wgrad: channels must be multiples of 8");
   const long long P = (long long)N * H * W;
   if (taps == 9 && Cin % 32 == 0 && Cout % 32 == 0)
-    return wgrad_lds(x, nullptr, 0, g, dw, nullptr, part, (size_t)part_splits * Cout * 9 * Cin, N, H, W, Cin,
+    return wgrad_lds(x, nullptr, 0, g, dw, part, part_splits, nullptr, nullptr, 0, N, H, W, Cin,
                      Cout, (hipStream_t)stream);
   int chunk = (int)((P + part_splits - 1) / part_splits);
 
@@ -2047,7 +2129,7 @@ int shy_nn_conv_wgrad(const void* x, const void* g, float* dw, float* part, int 
   conv_wgrad_kernel<<<grid, 64, 0, s>>>(a);
   if (int r = nn_check("conv_wgrad")) return r;
   const int n = Cout * a.K;
-  wgrad_reduce_kernel<<<(n + 31) / 32, 256, 0, s>>>(part, dw, nullptr, n, n, splits);
+  wgrad_reduce_kernel<<<(n + 31) / 32, 256, 0, s>>>(part, dw, n, splits, nullptr, nullptr, 0, 0);
   return nn_check("wgrad_reduce");
 }
 
@@ -2072,9 +2154,7 @@ int shy_nn_bias_grad(const void* g, float* db, float* part, int part_rows, int P
     return nn_fail("bias_grad: bad argument");
   hipStream_t s = (hipStream_t)stream;
   if (C % 8 == 0 && ((uintptr_t)g & 15) == 0 && ((uintptr_t)part & 15) == 0) {
-    // at least 2048 pixels per block (two 1024-thread blocks per CU on the
-    // largest layers, eight rows in flight per thread)
-    const int rows = std::max((P + part_rows - 1) / part_rows, 2048);
+    const int rows = bias_rows_per_block(P, part_rows);
     const int nb = (P + rows - 1) / rows;
     bias_grad_v8_kernel<<<nb, 1024, 0, s>>>((const __bf16*)g, part, P, C, rows);
     if (int r = nn_check("bias_grad")) return r;
@@ -2085,23 +2165,39 @@ int shy_nn_bias_grad(const void* g, float* db, float* part, int part_rows, int P
   const int nb = (P + rows - 1) / rows;
   bias_grad_kernel<<<nb, 256, 0, s>>>((const __bf16*)g, part, P, C, rows);
   if (int r = nn_check("bias_grad")) return r;
-  wgrad_reduce_kernel<<<(C + 31) / 32, 256, 0, s>>>(part, db, nullptr, C, C, nb);
+  wgrad_reduce_kernel<<<(C + 31) / 32, 256, 0, s>>>(part, db, C, nb, nullptr, nullptr, 0,
+                                                     0);
   return nn_check("bias_grad_reduce");
 }
 
 int shy_nn_conv_wgrad_bias(const void* x, const void* g, float* dw, float* db, float* part,
                            int part_splits, float* bias_part, int bias_rows, int N, int H, int W,
                            int Cin, int Cout, int taps, void* stream) {
-  // one pass over g gives both where the weight gradient stages it by tiles and
-  // part has room for the bias sums beside the weights'
-  if (x && g && dw && db && part && part_splits > 1 && taps == 9 && Cin > 0 && Cout > 0 &&
-      Cout <= 1024 &&  // as shy_nn_bias_grad
-      Cin % 32 == 0 && Cout % 32 == 0)
-    return wgrad_lds(x, nullptr, 0, g, dw, db, part, (size_t)part_splits * Cout * 9 * Cin, N, H, W,
+  // the tiled weight gradient's launches take the bias sums along, where these
+  // are shy_nn_bias_grad's 8-channel ones
+  const long long P = (long long)N * H * W;
+  if (x && g && dw && db && part && part_splits > 0 && bias_part && bias_rows > 0 && taps == 9 &&
+      Cin > 0 && Cout > 0 && Cout <= 1024 && Cin % 32 == 0 && Cout % 32 == 0 && P > 0 &&
+      P <= INT32_MAX && a16(g) && a16(bias_part))
+    return wgrad_lds(x, nullptr, 0, g, dw, part, part_splits, db, bias_part, bias_rows, N, H, W,
                      Cin, Cout, (hipStream_t)stream);
   if (int r = shy_nn_conv_wgrad(x, g, dw, part, part_splits, N, H, W, Cin, Cout, taps, stream))
     return r;
   return shy_nn_bias_grad(g, db, bias_part, bias_rows, N * H * W, Cout, stream);
+}
+
+int shy_nn_conv_wgrad_bias_cat(const void* x_half, const void* skip, const void* g, float* dw,
+                               float* db, float* part, int part_splits, float* bias_part,
+                               int bias_rows, int N, int H, int W, int C1, int C2, int Cout,
+                               void* stream) {
+  if (!x_half || !skip || !g || !dw || !db || !part || part_splits < 1 || !bias_part ||
+      bias_rows < 1 || !a16(g) || !a16(bias_part))
+    return nn_fail("conv_wgrad_bias_cat: bad pointers");
+  if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || C1 < 32 || C1 % 32 || C2 < 32 || C2 % 32 ||
+      Cout < 32 || Cout % 32 || Cout > 1024 || (long long)N * H * W > INT32_MAX)
+    return nn_fail("conv_wgrad_bias_cat: need H, W even and C1, C2, Cout multiples of 32");
+  return wgrad_lds(x_half, skip, C1, g, dw, part, part_splits, db, bias_part, bias_rows, N, H, W,
+                   C1 + C2, Cout, (hipStream_t)stream);
 }
 
 int shy_nn_conv_wgrad_bias_upcat(const void* x_half, const void* skip, const void* g, float* dw,
@@ -2110,13 +2206,15 @@ int shy_nn_conv_wgrad_bias_upcat(const void* x_half, const void* skip, const voi
   if (!x_half || !skip || !g || !dw || !db || !part || part_splits < 2)
     return nn_fail("conv_wgrad_bias_upcat: bad pointers, or fewer than two partials");
   if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || C1 < 32 || C1 % 32 || C2 < 32 || C2 % 32 ||
-      Cout < 32 || Cout % 32 || Cout > 1024)
+      Cout < 32 || Cout % 32 || Cout > 1024 || (long long)N * H * W > INT32_MAX)
     return nn_fail("conv_wgrad_bias_upcat: need H, W even and C1, C2, Cout multiples of 32");
-  return wgrad_lds(x_half, skip, C1, g, dw, db, part, (size_t)part_splits * Cout * 9 * (C1 + C2), N,
-                   H, W, C1 + C2, Cout, (hipStream_t)stream);
+  // the bias partials first, in the memory of the others (at least 576 Cout
+  // floats)
+  const size_t rows = std::min<size_t>(1024, (size_t)part_splits * 9 * (C1 + C2));
+  if (int r = shy_nn_bias_grad(g, db, part, (int)rows, N * H * W, Cout, stream)) return r;
+  return wgrad_lds(x_half, skip, C1, g, dw, part, part_splits, nullptr, nullptr, 0, N, H, W,
+                   C1 + C2, Cout, (hipStream_t)stream);
 }
-
-inline bool a16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 int shy_nn_relu_bwd(const void* y, const void* g, void* out, size_t n, void* stream) {
   if (n % 8 == 0 && a16(y) && a16(g) && a16(out))

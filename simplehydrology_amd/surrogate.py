@@ -56,6 +56,8 @@ def nn():
             "shy_nn_conv_wgrad_noalloc": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
             "shy_nn_conv_wgrad_bias": (i32, [vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32,
                                              i32, i32, vp]),
+            "shy_nn_conv_wgrad_bias_cat": (i32, [vp, vp, vp, vp, vp, vp, i32, vp, i32, i32, i32,
+                                                 i32, i32, i32, i32, vp]),
             "shy_nn_conv_wgrad_bias_upcat": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32,
                                                    i32, i32, vp]),
             "shy_nn_up2_bwd_relu": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]),
@@ -237,10 +239,11 @@ class Conv:
         part, splits = scratch.part_for(self, P)
         if isinstance(x, tuple):
             xh, skip = x
-            _ck(nn().shy_nn_conv_wgrad_bias_upcat(_p(xh), _p(skip), _p(g), _p(self.dw),
-                                                  _p(self.db), _p(part), splits, N, H, W,
-                                                  xh.shape[-1], skip.shape[-1], self.cout,
-                                                  _stream()))
+            _ck(nn().shy_nn_conv_wgrad_bias_cat(_p(xh), _p(skip), _p(g), _p(self.dw),
+                                                _p(self.db), _p(part), splits,
+                                                _p(scratch.bias_part), scratch.bias_rows, N, H, W,
+                                                xh.shape[-1], skip.shape[-1], self.cout,
+                                                _stream()))
         else:
             _ck(nn().shy_nn_conv_wgrad_bias(_p(x), _p(g), _p(self.dw), _p(self.db), _p(part),
                                             splits, _p(scratch.bias_part), scratch.bias_rows, N, H,
@@ -286,12 +289,10 @@ class Scratch:
         self.bias_part = torch.empty(self.bias_rows * 1024, dtype=torch.float32, device=device)
 
     def part_for(self, conv, P):
-        fit = self.part.numel() // (conv.cout * conv.taps * conv.cin)
-        if conv.taps == 9 and conv.cin % 32 == 0 and conv.cout % 32 == 0:
-            return self.part, max(1, fit)  # an upper bound: the library splits by its grid
         tiles = ((conv.cout + 31) // 32) * ((conv.taps * conv.cin + 31) // 32)
         splits = max(1, min(P // 512, -(-4096 // tiles)))
-        return self.part, max(1, min(splits, fit))
+        splits = min(splits, self.part.numel() // (conv.cout * conv.taps * conv.cin))
+        return self.part, max(1, splits)
 
 
 def _relu_bwd(y, g):
