@@ -59,10 +59,11 @@ int shy_nn_conv_fwd_pool(const void* x, const void* w, const float* bias, const 
 /* The whole 4-level residual U-Net of surrogate.py, inference only: its 22
    convolutions' weights w (BF16, the layouts above) and biases b in the order
    encoder stages of levels 0..3, decoder stages of levels 0..2 (three each),
-   head; x [N][H][W][cin], ch[4] the levels' channels (ch[0] 32 or 64, a
-   multiple of 32 each), out [N][H][W][head_c] FP32.  H, W multiples of 8.  The
-   tables are read during the call.  work holds at least
-   shy_nn_unet_work_bytes(ch, N, H, W) bytes. */
+   head; x [N][H][W][cin], cin a multiple of 8; ch[4] the levels' channels:
+   ch[0] = 32, the others multiples of 32; out [N][H][W][head_c] FP32, head_c in
+   {4, 8, 12, 16}.  H, W multiples of 8.  The tables are read during the call.
+   work holds at least shy_nn_unet_work_bytes(ch, N, H, W) bytes (-1: a channel
+   or side that the network does not take). */
 long long shy_nn_unet_work_bytes(const int* ch, int N, int H, int W);
 int shy_nn_unet_forward(const void* x, const void* const* w, const float* const* b, const int* ch,
                         int cin, int head_c, void* work, long long work_bytes, float* out, int N,

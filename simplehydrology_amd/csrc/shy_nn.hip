@@ -1950,8 +1950,16 @@ int shy_nn_conv_fwd_pool(const void* x, const void* w, const float* bias, const 
 // channels (stage output and two between), the pooled input of the next level.
 static size_t unet_align(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
+// the levels' channels that the network's convolutions take: the fused head
+// reads 32, the others are multiples of 32
+static bool unet_channels(const int* ch) {
+  for (int k = 0; k < 4; ++k)
+    if (ch[k] < 32 || ch[k] % 32) return false;
+  return ch[0] == 32;
+}
+
 long long shy_nn_unet_work_bytes(const int* ch, int N, int H, int W) {
-  if (!ch || N < 1 || H < 8 || W < 8 || H % 8 || W % 8) return -1;
+  if (!ch || !unet_channels(ch) || N < 1 || H < 8 || W < 8 || H % 8 || W % 8) return -1;
   size_t sum = 0;
   for (int k = 0; k < 4; ++k) {
     const size_t p = (size_t)N * (H >> k) * (W >> k) * 2;
@@ -1964,6 +1972,10 @@ int shy_nn_unet_forward(const void* x, const void* const* w, const float* const*
                         int cin, int head_c, void* work, long long work_bytes, float* out, int N,
                         int H, int W, void* stream) {
   if (!x || !w || !b || !ch || !work || !out) return nn_fail("unet_forward: bad pointers");
+  // before the first launch
+  if (!unet_channels(ch) || cin < 8 || cin % 8 || head_c < 4 || head_c > 16 || head_c % 4)
+    return nn_fail("unet_forward: need ch[0] = 32, ch[1..3] multiples of 32, cin a multiple of 8, "
+                   "head_c in {4, 8, 12, 16}");
   const long long need = shy_nn_unet_work_bytes(ch, N, H, W);
   if (need < 0) return nn_fail("unet_forward: H and W must be multiples of 8");
   if (work_bytes < need) return nn_fail("unet_forward: work memory too small");

@@ -439,7 +439,8 @@ class UNet:
         ch = (C.c_int * 4)(*(s.a.cout for s in self.e))
         size = nn().shy_nn_unet_work_bytes(ch, N, H, W)
         if size < 0:
-            raise RuntimeError("shy_nn: unet_forward: H and W must be multiples of 8")
+            raise RuntimeError("shy_nn: unet_forward: need 32 channels at the first level, multiples "
+                               "of 32 at the others, H and W multiples of 8")
         work = torch.empty(size, dtype=torch.uint8, device=x.device)
         out = torch.empty(N, H, W, self.head.cout, dtype=torch.float32, device=x.device)
         _ck(nn().shy_nn_unet_forward(_p(x), w, b, ch, cs[0].cin, self.head.cout, _p(work), size,
