@@ -35,6 +35,27 @@ __host__ __device__ inline long long pack_records(int nx, int ny) {
   return (long long)((nx + 1) >> 1) * ((ny + 1) >> 1) * 4;
 }
 
+// The walk of one wave per drop (walk_solo_kernel) reads records by 32-bit byte
+// offsets and multiplies in 24 bits.  solo_rec: pack_rec with one multiply and no
+// masks (2 (x >> 1) + (x & 1) = x), stride4 = 4 records per block row less one.
+// solo_terrain: the terrains whose records' offsets all fit, and whose sides
+// leave a step's unit moves exact.  11585 x 11585 and 33 x 4067100 cells are maps
+// of a legal size, padded to more than 2^27 records, that do not.
+constexpr int kSoloMaxSide = 1 << 22;
+__host__ __device__ inline int solo_stride4(int ny) { return (((ny + 1) >> 1) - 1) * 4; }
+__host__ __device__ inline int solo_rec(int x, int y, int stride4) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const int b = __mul24(x >> 1, stride4);
+#else
+  const int b = (x >> 1) * stride4;
+#endif
+  return b + ((x << 1) + (((y >> 1) << 1) + y));
+}
+__host__ __device__ inline uint32_t solo_off(int rec) { return (uint32_t)rec << 5; }
+__host__ __device__ inline bool solo_terrain(int nx, int ny) {
+  return nx <= kSoloMaxSide && ny <= kSoloMaxSide && pack_records(nx, ny) <= (1LL << 27);
+}
+
 // Tile order of a terrain's cells: the index under which the step log names a
 // cell.  Blocks of 2^a x 2^b cells (64 x 64 where the sides allow), the blocks
 // x-major, so that the partition's 4096 consecutive indices are a square

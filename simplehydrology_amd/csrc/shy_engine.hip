@@ -181,8 +181,8 @@ constexpr int kReplayBlock = 64;
 constexpr int kReplayLds = 52 * 1024;
 // Drops (with padding) up to which a cycle runs one wave per drop
 // (walk_solo_kernel) on maps of up to / more than kSoloSmallCells cells (whose
-// drops soon leave a small map, so their waves end early), and the map sides it
-// takes (its window needs unit steps to move a position by at most two cells).
+// drops soon leave a small map, so their waves end early).  Every terrain must
+// be one it can address (solo_terrain); others keep a lane per drop.
 // A cycle in us, one wave per drop / one lane per drop and the partition:
 // 128^2 with 1024 drops 103 / 214; 192^2 with 4096 249 / 336; 256^2 with 1024
 // 245 / 459, 4096 314 / 409, 6144 360 / 405, 8192 397 / 399; 384^2 with 2048
@@ -192,7 +192,6 @@ constexpr int kReplayLds = 52 * 1024;
 // the walk with a lane per drop, and keeps that walk.
 constexpr int kSoloMaxDropsSmall = 6144, kSoloMaxDrops = 2560;
 constexpr size_t kSoloSmallCells = 65536;
-constexpr int kSoloMaxSide = 1 << 22;
 constexpr int kWalkBlock = 256;  // default threads per block of the walk
 
 // Threads per walk block, which are a partition block's drops too: unless the
@@ -213,7 +212,7 @@ bool solo_cycle(const shy_ctx* c) {
   if (c->total_drops < 1 || c->total_drops > most) return false;
   if (c->tune.walk_block != kWalkBlock || c->tune.walk_grid != 0 || c->drop_order > 0) return false;
   for (const Terrain& t : c->ter)
-    if (t.nx > kSoloMaxSide || t.ny > kSoloMaxSide) return false;
+    if (!solo_terrain(t.nx, t.ny)) return false;
   return true;
 }
 

@@ -872,21 +872,15 @@ __device__ inline void lds_store_release(int* p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// byte offset of cell (x, y)'s record, in 32-byte units: pack_rec with one
-// multiply and no masks (2 (x >> 1) + (x & 1) = x)
-__device__ inline int solo_rec(int x, int y, int stride4) {
-  return __mul24(x >> 1, stride4) + ((x << 1) + (((y >> 1) << 1) + y));
-}
-
 // The walker.  SHORT: the arithmetic of walk_short; else the full sequences.
-// Both need positions below 2^22 (window, exact unit steps); the host checks.
+// Both need a terrain in solo_terrain's range; the host checks.
 template <bool SHORT>
 __device__ __forceinline__ void solo_walker(const WaveArgs& w, const Terrain& T,
                                             const float2* __restrict__ vt, SoloShared& sh,
                                             int slot, int x0, int y0) {
   const int lane = threadIdx.x & 63;
   const int nx = T.nx, ny = T.ny;
-  const int stride4 = (((ny + 1) >> 1) - 1) * 4;
+  const int stride4 = solo_stride4(ny);
   const int nrec = ((nx + 1) >> 1) * ((ny + 1) >> 1) * 4;
   const float mt = kLod * T.P.momentumTransfer;
   const char* pack = reinterpret_cast<const char*>(w.pack + 2 * T.pack_off);
@@ -900,7 +894,7 @@ __device__ __forceinline__ void solo_walker(const WaveArgs& w, const Terrain& T,
     v.base = 27 - ix * 8 - iy;
     int r = solo_rec(ix + lx, iy + ly, stride4);
     r = r < 0 ? 0 : (r > nrec - 1 ? nrec - 1 : r);
-    const size_t o = (uint32_t)r << 5;
+    const size_t o = solo_off(r);
     v.a = *reinterpret_cast<const float4*>(pack + o);
     v.b = *reinterpret_cast<const float4*>(pack + o + 16);
   };
@@ -1001,7 +995,7 @@ __device__ __forceinline__ void solo_helper(const WaveArgs& w, const Terrain& T,
                                             const float2* __restrict__ vt, SoloShared& sh,
                                             int slot, int g, uint32_t cid) {
   const int lane = threadIdx.x & 63;
-  const int ny = T.ny, stride4 = (((ny + 1) >> 1) - 1) * 4;
+  const int ny = T.ny, stride4 = solo_stride4(ny);
   const char* pack = reinterpret_cast<const char*>(w.pack + 2 * T.pack_off);
   int2* log = w.solo + (size_t)g * w.solo_stride;
   for (int k0 = 0;; k0 += 64) {
@@ -1020,9 +1014,9 @@ __device__ __forceinline__ void solo_helper(const WaveArgs& w, const Terrain& T,
       // where the step led (the walker's own sum)
       const int jx = ex ? x : cvt_i32(s.x + s.z), jy = ex ? y : cvt_i32(s.y + s.w);
       const float4 ra =
-          *reinterpret_cast<const float4*>(pack + ((size_t)(uint32_t)solo_rec(x, y, stride4) << 5));
-      const float hn = *reinterpret_cast<const float*>(
-          pack + ((size_t)(uint32_t)solo_rec(jx, jy, stride4) << 5));
+          *reinterpret_cast<const float4*>(pack + solo_off(solo_rec(x, y, stride4)));
+      const float hn =
+          *reinterpret_cast<const float*>(pack + solo_off(solo_rec(jx, jy, stride4)));
       const float vol = vt[k0 + lane].x;
       const float h2 = ex ? (float)((double)ra.x - 0.002) : hn;   // water.h:120-124
       float c_eq = (1.0f + T.P.entrainment * ra.w) * (ra.x - h2);  // water.h:127
