@@ -92,7 +92,7 @@ struct ConvArgs {
   // shy_nn_add then shy_nn_relu_bwd on the rounded output.
   const __bf16* __restrict__ gres;
   const __bf16* __restrict__ mask;
-  // When head_w is set (conv_tiles_kernel, 32 output channels, BF16 output):
+  // When head_w is set (HEAD instantiations, 32 output channels, BF16 output):
   // the epilogue also applies a 1x1 convolution to the rounded output,
   // head_y [P][head_c] (FP32) = head_b + head_w [head_c][32] . y, with one
   // MFMA per row of pixels; y_bf may then be null (y not stored).
@@ -110,8 +110,10 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 // One lane's 4 consecutive output channels co..co+3 of output element o:
 // bias, residual (before rounding), ReLU, then the store, FP32 or BF16 (with
-// the backward-pass residual and mask after rounding).
-__device__ inline void store_out4(const ConvArgs& a, size_t o, int co, const f32x4& acc) {
+// the backward-pass residual and mask after rounding).  Returns the BF16 values
+// (zeros for an FP32 output); with HEAD a null y_bf stores nothing.
+template <bool HEAD>
+__device__ inline bf16x4 store_out4(const ConvArgs& a, size_t o, int co, const f32x4& acc) {
   float v[4];
   // the lane's 4 biases in one load: co is a multiple of 4 and the entry
   // points require a 16-byte aligned bias
@@ -129,10 +131,10 @@ __device__ inline void store_out4(const ConvArgs& a, size_t o, int co, const f32
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
   }
+  bf16x4 q = {};
   if (a.y_f) {
     *reinterpret_cast<float4*>(a.y_f + o) = make_float4(v[0], v[1], v[2], v[3]);
   } else {
-    bf16x4 q;
 #pragma unroll
     for (int i = 0; i < 4; ++i) q[i] = (__bf16)v[i];
     if (a.gres) {
@@ -143,8 +145,9 @@ __device__ inline void store_out4(const ConvArgs& a, size_t o, int co, const f32
 #pragma unroll
       for (int i = 0; i < 4; ++i) q[i] = (float)a.mask[o + i] > 0.0f ? q[i] : (__bf16)0.0f;
     }
-    *reinterpret_cast<bf16x4*>(a.y_bf + o) = q;
+    if (!HEAD || a.y_bf) *reinterpret_cast<bf16x4*>(a.y_bf + o) = q;
   }
+  return q;
 }
 
 // The 1x1 head on a tile's rounded 32-channel output q (ConvArgs::head_w),
@@ -237,11 +240,12 @@ __device__ inline void conv_after(const ConvArgs& a, const bf16x4 (&q)[MT][NT], 
 }
 
 // The epilogue of a block's tile: lane holds channels cb + 16m + 4(lane/16)
-// + i of pixel (y0 + NT wave + t, x0 + lane%16).
-template <int MT, int NT>
+// + i of pixel (y0 + NT wave + t, x0 + lane%16).  HEAD: then the 1x1 head.
+template <int MT, int NT, bool HEAD>
 __device__ inline void conv_epilogue(const ConvArgs& a, const f32x4 (&acc)[MT][NT], int n, int y0,
                                      int x0, int cb, int wave, int lane) {
   const int gx = x0 + (lane & 15);
+  bf16x4 q[MT][NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int gy = y0 + wave * NT + t;
@@ -249,9 +253,12 @@ __device__ inline void conv_epilogue(const ConvArgs& a, const f32x4 (&acc)[MT][N
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const int co = cb + m * 16 + (lane >> 4) * 4;
-      if (gy < a.H && gx < a.W && co < a.Cout) store_out4(a, p * a.Cout + co, co, acc[m][t]);
+      q[m][t] = bf16x4{};
+      if (gy < a.H && gx < a.W && co < a.Cout)
+        q[m][t] = store_out4<HEAD>(a, p * a.Cout + co, co, acc[m][t]);
     }
   }
+  if constexpr (HEAD) conv_head<NT>(a, q, n, y0, x0, wave, lane);
 }
 
 // Forward (and dgrad) convolution.  Block = 4 waves; each wave owns 32 pixels
@@ -344,7 +351,7 @@ constexpr int kPS = 40;
 // read from LDS once per column shift dx and used for the three row shifts
 // dy (a wave's NT output rows need NT + 2 patch rows): per chunk and wave
 // 3 (NT + 2) B reads and 9 MT A reads feed 9 MT NT MFMAs.
-template <int TAPS, int MT, int NT, bool UPCAT = false>
+template <int TAPS, int MT, int NT, bool UPCAT = false, bool HEAD = false>
 __global__ void __launch_bounds__(256, 2) conv_pf_kernel(ConvArgs a) {
   constexpr int kTH = 4 * NT;
   constexpr int HALO = TAPS == 9 ? 1 : 0;
@@ -457,7 +464,7 @@ __global__ void __launch_bounds__(256, 2) conv_pf_kernel(ConvArgs a) {
       __syncthreads();
     }
   }
-  conv_epilogue<MT, NT>(a, acc, n, y0, x0, cb, wave, lane);
+  conv_epilogue<MT, NT, HEAD>(a, acc, n, y0, x0, cb, wave, lane);
 }
 
 // The same convolution with persistent blocks: block (b, co) takes the tiles
@@ -777,7 +784,7 @@ __global__ void __launch_bounds__(256) conv_c8_kernel(ConvArgs a) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[m][t] = mfma(A[m], B[t], acc[m][t]);
   }
-  conv_epilogue<MT, NT>(a, acc, n, y0, x0, cb, wave, lane);
+  conv_epilogue<MT, NT, false>(a, acc, n, y0, x0, cb, wave, lane);
 }
 
 // dgrad weights: Wf[ci][tap'*Cout + co] = W[co][(TAPS-1-tap')*Cin + ci]
@@ -1767,6 +1774,7 @@ int launch_pf(const ConvArgs& a, int taps, hipStream_t s, const char* what) {
   const bool big = taps == 9 || tiles16 * gy >= 1024;
   const dim3 g((unsigned)(big ? tiles16 : tiles8), gy);
   if (a.x2) conv_pf_kernel<9, 2, 4, true><<<g, 256, 0, s>>>(a);  // the input is [up2(x), x2]
+  else if (a.head_w) conv_pf_kernel<9, 2, 4, false, true><<<g, 256, 0, s>>>(a);
   else if (taps == 9) conv_pf_kernel<9, 2, 4><<<g, 256, 0, s>>>(a);
   else if (big) conv_pf_kernel<1, 2, 4><<<g, 256, 0, s>>>(a);
   else conv_pf_kernel<1, 2, 2><<<g, 256, 0, s>>>(a);
@@ -1875,14 +1883,7 @@ int shy_nn_conv_fwd_head(const void* x, const void* w, const float* bias, const 
   a.head_b = head_b;
   a.head_y = head_y;
   a.head_c = head_c;
-  if (!tile_rows_fit(a)) {  // rows beyond the tile loop's offsets: two passes
-    if (!y_bf16) return nn_fail("conv_fwd_head: rows too long without an output for y");
-    if (int r = shy_nn_conv_fwd(x, w, bias, res, y_bf16, nullptr, N, H, W, Cin, 32, 9, relu, stream))
-      return r;
-    return shy_nn_conv_fwd(y_bf16, head_w, head_b, nullptr, nullptr, head_y, N, H, W, 32, head_c, 1,
-                           0, stream);
-  }
-  return launch_tiles(a, (hipStream_t)stream, "conv_fwd_head");
+  return launch_pf(a, 9, (hipStream_t)stream, "conv_fwd_head");
 }
 
 int shy_nn_conv_fwd_upcat(const void* x_half, const void* skip, const void* w, const float* bias,
