@@ -111,8 +111,7 @@ int shy_nn_conv_wgrad_bias(const void* x, const void* g, float* dw, float* db, f
 /* The same of a convolution of [up2(x_half), skip] along channels (C1 + C2),
    read from the two tensors (shy_nn_conv_fwd_upcat's input): the bits of the
    gradients of the concatenated input.  H, W even; C1, C2, Cout multiples of 32,
-   Cout <= 1024; part holds part_splits*Cout*9*(C1+C2) floats; g and bias_part
-   16-byte aligned. */
+   Cout <= 1024; part holds part_splits*Cout*9*(C1+C2) floats. */
 int shy_nn_conv_wgrad_bias_cat(const void* x_half, const void* skip, const void* g, float* dw,
                                float* db, float* part, int part_splits, float* bias_part,
                                int bias_rows, int N, int H, int W, int C1, int C2, int Cout,

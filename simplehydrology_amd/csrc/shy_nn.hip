@@ -2204,11 +2204,15 @@ int shy_nn_conv_wgrad_bias_cat(const void* x_half, const void* skip, const void*
                                int bias_rows, int N, int H, int W, int C1, int C2, int Cout,
                                void* stream) {
   if (!x_half || !skip || !g || !dw || !db || !part || part_splits < 1 || !bias_part ||
-      bias_rows < 1 || !a16(g) || !a16(bias_part))
+      bias_rows < 1)
     return nn_fail("conv_wgrad_bias_cat: bad pointers");
   if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || C1 < 32 || C1 % 32 || C2 < 32 || C2 % 32 ||
       Cout < 32 || Cout % 32 || Cout > 1024 || (long long)N * H * W > INT32_MAX)
     return nn_fail("conv_wgrad_bias_cat: need H, W even and C1, C2, Cout multiples of 32");
+  if (!a16(g) || !a16(bias_part)) {  // shy_nn_bias_grad's element-wise sums
+    if (int r = shy_nn_bias_grad(g, db, bias_part, bias_rows, N * H * W, Cout, stream)) return r;
+    db = nullptr;
+  }
   return wgrad_lds(x_half, skip, C1, g, dw, part, part_splits, db, bias_part, bias_rows, N, H, W,
                    C1 + C2, Cout, (hipStream_t)stream);
 }
@@ -2216,8 +2220,8 @@ int shy_nn_conv_wgrad_bias_cat(const void* x_half, const void* skip, const void*
 int shy_nn_conv_wgrad_bias_upcat(const void* x_half, const void* skip, const void* g, float* dw,
                                  float* db, float* part, int part_splits, int N, int H, int W,
                                  int C1, int C2, int Cout, void* stream) {
-  if (!x_half || !skip || !g || !dw || !db || !part || part_splits < 2)
-    return nn_fail("conv_wgrad_bias_upcat: bad pointers, or fewer than two partials");
+  if (!x_half || !skip || !g || !dw || !db || !part || part_splits < 1)
+    return nn_fail("conv_wgrad_bias_upcat: bad pointers");
   if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || C1 < 32 || C1 % 32 || C2 < 32 || C2 % 32 ||
       Cout < 32 || Cout % 32 || Cout > 1024 || (long long)N * H * W > INT32_MAX)
     return nn_fail("conv_wgrad_bias_upcat: need H, W even and C1, C2, Cout multiples of 32");
