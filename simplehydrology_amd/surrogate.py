@@ -358,6 +358,22 @@ class ResStage:
         return [self.a, self.b, self.c]
 
 
+# the layers' methods as they stand here (a program may replace or wrap them)
+_CONV_FORWARDS = ("forward", "forward_head", "forward_pool", "forward_upcat")
+_STAGE_PASSES = ("forward", "backward")
+_OWN = [getattr(Conv, n) for n in _CONV_FORWARDS] + [getattr(ResStage, n) for n in _STAGE_PASSES]
+
+
+def _own_classes():
+    return _OWN == ([getattr(Conv, n) for n in _CONV_FORWARDS]
+                    + [getattr(ResStage, n) for n in _STAGE_PASSES])
+
+
+def _own(layer, cls, methods):
+    """Whether layer is a cls of this module with none of the methods replaced."""
+    return type(layer) is cls and vars(layer).keys().isdisjoint(methods)
+
+
 class UNet:
     CH = (32, 64, 96, 128)
 
@@ -401,11 +417,18 @@ class UNet:
         ``keep`` saves what :meth:`backward` needs.  The decoder stages read
         their upsampled-and-concatenated input straight from the two
         tensors."""
+        import torch
         N, H, W, _ = x.shape
         self.shapes = [(N, H >> k, W >> k) for k in range(4)]
         self.kept = keep
+        # stages of a program's own know only forward's and backward's first
+        # arguments, and what the fused passes take comes in multiples of 32
+        self.fused = _own_classes() and all(_own(s, ResStage, _STAGE_PASSES) and s.c.cout % 32 == 0
+                                            for s in self.e + self.d)
         if not keep:
-            return self._infer(x, N, H, W)
+            one = self._one_call()
+            if one is not None:
+                return self._infer(x, N, H, W, *one)
         skips = []
         h = x
         for k in range(4):
@@ -421,22 +444,50 @@ class UNet:
         for k in (2, 1, 0):
             self.cat.append((h.shape[-1], skips[k].shape[-1]))
             # the last stage's last convolution applies the head in its own pass
-            h = self.d[k].forward(h, self.shapes[k], skip=skips[k],
-                                  head=self.head if k == 0 else None, keep=keep)
+            head = self.head if k == 0 else None
+            if not keep:
+                h = self.d[k].forward(h, self.shapes[k], skip=skips[k], head=head)
+                continue
+            if self.fused:
+                h = self.d[k].forward(h, self.shapes[k], skip=skips[k], head=head, keep=True)
+                continue
+            n, hh, ww = self.shapes[k]
+            cu, cs = self.cat[-1]
+            u = torch.empty(n, hh, ww, cu + cs, dtype=torch.bfloat16, device=x.device)
+            _ck(nn().shy_nn_up2(_p(h), _p(u), n, hh // 2, ww // 2, cu, cu + cs, 0, 0, _stream()))
+            _ck(nn().shy_nn_channels(_p(skips[k]), _p(u), n * hh * ww, cs, cu + cs, cu, 0,
+                                     _stream()))
+            h = self.d[k].forward(u, self.shapes[k], head=head)
         self.h0, out = h
         return out
 
-    def _infer(self, x, N, H, W):
+    def _one_call(self):
+        """What the library's one-call forward needs, (convolutions, channels),
+        or None where the network is not the one it computes: a layer replaced,
+        wrapped or of another shape."""
+        stages = self.e + self.d
+        if not self.fused or len(self.e) != 4 or len(self.d) != 3:
+            return None
+        cs = [c for s in stages for c in (s.a, s.b, s.c)] + [self.head]
+        c0, c1, c2, c3 = ch = [s.c.cout for s in self.e]
+        cin = [cs[0].cin, c0, c1, c2, c1 + c0, c2 + c1, c3 + c2]
+        want = [d for i, c in zip(cin, ch + ch[:3]) for d in ((i, c, 9), (c, c, 9), (c, c, 9))]
+        want.append((c0, self.head.cout, 1))
+        if c0 != 32 or any((c.cin, c.cout, c.taps) != d or not _own(c, Conv, _CONV_FORWARDS)
+                           for c, d in zip(cs, want)):
+            return None
+        return cs, ch
+
+    def _infer(self, x, N, H, W, cs, ch):
         """The forward without what backward needs, in one call: 21 launches
         made one by one from here take 9 us of host time each, more than a
         small batch's kernels."""
         import torch
         for s in self.e + self.d:
             s.saved = None
-        cs = self.convs()
         w = (C.c_void_p * len(cs))(*(c.w_bf.data_ptr() for c in cs))
         b = (C.c_void_p * len(cs))(*(c.b.data_ptr() for c in cs))
-        ch = (C.c_int * 4)(*(s.a.cout for s in self.e))
+        ch = (C.c_int * 4)(*ch)
         size = nn().shy_nn_unet_work_bytes(ch, N, H, W)
         if size < 0:
             raise RuntimeError("shy_nn: unet_forward: need 32 channels at the first level, multiples "
@@ -453,6 +504,8 @@ class UNet:
         if not self.kept:
             raise RuntimeError("backward needs a forward(..., keep=True)")
         g = self.head.backward(self.h0, gy, self.shapes[0], self.scratch)
+        if not self.fused:
+            return self._backward_by_passes(g)
         gus = []
         for k, (cu, cs) in zip((0, 1, 2), reversed(self.cat)):
             n, hh, ww = self.shapes[k]
@@ -474,6 +527,28 @@ class UNet:
             g = torch.empty(n, hh, ww, c, dtype=torch.bfloat16, device=gy.device)
             _ck(nn().shy_nn_skip_bwd(_p(gx), _p(gus[k - 1]), _p(self.e[k - 1].saved[3]), _p(g), n,
                                      hh, ww, c, cu + cs, cu, _stream()))
+
+    def _backward_by_passes(self, g):
+        """The rest of backward with the passes between two stages one by one,
+        from the stages' forward and backward alone: the same bits."""
+        import torch
+        gskip = [None, None, None]
+        for k, (cu, cs) in zip((0, 1, 2), reversed(self.cat)):
+            n, hh, ww = self.shapes[k]
+            gu = self.d[k].backward(g, self.shapes[k], self.scratch)
+            gskip[k] = torch.empty(n, hh, ww, cs, dtype=torch.bfloat16, device=g.device)
+            _ck(nn().shy_nn_channels(_p(gu), _p(gskip[k]), n * hh * ww, cs, cu + cs, cu, 1,
+                                     _stream()))
+            g = torch.empty(n, hh // 2, ww // 2, cu, dtype=torch.bfloat16, device=g.device)
+            _ck(nn().shy_nn_up2(_p(gu), _p(g), n, hh // 2, ww // 2, cu, cu + cs, 0, 1, _stream()))
+        for k in (3, 2, 1, 0):
+            gx = self.e[k].backward(g, self.shapes[k], self.scratch, need_dx=k > 0)
+            if k == 0:
+                break
+            n, hh, ww = self.shapes[k - 1]
+            gp = torch.empty(n, hh, ww, gx.shape[-1], dtype=torch.bfloat16, device=g.device)
+            _ck(nn().shy_nn_pool2(_p(gx), _p(gp), n, hh, ww, gx.shape[-1], 1, _stream()))
+            g = _add(gp, gskip[k - 1])
 
     def step(self, lr, wd=0.0):
         self.t += 1
