@@ -637,6 +637,15 @@ def predict_tiled(net, h, d, mx, my, tile=256, halo=32, batch=16):
         x = torch.empty(n, tile, tile, 8, dtype=torch.bfloat16, device=h.device)
         _ck(nn().shy_nn_window_input(_p(xs), _p(mean), _p(x), n, tile, H_SCALE, _stream()))
         y = net.forward(x, keep=False)
+        if (y.shape != (n, tile, tile, 8) or y.dtype != torch.float32 or y.device != h.device
+                or not y.is_contiguous()):
+            # a network of the program's own: its first three channels
+            for k, (wx, cx, lx, wy, cy, ly) in enumerate(js):
+                crop = torch.empty(lx, ly, 3, dtype=torch.float32, device=h.device)
+                crop[:] = y[k, cx - wx:cx - wx + lx, cy - wy:cy - wy + ly, :3]
+                for o, v in zip(out, decode_flow(crop)):
+                    o[cx:cx + lx, cy:cy + ly] = v
+            continue
         for k, m, table in parts:
             _ck(nn().shy_nn_window_output(_p(y[k]), table, m, _p(out[0]), _p(out[1]), _p(out[2]),
                                           X, Y, tile, D_SCALE, _stream()))
