@@ -24,17 +24,27 @@ FLAGS = [
 ]
 
 
-def build_library(verbose: bool = False) -> str:
-    srcs = [os.path.join(CSRC, s) for s in SOURCES]
-    tmp = LIB + ".tmp"
+def _hipcc(out: str, srcs: list[str], verbose: bool = False) -> str:
+    tmp = out + ".tmp"
     cmd = [HIPCC, *FLAGS, "-o", tmp, *srcs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("hipcc failed:\n" + " ".join(cmd) + "\n" + r.stdout + r.stderr)
     if verbose:
         print(" ".join(cmd))
-    os.replace(tmp, LIB)
-    return LIB
+    os.replace(tmp, out)
+    return out
+
+
+def build_library(verbose: bool = False) -> str:
+    return _hipcc(LIB, [os.path.join(CSRC, s) for s in SOURCES], verbose)
+
+
+def build_device_checks() -> str:
+    """tests/libshort_math_check.so: the kernels' headers checked on the device."""
+    tests = os.path.join(os.path.dirname(HERE), "tests")
+    return _hipcc(os.path.join(tests, "libshort_math_check.so"),
+                  [os.path.join(tests, "short_math_check.hip")])
 
 
 DEMO = os.path.join(HERE, "world_demo")

@@ -280,8 +280,8 @@ __device__ inline void block_add_stats(long long (&v)[NC], DeviceState* state, i
 // ------------------------------------------------------------------ walk
 // sqrt(x) and 1/x, correctly rounded, in 5 and 3 instructions: the hardware
 // approximation and one FMA-based correction.  Equal to __builtin_sqrtf and
-// to the division for every float in [2^-100, 2^126) (all 1.9e9 of them
-// compared on the device); outside it, and for 0, not used.  The full
+// to the division for every float in [2^-100, 2^126) (tests/short_math_check.hip
+// checks all 1.9e9 of them); outside it, and for 0, not used.  The full
 // sequences (about 14 and 11 instructions each, four and three of them per
 // step) were 40% of the 220 VALU instructions of a walk step, which are 880 of
 // its 1540 cycles at 256^2 and of its 2060 at 1024^2.  (1/sqrt(x) from the
