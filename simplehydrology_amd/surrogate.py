@@ -359,19 +359,17 @@ class ResStage:
 
 
 # the layers' methods as they stand here (a program may replace or wrap them)
-_CONV_FORWARDS = ("forward", "forward_head", "forward_pool", "forward_upcat")
-_STAGE_PASSES = ("forward", "backward")
-_OWN = [getattr(Conv, n) for n in _CONV_FORWARDS] + [getattr(ResStage, n) for n in _STAGE_PASSES]
+_OWN = [Conv.forward, Conv.forward_head, Conv.forward_pool, Conv.forward_upcat,
+        ResStage.forward, ResStage.backward]
+
+
+# ctypes forgets an array type that nothing holds, and makes it anew in 30 us
+_Pointers22, _Ints4 = C.c_void_p * 22, C.c_int * 4
 
 
 def _own_classes():
-    return _OWN == ([getattr(Conv, n) for n in _CONV_FORWARDS]
-                    + [getattr(ResStage, n) for n in _STAGE_PASSES])
-
-
-def _own(layer, cls, methods):
-    """Whether layer is a cls of this module with none of the methods replaced."""
-    return type(layer) is cls and vars(layer).keys().isdisjoint(methods)
+    return _OWN == [Conv.forward, Conv.forward_head, Conv.forward_pool, Conv.forward_upcat,
+                    ResStage.forward, ResStage.backward]
 
 
 class UNet:
@@ -421,14 +419,15 @@ class UNet:
         N, H, W, _ = x.shape
         self.shapes = [(N, H >> k, W >> k) for k in range(4)]
         self.kept = keep
-        # stages of a program's own know only forward's and backward's first
-        # arguments, and what the fused passes take comes in multiples of 32
-        self.fused = _own_classes() and all(_own(s, ResStage, _STAGE_PASSES) and s.c.cout % 32 == 0
-                                            for s in self.e + self.d)
         if not keep:
             one = self._one_call()
             if one is not None:
                 return self._infer(x, N, H, W, *one)
+        # stages of a program's own know only forward's and backward's first
+        # arguments, and what the fused passes take comes in multiples of 32
+        self.fused = _own_classes() and all(
+            type(s) is ResStage and vars(s).keys().isdisjoint(("forward", "backward"))
+            and s.c.cout % 32 == 0 for s in self.e + self.d)
         skips = []
         h = x
         for k in range(4):
@@ -462,40 +461,55 @@ class UNet:
         return out
 
     def _one_call(self):
-        """What the library's one-call forward needs, (convolutions, channels),
-        or None where the network is not the one it computes: a layer replaced,
-        wrapped or of another shape."""
-        stages = self.e + self.d
-        if not self.fused or len(self.e) != 4 or len(self.d) != 3:
+        """What the library's one-call forward needs, the addresses of the
+        weights and biases and the channels, or None where the network is not the
+        one it computes: a layer replaced, wrapped or of another shape.  (One
+        loop over the layers' dictionaries: a first pass waits for it.)"""
+        e, d, head = self.e, self.d, self.head
+        if len(e) != 4 or len(d) != 3 or not _own_classes() or head.cin != 32 or head.taps != 1:
             return None
-        cs = [c for s in stages for c in (s.a, s.b, s.c)] + [self.head]
-        c0, c1, c2, c3 = ch = [s.c.cout for s in self.e]
-        cin = [cs[0].cin, c0, c1, c2, c1 + c0, c2 + c1, c3 + c2]
-        want = [d for i, c in zip(cin, ch + ch[:3]) for d in ((i, c, 9), (c, c, 9), (c, c, 9))]
-        want.append((c0, self.head.cout, 1))
-        if c0 != 32 or any((c.cin, c.cout, c.taps) != d or not _own(c, Conv, _CONV_FORWARDS)
-                           for c, d in zip(cs, want)):
+        w, b, ch = [], [], []
+        for k, s in enumerate(e + d):
+            v = vars(s)
+            if type(s) is not ResStage or "forward" in v or "backward" in v:
+                return None
+            if k < 4:
+                cin, cout = ch[-1] if k else s.a.cin, s.a.cout
+                ch.append(cout)
+                if cout % 32:
+                    return None
+            else:
+                cin, cout = ch[k - 3] + ch[k - 4], ch[k - 4]
+            for c in (s.a, s.b, s.c):
+                v = vars(c)
+                if (type(c) is not Conv or v["cin"] != cin or v["cout"] != cout or v["taps"] != 9
+                        or "forward" in v or "forward_head" in v or "forward_pool" in v
+                        or "forward_upcat" in v):
+                    return None
+                cin = cout
+                w.append(v["w_bf"].data_ptr())
+                b.append(v["b"].data_ptr())
+        if ch[0] != 32:
             return None
-        return cs, ch
+        w.append(head.w_bf.data_ptr())
+        b.append(head.b.data_ptr())
+        return w, b, ch
 
-    def _infer(self, x, N, H, W, cs, ch):
+    def _infer(self, x, N, H, W, w, b, ch):
         """The forward without what backward needs, in one call: 21 launches
         made one by one from here take 9 us of host time each, more than a
         small batch's kernels."""
         import torch
         for s in self.e + self.d:
             s.saved = None
-        w = (C.c_void_p * len(cs))(*(c.w_bf.data_ptr() for c in cs))
-        b = (C.c_void_p * len(cs))(*(c.b.data_ptr() for c in cs))
-        ch = (C.c_int * 4)(*ch)
+        w, b, ch = _Pointers22(*w), _Pointers22(*b), _Ints4(*ch)
         size = nn().shy_nn_unet_work_bytes(ch, N, H, W)
         if size < 0:
-            raise RuntimeError("shy_nn: unet_forward: need 32 channels at the first level, multiples "
-                               "of 32 at the others, H and W multiples of 8")
+            raise RuntimeError("shy_nn: unet_forward: H and W must be multiples of 8")
         work = torch.empty(size, dtype=torch.uint8, device=x.device)
         out = torch.empty(N, H, W, self.head.cout, dtype=torch.float32, device=x.device)
-        _ck(nn().shy_nn_unet_forward(_p(x), w, b, ch, cs[0].cin, self.head.cout, _p(work), size,
-                                     _p(out), N, H, W, _stream()))
+        _ck(nn().shy_nn_unet_forward(_p(x), w, b, ch, self.e[0].a.cin, self.head.cout, _p(work),
+                                     size, _p(out), N, H, W, _stream()))
         return out
 
     def backward(self, gy):
