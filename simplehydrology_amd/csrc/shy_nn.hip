@@ -1608,7 +1608,7 @@ __global__ void flow_features_kernel(FlowMaps m, float* f, int X, int Y, float s
   const float d = m.d.at(x, y);
   float4* o = reinterpret_cast<float4*>(f + 8 * i);
   o[0] = make_float4(m.h.at(x, y), (xp - xm) * slope, (yp - ym) * slope,
-                     log1pf(d < 0.0f ? 0.0f : d) * scale);
+                     log1pf(d <= 0.0f ? 0.0f : d) * scale);
   o[1] = make_float4(signed_log1p(m.mx.at(x, y), scale), signed_log1p(m.my.at(x, y), scale), 0.0f,
                      0.0f);
 }
