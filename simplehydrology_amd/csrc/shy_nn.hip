@@ -903,7 +903,8 @@ __global__ void __launch_bounds__(64) conv_wgrad_kernel(WgradArgs a) {
 // the bias / these with 3 waves of 32 input channels / 6 of 16 / 6 and two halves
 // of LDS: 256^2 32 -> 32 channels 95.8 / 53.1 / 48.8 / 49.8, 256^2 96 -> 32 264 / 117 / 105
 // / 102, 128^2 64 -> 64 101 / 48.7 / 46.8 / 41.1, 128^2 160 -> 64 221 / 98.7 / 91.6 /
-// 83.5, 64^2 224 -> 96 125 / 56.3 / 52.3 / 50.5, 32^2 128 -> 128 48.2 / 24.4 / 23.2 / 22.9.
+// 83.5, 64^2 224 -> 96 125 / 56.3 / 52.3 / 50.5, 32^2 128 -> 128 48.2 / 24.4 / 23.2 / 20.0
+// (the last with its channel blocks dealt out, see wgrad_lds).
 // (The bias blocks first in the grid: 128^2 64 -> 64 51.0.)
 constexpr int kWgTW = 16, kWgTH = 8, kWgPix = kWgTW * kWgTH;
 constexpr int kWgXW = kWgTW + 2, kWgXPix = kWgXW * (kWgTH + 2);
@@ -922,6 +923,7 @@ struct WgArgs {
   int N, H, W, Cin, Cout, K;
   int tiles_x, tiles_y, tiles;
   int tiles_per_split;
+  int xcds;
   int blocks;            // of the weight gradient; those after it sum the bias gradient
   float* bias_part;      // [ranges of bias_rows pixels][Cout]
   int bias_rows;
@@ -997,8 +999,9 @@ __global__ void __launch_bounds__(kWgThreads) wgrad_lds_kernel(WgArgs a) {
   // Workgroups go round-robin over the 8 XCDs: the channel blocks of one
   // range of tiles, which read the same g and x, follow each other on one XCD
   // and share its L2 (training step: 96 -> 96 channels at 64^2 31 -> 23.5 us)
-  const int nco = Cout / 32, nch = nco * (Cin / 32), seq = (int)blockIdx.x >> 3;
-  const int split = seq / nch * 8 + ((int)blockIdx.x & 7), ch = seq % nch;
+  // (a.xcds = 8), unless that leaves the XCDs with unequal work (a.xcds = 1; wgrad_lds)
+  const int nco = Cout / 32, nch = nco * (Cin / 32), seq = (int)blockIdx.x / a.xcds;
+  const int split = seq / nch * a.xcds + (int)blockIdx.x % a.xcds, ch = seq % nch;
   const int cb = ch % nco * 32, ci0 = ch / nco * 32;
   const int t_begin = split * a.tiles_per_split;
   const int t_end = min(a.tiles, t_begin + a.tiles_per_split);
@@ -2102,7 +2105,13 @@ static int wgrad_lds(const void* x, const void* x2, int C1, const void* g, float
   splits = std::min<long long>(splits, part_splits);
   b.tiles_per_split = (int)((tiles + splits - 1) / splits);
   splits = (tiles + b.tiles_per_split - 1) / b.tiles_per_split;
-  b.blocks = (int)((splits + 7) / 8 * 8 * bxy);  // equally many on every XCD
+  // a range of tiles per XCD where the 8 XCDs then have equal work to 1/8.  Ranges
+  // on their XCD / channel blocks dealt out, us at batch 16: 2 ranges, 32^2 512 ->
+  // 512 channels 447 / 135; 4, 16^2 1024 -> 1024 at batch 2 220 / 113; 10, 64^2
+  // 224 -> 224 171 / 106; 26, 32^2 128 -> 128 23.0 / 20.0; 29, 64^2 128 -> 128 41.1 /
+  // 49.5; 46, 128^2 160 -> 64 83.0 / 112
+  b.xcds = (splits + 7) / 8 * 64 <= splits * 9 ? 8 : 1;
+  b.blocks = (int)((splits + b.xcds - 1) / b.xcds * b.xcds * bxy);
   b.bias_part = bias_part;
   b.bias_rows = 0;
   int nb = 0;
