@@ -486,9 +486,9 @@ __global__ void __launch_bounds__(256, 2) conv_pf_kernel(ConvArgs a) {
 // one past the buffer's end; both read zeros and store nothing, as the
 // hardware checks each offset against the buffer's size, so only the tiles at
 // the left and right edge compare columns.  The rows of one tile must span
-// less than 2^31 bytes (tile_rows_fit).  A tile's residual (kEpiRes) or mask
-// (kEpiMask) is on its way while the next tile goes to LDS; where there are both
-// (kEpiGrad), a row of them is.
+// less than 2^31 bytes (tile_rows_fit).  A tile's residual (kEpiRes) or the
+// backward pass's residual and mask (kEpiGrad, kEpiMask) are on their way while the next
+// tile goes to LDS, or a row of them.
 // Measured against the same loop with an address, a bounds check and a branch
 // per load (us, at batch 16): 256^2, 32 -> 32 channels 40.1 -> 28.9 (4.6 TB/s),
 // with residual and pool 65.2 -> 41.9; 128^2, 64 -> 64 38.2 -> 32.1; 64^2,
@@ -662,19 +662,22 @@ __global__ void __launch_bounds__(256, kTileBlocksPerCU) conv_tiles_kernel(ConvA
       __syncthreads();
     }
     u32x2 e0[MT][NT], e1[MT][NT];
+    constexpr bool rowwise = EPI == kEpiGrad && NT > 2;
     if (EPI == kEpiRes) load_out(a.res, e0);
-    if (EPI == kEpiMask) load_out(a.mask, e1);
+    if (EPI == kEpiGrad && !rowwise) load_out(a.gres, e0);
+    if ((EPI == kEpiGrad && !rowwise) || EPI == kEpiMask) load_out(a.mask, e1);
     const bool next = tile + (int)gridDim.x < total;  // uniform over the block
     if (next) {
       __syncthreads();
       lstore(reload_w);
     }
-    // The residual and the mask of the backward pass: a row of the wave ahead,
-    // from here on.  Whole tiles of both beside the next tile's registers spilled
-    // (NT 4: 52 bytes a thread; at batch 16, us with all rows before the store to
-    // LDS / row by row: 128^2 64 -> 64 channels 48.9 / 39.7, 96 -> 128 104.8 / 89.2, 64^2
-    // 96 -> 96 21.0 / 18.0), and without the fences the compiler moves them up.
-    if (EPI == kEpiGrad) {
+    // The residual and the mask of the backward pass with 16 x 16 tiles: a row of
+    // the wave ahead, from here on.  Whole tiles of both beside the next tile's
+    // registers spilled (52 bytes a thread; at batch 16, us with all rows before
+    // the store to LDS / row by row: 128^2 64 -> 64 channels 48.9 / 39.7, 96 -> 128 104.8
+    // / 89.2, 64^2 96 -> 96 21.0 / 18.0), and without the fences the compiler moves
+    // them up.  (Row by row with 16 x 8 tiles: 32^2 512 -> 512 at batch 1 23.9 / 29.2.)
+    if (rowwise) {
       __builtin_amdgcn_sched_barrier(0);
       load_row(a.gres, 0, e0);
       load_row(a.mask, 0, e1);
@@ -692,7 +695,7 @@ __global__ void __launch_bounds__(256, kTileBlocksPerCU) conv_tiles_kernel(ConvA
     const __amdgpu_buffer_rsrc_t fbuf = tile_buffer(a.y_f + out0, a.y_f ? 2 * out_bytes : 0);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      if (EPI == kEpiGrad) {
+      if (rowwise) {
         if (t + 1 < NT) {
           load_row(a.gres, t + 1, e0);
           load_row(a.mask, t + 1, e1);
