@@ -9,8 +9,8 @@
 // B[(l/16)*8+i][l%16] for i < 8 and C[(l/16)*4+i][l%16] for i < 4.
 //
 //   conv_tiles_kernel  3x3 forward / data gradient of every layer of 32-channel
-//                      multiples, 16x16 pixel tiles (16x8 where those leave a
-//                      CU without any): persistent blocks (three per CU, 32 output channels
+//                      multiples, 16x16 pixel tiles (16x8 where all of those
+//                      run at once): persistent blocks (three per CU, 32 output channels
 //                      each) over the tiles, patch and weights staged in LDS,
 //                      the next chunk's patch loaded into registers during
 //                      the current chunk's MFMAs; decoder inputs read as
@@ -1747,14 +1747,23 @@ int device_cus() {
 // 64-channel layer takes two such blocks per tile: at 16 x 128^2, 32->64
 // 31.1 -> 27.8 us and 64->64 41.7 -> 40.7 us against one 64-channel block
 // at two blocks per CU (the 64-channel block needs 255 VGPRs).
+// blocks per 32 output channels that run at once
+long long tile_blocks(const ConvArgs& a) {
+  return std::max(1LL, (long long)kTileBlocksPerCU * device_cus() / (a.Cout / 32));
+}
+
 template <int NT>
 int launch_tiles_of(const ConvArgs& a, hipStream_t s, const char* what) {
   constexpr int MT = 2;
   const long long tiles = (long long)a.N * ((a.H + 4 * NT - 1) / (4 * NT)) * ((a.W + kTW - 1) / kTW);
   if (tiles > INT32_MAX) return nn_fail(std::string(what) + ": too many tiles");
-  const int gy = a.Cout / (16 * MT);
-  const long long cap = std::max(1LL, (long long)kTileBlocksPerCU * device_cus() / gy);
-  const dim3 g((unsigned)std::min(tiles, cap), (unsigned)gy);
+  const long long cap = tile_blocks(a);
+  // One tile per block, dealt out as blocks end, where a wide layer's blocks
+  // would take one or two each (from 160 channels on a tile is long beside its
+  // first loads; us at batch 16, 32^2 512 -> 512 channels 86 / 78, 3 x 104 x 152 256 ->
+  // 256 from two tensors 70.5 / 65.9)
+  const bool one = a.Cin > 128 && tiles > cap && tiles < 2 * cap;
+  const dim3 g((unsigned)(one ? tiles : std::min(tiles, cap)), (unsigned)(a.Cout / (16 * MT)));
   if (a.x2) {
     if (a.res) conv_tiles_kernel<MT, NT, true, false, false, kEpiRes><<<g, 256, 0, s>>>(a);
     else conv_tiles_kernel<MT, NT, true, false, false, kEpiPlain><<<g, 256, 0, s>>>(a);
@@ -1775,13 +1784,16 @@ int launch_tiles_of(const ConvArgs& a, hipStream_t s, const char* what) {
   return nn_check(what);
 }
 
-// 16 x 8 tiles where 16 x 16 ones leave a CU without any: twice the blocks,
-// each half as long (a whole forward, us with 16 x 16 blocks of one tile each,
-// an address and a check per load and a pool pass of its own / with these: one
-// window of 64^2 160 / 144, two of 128^2 170 / 149, four of 256^2 243 / 234)
+// 16 x 8 tiles where all of them run at once (twice the blocks, each half as
+// long), or where 16 x 16 ones would be as many (maps of 8 rows and fewer).  Us
+// with 16 x 8 / 16 x 16 tiles: 60 x 36 at batch 7 128 -> 128 channels 13.1 / 14.8, all
+// 16 x 8 ones at once; not all of them: 48 x 80 at batch 10 96 -> 96 18.4 / 12.6, 224 ->
+// 96 35.3 / 23.4, 88 x 24 at batch 9 128 -> 128 17.7 / 14.0.
 int launch_tiles(const ConvArgs& a, hipStream_t s, const char* what) {
-  const long long tiles16 = (long long)a.N * ((a.H + 15) / 16) * ((a.W + kTW - 1) / kTW);
-  return tiles16 >= device_cus() ? launch_tiles_of<4>(a, s, what) : launch_tiles_of<2>(a, s, what);
+  const long long across = (long long)a.N * ((a.W + kTW - 1) / kTW);
+  const long long tiles8 = across * ((a.H + 7) / 8), tiles16 = across * ((a.H + 15) / 16);
+  return tiles8 <= tile_blocks(a) || tiles8 == tiles16 ? launch_tiles_of<2>(a, s, what)
+                                                       : launch_tiles_of<4>(a, s, what);
 }
 
 // Cin and Cout multiples of 32: the tile loop for 3x3 (against one tile per

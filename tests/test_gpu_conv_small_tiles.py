@@ -1,6 +1,8 @@
-"""GPU: the 16 x 8 tiles of the 3x3 convolutions (layers of fewer than 256 tiles of
-16 x 16 pixels) at their edges, with each epilogue, against float64, and the
-first layer that takes 16 x 16 tiles beside the last that does not.
+"""GPU: the 16 x 8 tiles of the 3x3 convolutions (layers whose 16 x 8 tiles all run
+at once: 768 blocks of 32 output channels on 256 CUs; maps of up to 8 rows) at
+their edges, with each epilogue, against float64, and the layers on both sides of
+the lines: the last of 16 x 8 tiles and the first of 16 x 16 ones, and wide layers
+of one tile per block.
 
 Tolerances as in test_gpu_conv_tiles; a head output is an FP32 sum of 32 products
 of the rounded values (1e-6 is beyond 10 times its rounding), a pooled value is
@@ -13,13 +15,22 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-SIZES = [(1, 1, 1), (1, 7, 15), (2, 8, 16), (1, 9, 17), (3, 17, 33), (1, 24, 64), (5, 47, 65),
-         (255, 16, 16), (256, 16, 16)]
+SIZES = [(1, 1, 1), (1, 7, 15), (2, 8, 16), (1, 9, 17), (3, 17, 33), (1, 24, 64), (5, 47, 65)]
 
 
 @pytest.mark.parametrize("N,H,W", SIZES)
 @pytest.mark.parametrize("cin,cout", [(32, 32), (64, 96)])
 def test_forward_epilogues(shy, N, H, W, cin, cout):
+    tiles.test_forward_epilogues(shy, N, H, W, cin, cout)
+
+
+@pytest.mark.parametrize("N,H,W,cin,cout", [
+    (384, 16, 16, 32, 32), (385, 16, 16, 32, 32),  # 768 and 770 tiles of 16 x 8
+    (128, 16, 16, 64, 96), (129, 16, 16, 64, 96),  # 256 and 258, three channel blocks each
+    (770, 8, 15, 32, 32),                          # more than run at once, of 8 rows
+    (97, 15, 16, 160, 256),                        # 97 tiles of 16 x 16 on 96 blocks: one each
+])
+def test_lines_between_the_variants(shy, N, H, W, cin, cout):
     tiles.test_forward_epilogues(shy, N, H, W, cin, cout)
 
 
